@@ -606,7 +606,7 @@ __global__ void k_rec_write(int64_t ncells, const int32_t* __restrict__ CH, cons
 }
 
 // The expansion of each internal record as one polynomial in the direction
-// to the query (far_field_poly, device_math.h), formed in FP64 from the cell's
+// to the query (far_field_bracket, device_math.h), formed in FP64 from the cell's
 // FP32 EC and rounded once.  With l = CM - q, x = l/|l| and m = 1/|l|, the
 // terms of the reference's expansion (fast_winding_number.cpp:174-228) are
 //   order 0: m^2 (x.E0) / 4pi
@@ -681,14 +681,11 @@ __global__ void k_rec_poly(uint32_t nrec, const uint2* __restrict__ meta, const 
     g[2] -= 3.0 * sv[2];  // z^3
     for (int j = 0; j < 10; ++j) g[j] *= k;
   }
-  // record layout of far_field_poly: b, c, d, e, f
-  float4* r = poly + 5 * (size_t)p;
-  r[0] = make_float4((float)b[0], (float)b[1], (float)b[2], 0.0f);
-  r[1] = make_float4((float)q[0], (float)q[1], (float)q[2], (float)q[3]);
-  // d = (yz, xz, x^3, y^3), e = (z^3, x^2y, x^2z, xy^2), f = (y^2z, xz^2, yz^2, xyz)
-  r[2] = make_float4((float)q[4], (float)q[5], (float)g[0], (float)g[1]);
-  r[3] = make_float4((float)g[2], (float)g[3], (float)g[4], (float)g[5]);
-  r[4] = make_float4((float)g[6], (float)g[7], (float)g[8], (float)g[9]);
+  float v[20];
+  pack_far_field(b, q, g, v);
+  float4* r = poly + 5 * (size_t)p;  // b, c, d, e, f of far_field_bracket
+  r[0] = make_float4(v[0], v[1], v[2], 0.0f);
+  for (int j = 1; j < 5; ++j) r[j] = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
 }
 
 // ---------------- evaluation ----------------

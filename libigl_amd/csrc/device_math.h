@@ -22,7 +22,7 @@ __device__ __forceinline__ float atan01(float a) {
   return a * p;
 }
 
-// atan2 for y != 0 (the caller returns early on a zero numerator).
+// atan2 (not both arguments zero; for y = 0 it takes the sign of y).
 __device__ __forceinline__ float atan2_fast(float y, float x) {
   const float ax = fabsf(x), ay = fabsf(y);
   const float mx = fmaxf(ax, ay), mn = fminf(ax, ay);
@@ -32,41 +32,119 @@ __device__ __forceinline__ float atan2_fast(float y, float x) {
   return copysignf(r, y);
 }
 
-// FP32 far field of an order-0/1/2 Taylor expansion written as one
-// polynomial in the direction to the query.  For the offset q (l2 = |q|^2),
-// x = q/|q| (kept normalised so that the cubic cannot overflow for distant
-// queries) and m = 1/|q| the value is
+// Far field of an order-0/1/2 Taylor expansion written as one polynomial in
+// the direction to the query.  For the offset q (l2 = |q|^2), x = q/|q| (kept
+// normalised so that the cubic cannot overflow for distant queries) and
+// m = 1/|q| the value is
 //   m^2 [ x.b + m ( Qf(x) + m G(x) ) ]
-// with b = b.xyz, the quadratic form Qf(x) = c.x x^2 + c.y y^2 + c.z z^2 +
-// c.w xy + d.x yz + d.y xz and the cubic G(x) = d.z x^3 + d.w y^3 + e.x z^3 +
-// e.y x^2y + e.z x^2z + e.w xy^2 + f.x y^2z + f.y xz^2 + f.z yz^2 + f.w xyz.
+// with b = b.xyz.  |x| = 1 takes z^2 out of the quadratic form and of the
+// cubic, which leaves a constant and three linear terms in its place and
+// fewer operations (31 with the reciprocal square root, against 36 with both
+// in homogeneous form):
+//   Qf(x) = c.z + x (c.x x + c.w y + d.y z) + y (c.y y + d.x z)
+//   G(x)  = x (f.y + x (d.z x + e.y y + e.z z) + y (e.w y + f.w z))
+//         + y (f.z + y (d.w y + f.x z)) + e.x z
 // The soup's slot records (k_write_slots) and the cloud's cell records
-// (k_rec_poly) store their expansions in this form.
+// (k_rec_poly) store their expansions in this form, through pack_far_field.
+
+// m and m^2, and the bracket of the formula above
+template <int ORDER, typename T, typename V4>
+__device__ __forceinline__ T far_field_bracket(T x, T y, T z, T m, const V4& b, const V4& c, const V4& d, const V4& e,
+                                               const V4& f) {
+  // explicit multiply-adds (no compiler contraction): every kernel that
+  // inlines this computes each term bit for bit the same
+  x *= m;
+  y *= m;
+  z *= m;
+  T t = fma(z, b.z, fma(y, b.y, x * b.x));  // x.b
+  if (ORDER >= 1) {
+    const T q1 = fma(d.y, z, fma(c.w, y, c.x * x)), q2 = fma(d.x, z, c.y * y);
+    T qf = fma(x, q1, fma(y, q2, c.z));
+    if (ORDER >= 2) {
+      const T g1 = fma(e.z, z, fma(e.y, y, d.z * x)), g2 = fma(f.w, z, e.w * y), g3 = fma(f.x, z, d.w * y);
+      const T gx = fma(x, g1, fma(y, g2, f.y)), gy = fma(y, g3, f.z);
+      qf = fma(m, fma(x, gx, fma(y, gy, e.x * z)), qf);
+    }
+    t = fma(m, qf, t);
+  }
+  return t;
+}
+
+// the FP32 value; a caller that sums it may add m * m * bracket by itself
 template <int ORDER>
 __device__ __forceinline__ float far_field_poly(float x, float y, float z, float l2, const float4& b,
                                                 const float4& c, const float4& d, const float4& e,
                                                 const float4& f) {
-  // explicit multiply-adds (no compiler contraction): every kernel that
-  // inlines this computes each term bit for bit the same
   const float m = __builtin_amdgcn_rsqf(l2);
-  x *= m;
-  y *= m;
-  z *= m;
-  float t = fmaf(z, b.z, fmaf(y, b.y, x * b.x));  // x.b
-  if (ORDER >= 1) {
-    const float z2 = z * z;
-    const float q1 = fmaf(d.y, z, fmaf(c.w, y, c.x * x)), q2 = fmaf(d.x, z, c.y * y);
-    float qf = fmaf(c.z, z2, fmaf(y, q2, x * q1));
-    if (ORDER >= 2) {
-      const float g1 = fmaf(e.z, z, fmaf(e.y, y, d.z * x)), g2 = fmaf(f.w, z, e.w * y);
-      const float gx = fmaf(f.y, z2, fmaf(y, g2, x * g1));
-      const float gy = fmaf(f.z, z2, y * fmaf(f.x, z, d.w * y));
-      const float g = fmaf(e.x, z2 * z, fmaf(y, gy, x * gx));
-      qf = fmaf(m, g, qf);
-    }
-    t = fmaf(m, qf, t);
-  }
-  return (m * m) * t;
+  return (m * m) * far_field_bracket<ORDER>(x, y, z, m, b, c, d, e, f);
 }
+
+// Coefficients of an expansion in the record form of far_field_bracket:
+// b.xyz; the quadratic form by xx yy zz xy yz xz; the cubic by
+// x^3 y^3 z^3 x^2y x^2z xy^2 y^2z xz^2 yz^2 xyz.  r: the 20 values of
+// b c d e f (r[3], the free fourth value of b, is not written).
+template <typename T>
+__device__ __forceinline__ void pack_far_field(const double* b, const double* q, const double* g, T* r) {
+  for (int k = 0; k < 3; ++k) r[k] = (T)b[k];
+  r[4] = (T)(q[0] - q[2]);   // c.x  x^2
+  r[5] = (T)(q[1] - q[2]);   // c.y  y^2
+  r[6] = (T)q[2];            // c.z  1
+  r[7] = (T)q[3];            // c.w  xy
+  r[8] = (T)q[4];            // d.x  yz
+  r[9] = (T)q[5];            // d.y  xz
+  r[10] = (T)(g[0] - g[7]);  // d.z  x^3
+  r[11] = (T)(g[1] - g[8]);  // d.w  y^3
+  r[12] = (T)g[2];           // e.x  z
+  r[13] = (T)(g[3] - g[8]);  // e.y  x^2y
+  r[14] = (T)(g[4] - g[2]);  // e.z  x^2z
+  r[15] = (T)(g[5] - g[7]);  // e.w  xy^2
+  r[16] = (T)(g[6] - g[2]);  // f.x  y^2z
+  r[17] = (T)g[7];           // f.y  x
+  r[18] = (T)g[8];           // f.z  y
+  r[19] = (T)g[9];           // f.w  xyz
+}
+
+// A running sum of angles atan2(y, x), kept as the product of the x + i y
+// scaled by powers of two and the number of full turns: the sum is
+// 2 pi turns + atan2(im, re).  A term costs a complex multiplication, a
+// rescaling and the turn count (16 operations) where an atan2 of its own
+// costs about 25 in FP32 and over 100 in FP64, and each multiplication moves
+// the angle by at most about one unit of rounding of 1 rad, where a running
+// sum of angles rounds at the size of the sum.
+template <typename T>
+struct AngleSum {
+  T re = T(1), im = T(0);
+  int32_t turns = 0;
+
+  // Adds atan2(y, x) (y, x not NaN, not both zero, their product with the
+  // unit-sized sum neither overflowing nor vanishing) and returns true;
+  // otherwise leaves the sum as it is and returns false.
+  __device__ __forceinline__ bool add(T y, T x) {
+    const T r = fma(-im, y, re * x), i = fma(re, y, im * x);
+    const T s = fmax(fabs(r), fabs(i));
+    if (!(s > T(0) && s < T(INFINITY))) return false;
+    // both arguments on one side of the real axis and the product on the
+    // other: the sum of the two left [-pi, pi]
+    const int32_t a = sign_word(im), b = sign_word(y), c = sign_word(i);
+    turns += ((~(a ^ b) & (a ^ c)) >> 31) & ((a >> 31) | 1);
+    const int e = -frexp_exponent(s);
+    re = scale(r, e);
+    im = scale(i, e);
+    return true;
+  }
+  __device__ __forceinline__ double total() const {
+    return fma((double)turns, 6.283185307179586476925286766559, (double)argument(im, re));
+  }
+
+ private:
+  static __device__ __forceinline__ float argument(float y, float x) { return atan2_fast(y, x); }
+  static __device__ __forceinline__ double argument(double y, double x) { return atan2(y, x); }
+  static __device__ __forceinline__ int32_t sign_word(float v) { return __float_as_int(v); }
+  static __device__ __forceinline__ int32_t sign_word(double v) { return __double2hiint(v); }
+  static __device__ __forceinline__ int frexp_exponent(float v) { return __builtin_amdgcn_frexp_expf(v); }
+  static __device__ __forceinline__ int frexp_exponent(double v) { return __builtin_amdgcn_frexp_exp(v); }
+  static __device__ __forceinline__ float scale(float v, int e) { return __builtin_ldexpf(v, e); }
+  static __device__ __forceinline__ double scale(double v, int e) { return __builtin_ldexp(v, e); }
+};
 
 }  // namespace gwn

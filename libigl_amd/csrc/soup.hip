@@ -178,20 +178,32 @@ __global__ void k_positions(const int32_t* __restrict__ level_nodes, int64_t cou
   }
 }
 
-// Slot record (6 x float4):
-//   0: P.x P.y P.z maxP2          1: -N.x -N.y -N.z link
-//   2: A B C Dxy                  3: Dyz Dzx g300 g030
-//   4: g003 g210 g201 g120        5: g021 g102 g012 g111
-// The far-field terms of the reference (7199-7245), with x = q/|q|:
+// Slot record (6 x float4): [P.xyz, maxP2] and the far field of
+// far_field_bracket (device_math.h) for b = -N with the link word in b.w.
+// The reference's terms (7199-7245), with x = q/|q|:
 //   -(x.N)/|q|^2 + (tr Nd - 3 x'Nd x)/|q|^3 + (1.5 (x.s) - 7.5 K(x))/|q|^4,
 // s and the cubic K as in the reference (temp0/temp1), are rewritten with
-// |x| = 1 as m^2 [ x.(-N) + m ( Qf(x) + m G(x) ) ], m = 1/|q|, where
-// Qf(x) = A x^2 + B y^2 + C z^2 + Dxy xy + Dyz yz + Dzx zx with
-// A = tr - 3 Ndx ... and Dxy = -3 (Nxy+Nyx) ..., and the cubic
-// G(x) = 1.5 (s.x) |x|^2 - 7.5 K(x) with coefficients g_ijk (of x^i y^j z^k).
-// The coefficients are formed in FP64 from the reference's FP32 BoxData and
-// rounded once.
-// link = skip index for an internal child, LINK_LEAF|triangle for an item.
+// |x| = 1 as m^2 [ x.(-N) + m ( Qf(x) + m G(x) ) ], m = 1/|q|, with the
+// quadratic form Qf(x) = tr |x|^2 - 3 x'Nd x and the cubic
+// G(x) = 1.5 (s.x) |x|^2 - 7.5 K(x).  The coefficients are formed in FP64 from
+// the BoxData of the record's precision (the reference's in FP32) and rounded
+// once.  link = skip index for an internal child, LINK_LEAF|triangle for an item.
+template <typename T>
+__device__ __forceinline__ void slot_far_field(const T* __restrict__ bd, int s, T* r) {
+  const double nd0 = bd[BD_ND + s], nd1 = bd[BD_ND + 4 + s], nd2 = bd[BD_ND + 8 + s];
+  const double tr = nd0 + nd1 + nd2;
+  const double k0 = bd[BD_NKD + s], k1 = bd[BD_NKD + 4 + s], k2 = bd[BD_NKD + 8 + s];
+  const double cxxy = bd[BD_CXXY + s], cxxz = bd[BD_CXXZ + s], cyyz = bd[BD_CYYZ + s];
+  const double cyyx = bd[BD_CYYX + s], czzx = bd[BD_CZZX + s], czzy = bd[BD_CZZY + s];
+  const double s0 = 3.0 * k0 + (cyyx + czzx), s1 = 3.0 * k1 + (czzy + cxxy), s2 = 3.0 * k2 + (cxxz + cyyz);
+  const double b[3] = {-(double)bd[BD_N + s], -(double)bd[BD_N + 4 + s], -(double)bd[BD_N + 8 + s]};
+  const double q[6] = {tr - 3.0 * nd0, tr - 3.0 * nd1, tr - 3.0 * nd2, -3.0 * (double)bd[BD_NXY + s],
+                       -3.0 * (double)bd[BD_NYZ + s], -3.0 * (double)bd[BD_NZX + s]};
+  const double g[10] = {1.5 * s0 - 7.5 * k0,   1.5 * s1 - 7.5 * k1,   1.5 * s2 - 7.5 * k2,   1.5 * s1 - 7.5 * cxxy,
+                        1.5 * s2 - 7.5 * cxxz, 1.5 * s0 - 7.5 * cyyx, 1.5 * s2 - 7.5 * cyyz, 1.5 * s0 - 7.5 * czzx,
+                        1.5 * s1 - 7.5 * czzy, -7.5 * (double)bd[BD_SP + s]};
+  pack_far_field(b, q, g, r);
+}
 __global__ void k_write_slots(int64_t nn, const uint32_t* __restrict__ nodes, const float* __restrict__ boxdata,
                               const uint32_t* __restrict__ nslots_sub, const uint32_t* __restrict__ first_slot,
                               float4* __restrict__ slots) {
@@ -211,27 +223,17 @@ __global__ void k_write_slots(int64_t nn, const uint32_t* __restrict__ nodes, co
       link = LINK_LEAF | c;
     }
     float4* r = slots + 6 * (int64_t)pos;
-    const double nd0 = bd[BD_ND + s], nd1 = bd[BD_ND + 4 + s], nd2 = bd[BD_ND + 8 + s];
-    const double tr = nd0 + nd1 + nd2;
-    const double k0 = bd[BD_NKD + s], k1 = bd[BD_NKD + 4 + s], k2 = bd[BD_NKD + 8 + s];
-    const double cxxy = bd[BD_CXXY + s], cxxz = bd[BD_CXXZ + s], cyyz = bd[BD_CYYZ + s];
-    const double cyyx = bd[BD_CYYX + s], czzx = bd[BD_CZZX + s], czzy = bd[BD_CZZY + s];
-    const double s0 = 3.0 * k0 + (cyyx + czzx), s1 = 3.0 * k1 + (czzy + cxxy), s2 = 3.0 * k2 + (cxxz + cyyz);
+    float v[20];
+    slot_far_field(bd, s, v);
     r[0] = make_float4(bd[BD_P + s], bd[BD_P + 4 + s], bd[BD_P + 8 + s], bd[BD_MAXP2 + s]);
-    r[1] = make_float4(-bd[BD_N + s], -bd[BD_N + 4 + s], -bd[BD_N + 8 + s], __uint_as_float(link));
-    r[2] = make_float4((float)(tr - 3.0 * nd0), (float)(tr - 3.0 * nd1), (float)(tr - 3.0 * nd2),
-                       (float)(-3.0 * (double)bd[BD_NXY + s]));
-    r[3] = make_float4((float)(-3.0 * (double)bd[BD_NYZ + s]), (float)(-3.0 * (double)bd[BD_NZX + s]),
-                       (float)(1.5 * s0 - 7.5 * k0), (float)(1.5 * s1 - 7.5 * k1));
-    r[4] = make_float4((float)(1.5 * s2 - 7.5 * k2), (float)(1.5 * s1 - 7.5 * cxxy), (float)(1.5 * s2 - 7.5 * cxxz),
-                       (float)(1.5 * s0 - 7.5 * cyyx));
-    r[5] = make_float4((float)(1.5 * s2 - 7.5 * cyyz), (float)(1.5 * s0 - 7.5 * czzx), (float)(1.5 * s1 - 7.5 * czzy),
-                       (float)(-7.5 * (double)bd[BD_SP + s]));
+    r[1] = make_float4(v[0], v[1], v[2], __uint_as_float(link));
+    for (int k = 1; k < 5; ++k) r[1 + k] = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
     pos = next;
   }
 }
 
-// FP64 slot record: 24 doubles in the same field order (link kept in the FP32 record).
+// FP64 slot record: 24 doubles in the order of the FP32 record's 24 floats,
+// the link word in the low half of the eighth.
 __global__ void k_write_slots64(int64_t nn, const uint32_t* __restrict__ nodes, const double* __restrict__ bd64,
                                 const uint32_t* __restrict__ first_slot, const uint32_t* __restrict__ nslots_sub,
                                 double* __restrict__ slots64) {
@@ -242,32 +244,15 @@ __global__ void k_write_slots64(int64_t nn, const uint32_t* __restrict__ nodes, 
   for (int s = 0; s < 4; ++s) {
     const uint32_t c = nodes[4 * node + s];
     if (c == NODE_EMPTY) break;
+    const uint32_t next = (c & NODE_INTERNAL) ? pos + 1 + nslots_sub[c & ~NODE_INTERNAL] : pos + 1;
     double* r = slots64 + 24 * (int64_t)pos;
-    r[0] = bd[BD_P + s];
-    r[1] = bd[BD_P + 4 + s];
-    r[2] = bd[BD_P + 8 + s];
+    for (int k = 0; k < 3; ++k) r[k] = bd[BD_P + 4 * k + s];
     r[3] = bd[BD_MAXP2 + s];
-    r[4] = bd[BD_N + s];
-    r[5] = bd[BD_N + 4 + s];
-    r[6] = bd[BD_N + 8 + s];
-    r[7] = 0.0;
-    r[8] = bd[BD_ND + s];
-    r[9] = bd[BD_ND + 4 + s];
-    r[10] = bd[BD_ND + 8 + s];
-    r[11] = bd[BD_NXY + s];
-    r[12] = bd[BD_NYZ + s];
-    r[13] = bd[BD_NZX + s];
-    r[14] = bd[BD_NKD + s];
-    r[15] = bd[BD_NKD + 4 + s];
-    r[16] = bd[BD_NKD + 8 + s];
-    r[17] = bd[BD_SP + s];
-    r[18] = bd[BD_CXXY + s];
-    r[19] = bd[BD_CXXZ + s];
-    r[20] = bd[BD_CYYZ + s];
-    r[21] = bd[BD_CYYX + s];
-    r[22] = bd[BD_CZZX + s];
-    r[23] = bd[BD_CZZY + s];
-    pos += (c & NODE_INTERNAL) ? 1 + nslots_sub[c & ~NODE_INTERNAL] : 1;
+    double v[20];
+    slot_far_field(bd, s, v);
+    v[3] = __longlong_as_double((long long)((c & NODE_INTERNAL) ? next : (LINK_LEAF | c)));
+    for (int k = 0; k < 20; ++k) r[4 + k] = v[k];
+    pos = next;
   }
 }
 
@@ -430,38 +415,57 @@ __device__ __forceinline__ float tri_solid_angle_fast(float ax, float ay, float 
   return 2.0f * atan2_fast(num, den);
 }
 
-// Far-field Taylor value of one child slot (SolidAngleFunctors::pre,
-// 7199-7245) from the reference's moment layout (FP64 records), for
-// q = query - P already formed and l2 = |q|^2.
-template <int ORDER, typename T, typename V4>
-__device__ __forceinline__ T far_field(T x, T y, T z, T l2, const V4& b, const V4& c, const V4& d, const V4& e,
-                                       const V4& f) {
-#pragma clang fp contract(fast)
-  const T m2 = T(1) / l2;
-  const T m1 = sqrt(m2);
-  x *= m1;
-  y *= m1;
-  z *= m1;
-  T o = -m2 * (x * b.x + y * b.y + z * b.z);
-  if (ORDER >= 1) {
-    const T x2 = x * x, y2 = y * y, z2 = z * z;
-    const T m3 = m2 * m1;
-    o += m3 * (c.x + c.y + c.z - T(3) * ((x2 * c.x + y2 * c.y + z2 * c.z) + x * y * c.w + x * z * d.y + y * z * d.x));
-    if (ORDER >= 2) {
-      const T m4 = m2 * m2;
-      // temp0 / temp1 of the reference
-      const T t00 = f.y + f.z, t01 = f.w + e.z, t02 = e.w + f.x;
-      const T t10 = y * e.z + z * e.w, t11 = z * f.x + x * f.y, t12 = x * f.z + y * f.w;
-      const T s0 = T(3) * d.z + t00, s1 = T(3) * d.w + t01, s2 = T(3) * e.x + t02;
-      o += m4 * (T(1.5) * (x * s0 + y * s1 + z * s2) -
-                 T(7.5) * ((x2 * x * d.z + y2 * y * d.w + z2 * z * e.x) + x * y * z * e.y + (x2 * t10 + y2 * t11 + z2 * t12)));
-    }
-  }
-  return o;
-}
-
 struct D4 {
   double x, y, z, w;
+};
+
+// 1/sqrt(x) to FP64 rounding: the hardware estimate (about 2^-26 relative) and
+// one third-order step
+__device__ __forceinline__ double rsqrt64(double x) {
+  const double r = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * r), r, 1.0);
+  return fma(r * e, fma(0.375, e, 0.5), r);
+}
+__device__ __forceinline__ float tri_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
+__device__ __forceinline__ double tri_rsqrt(double x) { return rsqrt64(x); }
+
+// Signed solid angles of triangles (UTsignedSolidAngleTri, 6070-6110), summed.
+// The half angles atan2(num, den) go into an AngleSum; a term it does not
+// take, and a triangle with a corner (nearly) at the query, is summed on its
+// own as the per-triangle functions above give it.
+template <typename T>
+struct SolidAngleSum {
+  AngleSum<T> half;
+  T extra = T(0);
+
+  __device__ __forceinline__ void add(const float* __restrict__ p, T qx, T qy, T qz) {
+    constexpr T tiny = sizeof(T) == 4 ? T(1e-30) : T(1e-290);  // keeps the reciprocal square roots away from denormals
+    T a0 = p[0] - qx, a1 = p[1] - qy, a2 = p[2] - qz;
+    T b0 = p[3] - qx, b1 = p[4] - qy, b2 = p[5] - qz;
+    T c0 = p[6] - qx, c1 = p[7] - qy, c2 = p[8] - qz;
+    const T la = fma(a2, a2, fma(a1, a1, a0 * a0));
+    const T lb = fma(b2, b2, fma(b1, b1, b0 * b0));
+    const T lc = fma(c2, c2, fma(c1, c1, c0 * c0));
+    if (fmin(la, fmin(lb, lc)) < tiny) {
+      extra += tri_solid_angle<T>(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], qx, qy, qz);
+      return;
+    }
+    const T ra = tri_rsqrt(la), rb = tri_rsqrt(lb), rc = tri_rsqrt(lc);
+    a0 *= ra; a1 *= ra; a2 *= ra;
+    b0 *= rb; b1 *= rb; b2 *= rb;
+    c0 *= rc; c1 *= rc; c2 *= rc;
+    const T u0 = b0 - a0, u1 = b1 - a1, u2 = b2 - a2;
+    const T w0 = c0 - a0, w1 = c1 - a1, w2 = c2 - a2;
+    const T k0 = fma(u1, w2, -(u2 * w1)), k1 = fma(u2, w0, -(u0 * w2)), k2 = fma(u0, w1, -(u1 * w0));
+    const T num = fma(a2, k2, fma(a1, k1, a0 * k0));
+    if (num == T(0)) return;
+    const T ab = fma(a2, b2, fma(a1, b1, a0 * b0));
+    const T ac = fma(a2, c2, fma(a1, c1, a0 * c0));
+    const T bc = fma(b2, c2, fma(b1, c1, b0 * c0));
+    const T den = ((T(1) + ab) + ac) + bc;
+    if (!half.add(num, den)) extra += T(2) * atan2(num, den);
+  }
+  __device__ __forceinline__ double total() const { return (double)extra + 2.0 * half.total(); }
 };
 
 // ---------------------------------------------------------------------------
@@ -491,7 +495,7 @@ __device__ __forceinline__ uint32_t wave_uniform(uint32_t v) { return __builtin_
 // 6070-6110, in double) and summed in an FP64 accumulator of its own; the far
 // field and every other exact term go to the FP32 running sum.
 __device__ __forceinline__ bool near_triangle(float maxp2, float l2, float near_d) {
-  const float rr = sqrtf(maxp2) + near_d;
+  const float rr = __builtin_amdgcn_sqrtf(maxp2) + near_d;
   return l2 < rr * rr;
 }
 
@@ -512,34 +516,43 @@ struct NearList {
   uint32_t n;     // kDefer + 1 after an overflow
 };
 
-// Exact term of a near triangle slot: added to sum (FP32) or, in the mixed
-// form for a triangle near the query, noted for the FP64 sum.
-template <bool MIXED>
-__device__ __forceinline__ void exact_term(const float* __restrict__ tri, uint32_t t, float maxp2, float l2, float qx,
-                                           float qy, float qz, float near_d, float& sum, NearList& L) {
-  if (MIXED && near_triangle(maxp2, l2, near_d)) {
-    if (L.n < (uint32_t)kDefer) L.lds[L.n * kTravThreads] = t;
-    L.n = L.n < (uint32_t)kDefer ? L.n + 1 : (uint32_t)kDefer + 1;
-  } else {
-    const float* p = tri + 9 * (size_t)t;
-    sum = __fadd_rn(sum, tri_solid_angle_fast(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], qx, qy, qz));
-  }
+__device__ __forceinline__ void note_near(NearList& L, uint32_t t) {
+  if (L.n < (uint32_t)kDefer) L.lds[L.n * kTravThreads] = t;
+  L.n = L.n < (uint32_t)kDefer ? L.n + 1 : (uint32_t)kDefer + 1;
 }
 
-// W of a walk: the FP32 sum, plus (mixed form) the noted near triangles'
-// FP64 solid angles summed in order; NaN after an overflow.
-template <bool MIXED>
-__device__ __forceinline__ double finish_walk(float sum, const NearList& L, const float* __restrict__ tri, float qx,
-                                              float qy, float qz) {
-  if (!MIXED) return (double)sum / (4.0 * PI_D);
-  if (L.n > (uint32_t)kDefer) return __longlong_as_double(0x7FF8000000000000ll);
-  double sum_near = 0.0;
-  for (uint32_t k = 0; k < L.n; ++k) {
-    const float* p = tri + 9 * (size_t)L.lds[k * kTravThreads];
-    sum_near = __dadd_rn(sum_near,
-                         tri_solid_angle<double>(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], qx, qy, qz));
+// Exact triangles of the wave-coherent walks wait in a per-lane LDS list until
+// some lane's is full; then every lane evaluates its own.  At a record only
+// the lanes near that triangle need it (61 of a lane's 1,180 records on the
+// 81,920-triangle workload at accuracy_scale 4.9, but some lane at 133 of the
+// wavefront's 1,502), so evaluating it there keeps the other lanes idle for
+// some 90 instructions; together the lanes take about 72 turns.  A lane's
+// triangles enter its sum in the order met, whatever its neighbours do, so a
+// query's result does not depend on its wavefront.
+template <int N>
+struct Pending {
+  uint32_t* lds;  // column threadIdx.x of an N x kTravThreads array
+  uint32_t n = 0;
+  __device__ __forceinline__ void push(uint32_t t) { lds[n++ * kTravThreads] = t; }
+  template <typename T>
+  __device__ __forceinline__ void flush(const float* __restrict__ tri, T qx, T qy, T qz, SolidAngleSum<T>& ex) {
+    for (uint32_t k = 0; k < n; ++k) ex.add(tri + 9 * (size_t)lds[k * kTravThreads], qx, qy, qz);
+    n = 0;
   }
-  return ((double)sum + sum_near) / (4.0 * PI_D);
+};
+
+// W of a walk: the far fields' FP32 sum and the exact triangles' angles, plus
+// (mixed form) the noted near triangles' FP64 solid angles summed in order;
+// NaN after an overflow.
+template <bool MIXED>
+__device__ __forceinline__ double finish_walk(float sum, const SolidAngleSum<float>& ex, const NearList& L,
+                                              const float* __restrict__ tri, float qx, float qy, float qz) {
+  const double w = (double)sum + ex.total();
+  if (!MIXED) return w / (4.0 * PI_D);
+  if (L.n > (uint32_t)kDefer) return __longlong_as_double(0x7FF8000000000000ll);
+  SolidAngleSum<double> near;
+  for (uint32_t k = 0; k < L.n; ++k) near.add(tri + 9 * (size_t)L.lds[k * kTravThreads], qx, qy, qz);
+  return (w + near.total()) / (4.0 * PI_D);
 }
 
 // Both walks are held to 8 wavefronts per SIMD (64 VGPRs): the walk loop fits
@@ -552,7 +565,8 @@ __device__ __forceinline__ double finish_walk(float sum, const NearList& L, cons
 template <int ORDER, bool MIXED>
 __device__ __forceinline__ void lane_walk(const float4* __restrict__ slots, uint32_t nslots,
                                           const float* __restrict__ tri, uint32_t j, float qx, float qy, float qz,
-                                          float acc2, float near_d, float& sum, NearList& L) {
+                                          float acc2, float near_d, float& sum, SolidAngleSum<float>& ex,
+                                          NearList& L) {
   while (j < nslots) {
     const float4* r = slots + 6 * (size_t)j;
     const float4 a = r[0], b = r[1];
@@ -570,14 +584,19 @@ __device__ __forceinline__ void lane_walk(const float4* __restrict__ slots, uint
         e = r[4];
         f = r[5];
       }
-      const float o = far_field_poly<ORDER>(x, y, z, l2, b, c, d, e, f);
-      if (isfinite(o)) {
-        sum = __fadd_rn(sum, o);
+      const float m = __builtin_amdgcn_rsqf(l2);
+      const float o = far_field_bracket<ORDER>(x, y, z, m, b, c, d, e, f), m2 = __fmul_rn(m, m);
+      if (isfinite(__fmul_rn(m2, o))) {  // otherwise the reference descends / evaluates the item
+        sum = fmaf(m2, o, sum);
         j = leaf ? j + 1 : link;
         continue;
       }
     }
-    if (leaf) exact_term<MIXED>(tri, link & ~LINK_LEAF, a.w, l2, qx, qy, qz, near_d, sum, L);
+    if (leaf) {
+      const uint32_t t = link & ~LINK_LEAF;
+      if (MIXED && near_triangle(a.w, l2, near_d)) note_near(L, t);
+      else ex.add(tri + 9 * (size_t)t, qx, qy, qz);
+    }
     ++j;
   }
 }
@@ -591,6 +610,17 @@ __device__ __forceinline__ float in_vgpr(float x) {
   return v;
 }
 
+// Lane masks of a wavefront held in scalar registers.  (A condition kept as a
+// bool and balloted later costs two VALU instructions more.)
+__device__ __forceinline__ uint64_t lanes_at_most(uint32_t v, uint32_t i) {
+  return __builtin_amdgcn_uicmp(v, i, 37);  // ICMP_ULE
+}
+__device__ __forceinline__ uint64_t lanes_beyond(float l2, float r2) {
+  return __builtin_amdgcn_fcmpf(l2, r2, 10);  // FCMP_UGT: !(l2 <= r2)
+}
+__device__ __forceinline__ uint64_t lanes_beyond(double l2, double r2) { return __builtin_amdgcn_fcmp(l2, r2, 10); }
+__device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+
 // HANDOVER: a wavefront whose lanes have stopped sharing records (fewer than
 // 16 lanes per step on average over a window of 256 steps: the union of their
 // paths exceeds the longest by far, as on fans of thin triangles) hands over
@@ -598,6 +628,17 @@ __device__ __forceinline__ float in_vgpr(float x) {
 // unchanged (same records, terms and order); the check costs about a tenth of
 // the walk's time on coherent batches, so only latency-bound callers (the
 // serving engine, on large trees) take it.
+//
+// The walk is bound by VALU issue, so its step holds only what a lane cannot
+// do without: which lanes take part, are far and stay near is kept in scalar
+// lane masks, and a far field is added without asking whether it is finite.
+// The reference descends where it is not; a sum that ends up not finite is
+// walked again by lane_walk, which asks.  A step takes 12 VALU instructions, a
+// far field 32 more and a waiting triangle's turn about 75: 66,000 per
+// wavefront on 81,920 triangles, 1M queries, accuracy_scale 4.9 (82,700 with
+// the conditions in VGPRs, the homogeneous polynomial and each triangle
+// evaluated, with an atan2 of its own, where it is met), and 1.70 ms a call
+// against 2.06; 1.31M triangles, 10M queries, mixed form: 19.4 against 22.4.
 template <int ORDER, bool MIXED, bool HANDOVER>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_traverse(
     const float4* __restrict__ slots, uint32_t nslots, const float* __restrict__ tri, const float* __restrict__ Q,
@@ -609,13 +650,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
   const int64_t qi = perm ? (int64_t)perm[t] : t;
   const float qx = Q[3 * qi], qy = Q[3 * qi + 1], qz = Q[3 * qi + 2];
   float sum = 0.0f;
-  __shared__ uint32_t near_lds[MIXED ? kDefer * kTravThreads : 1];  // mixed form: noted near triangles
+  SolidAngleSum<float> ex;
+  // mixed form: the noted near triangles take LDS too, and eight blocks of it
+  // fit a CU only with a shorter list of waiting ones
+  constexpr int kPend = MIXED ? 4 : 16;
+  __shared__ uint32_t pend_lds[kPend * kTravThreads];
+  __shared__ uint32_t near_lds[MIXED ? kDefer * kTravThreads : 1];
+  Pending<kPend> pend{pend_lds + threadIdx.x};
   NearList L{near_lds + threadIdx.x, 0};
   uint32_t skip = 0;
   uint32_t i = 0;
   uint32_t steps = 0, taken = 0;  // wave-uniform: steps in this window, lanes taking part summed over them
   while (i < nslots) {
-    if (HANDOVER) taken += (uint32_t)__popcll(__ballot(skip <= i));  // lanes taking part in record i
     const float4* r = slots + 6 * (size_t)i;
     const float4 a = r[0], b = r[1];
     float4 c, d, e, f;
@@ -640,88 +686,138 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     // skip >= i holds for every lane (nested intervals), so skip <= i means
     // skip == i; a lane that descends or evaluates an item leaves skip at i,
     // which is <= i + 1, the record it needs next
-    if (skip <= i) {
-      const float x = qx - a.x, y = qy - a.y, z = qz - a.z;
-      // |q-P|^2 rounded as the reference rounds it (no fused multiply-add),
-      // so every near/far decision is the reference's
-      const float l2 = __fadd_rn(__fadd_rn(__fmul_rn(x, x), __fmul_rn(y, y)), __fmul_rn(z, z));
-      bool exact = leaf;
-      if (!(l2 <= __fmul_rn(a.w, acc2))) {
-        const float o = far_field_poly<ORDER>(x, y, z, l2, b, c, d, e, f);
-        if (isfinite(o)) {  // otherwise the reference descends / evaluates the item
-          sum = __fadd_rn(sum, o);
-          exact = false;
-          skip = past;
-        }
-      }
-      if (exact) exact_term<MIXED>(tri, link & ~LINK_LEAF, a.w, l2, qx, qy, qz, near_d, sum, L);
+    const uint64_t part = lanes_at_most(skip, i);
+    const float x = qx - a.x, y = qy - a.y, z = qz - a.z;
+    // |q-P|^2 rounded as the reference rounds it (no fused multiply-add),
+    // so every near/far decision is the reference's
+    const float l2 = __fadd_rn(__fadd_rn(__fmul_rn(x, x), __fmul_rn(y, y)), __fmul_rn(z, z));
+    const uint64_t beyond = lanes_beyond(l2, __fmul_rn(a.w, acc2));
+    if (lane_in(part & beyond)) {
+      const float m = __builtin_amdgcn_rsqf(l2);
+      sum = fmaf(__fmul_rn(m, m), far_field_bracket<ORDER>(x, y, z, m, b, c, d, e, f), sum);
+      skip = past;
     }
-    const bool step = leaf || __ballot(skip <= i + 1) != 0;
-    i = wave_uniform(step ? i + 1 : link);
+    const uint64_t stay = part & ~beyond;
+    if (leaf && stay != 0) {
+      if (lane_in(stay)) {
+        const uint32_t tr = link & ~LINK_LEAF;
+        if (MIXED && near_triangle(a.w, l2, near_d)) note_near(L, tr);
+        else pend.push(tr);
+      }
+      if (__ballot(pend.n == (uint32_t)kPend) != 0) pend.flush(tri, qx, qy, qz, ex);
+    }
+    i = wave_uniform((leaf || stay != 0) ? i + 1 : link);
+    if (HANDOVER) taken += (uint32_t)__popcll(part);
     if (HANDOVER && ++steps == 256) {
       if (taken < 256u * 16u) break;
       steps = taken = 0;
     }
   }
+  pend.flush(tri, qx, qy, qz, ex);
   // after a hand-over each lane continues from the record it needs next
   if (HANDOVER && i < nslots)
-    lane_walk<ORDER, MIXED>(slots, nslots, tri, skip > i ? skip : i, qx, qy, qz, acc2, near_d, sum, L);
-  W[qi] = finish_walk<MIXED>(sum, L, tri, qx, qy, qz);
+    lane_walk<ORDER, MIXED>(slots, nslots, tri, skip > i ? skip : i, qx, qy, qz, acc2, near_d, sum, ex, L);
+  // a query that is not finite meets no finite term: its sum stays NaN
+  if (!isfinite(sum) && isfinite(qx) && isfinite(qy) && isfinite(qz)) {
+    sum = 0.0f;
+    ex = SolidAngleSum<float>();
+    L.n = 0;
+    lane_walk<ORDER, MIXED>(slots, nslots, tri, 0, qx, qy, qz, acc2, near_d, sum, ex, L);
+  }
+  W[qi] = finish_walk<MIXED>(sum, ex, L, tri, qx, qy, qz);
+}
+
+// FP64 term of record i for query q: adds a far-field or exact term to part
+// and ex and returns true, or returns false when the walk descends into the
+// record.  link: the record's link word.
+template <int ORDER>
+__device__ __forceinline__ bool record_term64(const double* __restrict__ s64, const float* __restrict__ tri,
+                                              uint32_t i, uint32_t& link, double qx, double qy, double qz,
+                                              double acc2, double& part, SolidAngleSum<double>& ex) {
+  const double* r = s64 + 24 * (size_t)i;
+  const D4 b{r[4], r[5], r[6], r[7]};
+  link = (uint32_t)__double_as_longlong(b.w);
+  const double x = qx - r[0], y = qy - r[1], z = qz - r[2];
+  const double l2 = x * x + y * y + z * z;
+  if (!(l2 <= r[3] * acc2)) {
+    const D4 c{r[8], r[9], r[10], r[11]}, d{r[12], r[13], r[14], r[15]}, e{r[16], r[17], r[18], r[19]},
+        f{r[20], r[21], r[22], r[23]};
+    const double m = rsqrt64(l2), m2 = __dmul_rn(m, m);
+    const double o = far_field_bracket<ORDER>(x, y, z, m, b, c, d, e, f);
+    if (isfinite(__dmul_rn(m2, o))) {
+      part = fma(m2, o, part);
+      return true;
+    }
+  }
+  if (!(link & LINK_LEAF)) return false;
+  ex.add(tri + 9 * (size_t)(link & ~LINK_LEAF), qx, qy, qz);
+  return true;
 }
 
 // all-FP64 form: FP64 moments, far field, atan2 and sum
+// The step of k_traverse in FP64, bound by FP64 VALU issue on large batches
+// and by the length of its few wavefronts on small ones.  The far field as
+// one polynomial with a refined reciprocal square root (it was a division, a
+// square root and the moments' own form, about twice the operations) and the
+// triangles as one AngleSum took 200,003 queries on 81,920 triangles at
+// accuracy_scale 2 from 0.92 to 0.55 ms.  Eight wavefronts per SIMD (64 VGPRs,
+// some spilled outside the step): 1.5M queries at 4.9 took 3.97 ms at eight,
+// 4.43 at seven, 4.63 at six, 4.50 at five and 4.96 at four.
+constexpr int kPend64 = 16;
 template <int ORDER>
-// Eight wavefronts per SIMD (64 VGPRs, some spilled): its 92 VGPRs allowed five, and on the
-// 1,310,720-triangle workload (10M queries) the walk took 59.1 ms at five, 56.7 at six, 54.3 at
-// seven and 52.8 at eight.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_traverse64(const float4* __restrict__ slots, const double* __restrict__ s64,
-                                                    uint32_t nslots, const float* __restrict__ tri,
-                                                    const float* __restrict__ Q, const uint32_t* __restrict__ perm,
-                                                    const uint32_t* __restrict__ order, int64_t nq,
-                                                    const uint32_t* __restrict__ dcount, double acc2,
-                                                    double* __restrict__ W) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_traverse64(
+    const double* __restrict__ s64, uint32_t nslots, const float* __restrict__ tri, const float* __restrict__ Q,
+    const uint32_t* __restrict__ perm, const uint32_t* __restrict__ order, int64_t nq, double acc2,
+    double* __restrict__ W) {
   // the same wave-coherent rope walk as k_traverse, over the FP64 records;
-  // dcount (when given) holds the number of queries, read on the device;
   // order (when given) is the block order
   const int64_t t = (int64_t)(order ? order[xcd_block()] : xcd_block()) * blockDim.x + threadIdx.x;
-  if (t >= (dcount ? (int64_t)*dcount : nq)) return;
+  if (t >= nq) return;
   const int64_t qi = perm ? (int64_t)perm[t] : t;
   const double qx = Q[3 * qi], qy = Q[3 * qi + 1], qz = Q[3 * qi + 2];
   double sum = 0.0;
+  SolidAngleSum<double> ex;
+  __shared__ uint32_t pend_lds[kPend64 * kTravThreads];
+  Pending<kPend64> pend{pend_lds + threadIdx.x};
   uint32_t skip = 0;
   uint32_t i = 0;
   while (i < nslots) {
     const double* r = s64 + 24 * (size_t)i;
-    const uint32_t link = __float_as_uint(slots[6 * (size_t)i + 1].w);
-    const double r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3];
-    // the link and the record's point and radius in one scalar-cache round
-    // trip (the compiler would otherwise wait for the link first)
-    asm volatile("" ::"s"(link), "s"(r0), "s"(r3));
+    const D4 a{r[0], r[1], r[2], r[3]}, b{r[4], r[5], r[6], r[7]};
+    asm volatile("" ::"s"(a.x), "s"(b.w));
+    const uint32_t link = (uint32_t)__double_as_longlong(b.w);
     const bool leaf = (link & LINK_LEAF) != 0;
-    if (skip == i) {
-      const double x = qx - r0, y = qy - r1, z = qz - r2;
-      const double l2 = x * x + y * y + z * z;
-      bool exact = leaf;
-      skip = i + 1;
-      if (!(l2 <= r3 * acc2)) {
-        const D4 b{r[4], r[5], r[6], 0.0}, c{r[8], r[9], r[10], r[11]}, d{r[12], r[13], r[14], r[15]},
-            e{r[16], r[17], r[18], r[19]}, f{r[20], r[21], r[22], r[23]};
-        const double o = far_field<ORDER, double, D4>(x, y, z, l2, b, c, d, e, f);
-        if (isfinite(o)) {
-          sum = __dadd_rn(sum, o);
-          exact = false;
-          if (!leaf) skip = link;
-        }
-      }
-      if (exact) {
-        const float* p = tri + 9 * (size_t)(link & ~LINK_LEAF);
-        sum = __dadd_rn(sum, tri_solid_angle<double>(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], qx, qy, qz));
-      }
+    const uint32_t past = leaf ? i + 1 : link;
+    const uint64_t part = lanes_at_most(skip, i);
+    const double x = qx - a.x, y = qy - a.y, z = qz - a.z;
+    const double l2 = x * x + y * y + z * z;
+    const uint64_t beyond = lanes_beyond(l2, a.w * acc2);
+    if (lane_in(part & beyond)) {
+      const D4 c{r[8], r[9], r[10], r[11]}, d{r[12], r[13], r[14], r[15]}, e{r[16], r[17], r[18], r[19]},
+          f{r[20], r[21], r[22], r[23]};
+      const double m = rsqrt64(l2);
+      sum = fma(__dmul_rn(m, m), far_field_bracket<ORDER>(x, y, z, m, b, c, d, e, f), sum);
+      skip = past;
     }
-    const bool step = leaf || __ballot(skip == i + 1) != 0;
-    i = wave_uniform(step ? i + 1 : link);
+    const uint64_t stay = part & ~beyond;
+    if (leaf && stay != 0) {
+      if (lane_in(stay)) pend.push(link & ~LINK_LEAF);
+      if (__ballot(pend.n == (uint32_t)kPend64) != 0) pend.flush(tri, qx, qy, qz, ex);
+    }
+    i = wave_uniform((leaf || stay != 0) ? i + 1 : link);
   }
-  W[qi] = sum / (4.0 * PI_D);
+  pend.flush(tri, qx, qy, qz, ex);
+  if (!isfinite(sum) && isfinite(qx) && isfinite(qy) && isfinite(qz)) {
+    // a far field was not finite: the walk again, descending where it is not
+    sum = 0.0;
+    ex = SolidAngleSum<double>();
+    for (uint32_t j = 0; j < nslots;) {
+      uint32_t link;
+      const bool done = record_term64<ORDER>(s64, tri, j, link, qx, qy, qz, acc2, sum, ex);
+      j = (done && !(link & LINK_LEAF)) ? link : j + 1;
+    }
+  }
+  W[qi] = (sum + ex.total()) / (4.0 * PI_D);
 }
 
 // ---- FP64 re-evaluation of a few scattered queries: one wavefront per query ----
@@ -734,52 +830,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
 // per lane and then across lanes in a fixed order, so the result is
 // deterministic and differs from the sequential sum only by rounding.
 
-// FP64 term of record i for query q: adds a far-field or exact term to part
-// and returns true, or returns false when the walk descends into the record.
-template <int ORDER>
-__device__ __forceinline__ bool record_term64(const double* __restrict__ s64, const float* __restrict__ tri,
-                                              uint32_t i, uint32_t link, double qx, double qy, double qz, double acc2,
-                                              double& part) {
-  const double* r = s64 + 24 * (size_t)i;
-  const bool leaf = (link & LINK_LEAF) != 0;
-  const double x = qx - r[0], y = qy - r[1], z = qz - r[2];
-  const double l2 = x * x + y * y + z * z;
-  if (!(l2 <= r[3] * acc2)) {
-    const D4 b{r[4], r[5], r[6], 0.0}, c{r[8], r[9], r[10], r[11]}, d{r[12], r[13], r[14], r[15]},
-        e{r[16], r[17], r[18], r[19]}, f{r[20], r[21], r[22], r[23]};
-    const double o = far_field<ORDER, double, D4>(x, y, z, l2, b, c, d, e, f);
-    if (isfinite(o)) {
-      part = __dadd_rn(part, o);
-      return true;
-    }
-  }
-  if (!leaf) return false;
-  const float* p = tri + 9 * (size_t)(link & ~LINK_LEAF);
-  part = __dadd_rn(part, tri_solid_angle<double>(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], qx, qy, qz));
-  return true;
-}
-
-
 // FP64 ring walk of query q: W = sum / 4 pi, the same on every lane
 template <int ORDER>
-__device__ __forceinline__ double ring_walk64(uint2* __restrict__ ring, int lane, const float4* __restrict__ slots,
-                                              const double* __restrict__ s64, uint32_t nslots,
-                                              const float* __restrict__ tri, double qx, double qy, double qz,
-                                              double acc2) {
+__device__ __forceinline__ double ring_walk64(uint2* __restrict__ ring, int lane, const double* __restrict__ s64,
+                                              uint32_t nslots, const float* __restrict__ tri, double qx, double qy,
+                                              double qz, double acc2) {
   double part = 0.0;
+  SolidAngleSum<double> ex;
   ring_walk(ring, lane, nslots, [&](uint32_t i, uint32_t& link) {
-    link = __float_as_uint(slots[6 * (size_t)i + 1].w);
-    return record_term64<ORDER>(s64, tri, i, link, qx, qy, qz, acc2, part);
+    return record_term64<ORDER>(s64, tri, i, link, qx, qy, qz, acc2, part, ex);
   });
-  return wave_sum(part) / (4.0 * PI_D);
+  return wave_sum(part + ex.total()) / (4.0 * PI_D);
 }
 
 // list[k] (k itself when list is null) for k < count (count = *dcount when
 // given, else n): 4 queries per 256-thread block, one per wavefront,
 // grid-strided.
 template <int ORDER>
-__global__ __launch_bounds__(256) void k_reeval64(const float4* __restrict__ slots, const double* __restrict__ s64,
-                                                  uint32_t nslots, const float* __restrict__ tri,
+__global__ __launch_bounds__(256) void k_reeval64(const double* __restrict__ s64, uint32_t nslots,
+                                                  const float* __restrict__ tri,
                                                   const float* __restrict__ Q, const uint32_t* __restrict__ list,
                                                   int64_t n, const uint32_t* __restrict__ dcount, double acc2,
                                                   double* __restrict__ W) {
@@ -788,7 +857,7 @@ __global__ __launch_bounds__(256) void k_reeval64(const float4* __restrict__ slo
   const int64_t count = dcount ? (int64_t)*dcount : n;
   for (int64_t k = (int64_t)blockIdx.x * 4 + wv; k < count; k += (int64_t)gridDim.x * 4) {
     const int64_t qi = list ? (int64_t)list[k] : k;
-    const double w = ring_walk64<ORDER>(ring_all[wv], lane, slots, s64, nslots, tri, Q[3 * qi], Q[3 * qi + 1],
+    const double w = ring_walk64<ORDER>(ring_all[wv], lane, s64, nslots, tri, Q[3 * qi], Q[3 * qi + 1],
                                         Q[3 * qi + 2], acc2);
     if (lane == 0) W[qi] = w;
   }
@@ -884,15 +953,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
 // A kernel of its own so that the FP64 walk's registers do not limit the
 // occupancy of the FP32 walk.
 template <int ORDER>
-__global__ __launch_bounds__(256) void k_reeval64_band(const float4* __restrict__ slots,
-                                                       const double* __restrict__ s64, uint32_t nslots,
+__global__ __launch_bounds__(256) void k_reeval64_band(const double* __restrict__ s64, uint32_t nslots,
                                                        const float* __restrict__ tri, const float* __restrict__ Q,
                                                        int64_t nq, double acc2, double band, double* __restrict__ W) {
   __shared__ uint2 ring_all[4][kReevalRing];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   for (int64_t qi = (int64_t)blockIdx.x * 4 + wv; qi < nq; qi += (int64_t)gridDim.x * 4) {
     if (fabs(W[qi] - 0.5) >= band) continue;  // wave-uniform; NaN (near-list overflow) is walked again
-    const double w = ring_walk64<ORDER>(ring_all[wv], lane, slots, s64, nslots, tri, Q[3 * qi], Q[3 * qi + 1],
+    const double w = ring_walk64<ORDER>(ring_all[wv], lane, s64, nslots, tri, Q[3 * qi], Q[3 * qi + 1],
                                         Q[3 * qi + 2], acc2);
     if (lane == 0) W[qi] = w;
   }
@@ -1349,9 +1417,9 @@ static void launch_traverse64(const gwn_soup* s, unsigned g, hipStream_t st, con
                               const uint32_t* order, int64_t nq, double a2, double* W) {
   const uint32_t ns = (uint32_t)s->nslots;
   switch (s->order) {
-    case 0: hipLaunchKernelGGL(k_traverse64<0>, dim3(g), dim3(256), 0, st, s->slots.p, s->slots64.p, ns, s->tri.p, Q, perm, order, nq, nullptr, a2, W); break;
-    case 1: hipLaunchKernelGGL(k_traverse64<1>, dim3(g), dim3(256), 0, st, s->slots.p, s->slots64.p, ns, s->tri.p, Q, perm, order, nq, nullptr, a2, W); break;
-    default: hipLaunchKernelGGL(k_traverse64<2>, dim3(g), dim3(256), 0, st, s->slots.p, s->slots64.p, ns, s->tri.p, Q, perm, order, nq, nullptr, a2, W); break;
+    case 0: hipLaunchKernelGGL(k_traverse64<0>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, perm, order, nq, a2, W); break;
+    case 1: hipLaunchKernelGGL(k_traverse64<1>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, perm, order, nq, a2, W); break;
+    default: hipLaunchKernelGGL(k_traverse64<2>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, perm, order, nq, a2, W); break;
   }
   check_launch("k_traverse64");
 }
@@ -1368,9 +1436,9 @@ static void launch_walk_ring(const gwn_soup* s, const float* Q, int64_t nq, floa
   ProfileScope prof("soup_walk_ring", st, prof_on);
   if (precision == GWN_PREC_FP64) {
     switch (s->order) {
-      case 0: hipLaunchKernelGGL(k_reeval64<0>, dim3(g), dim3(256), 0, st, s->slots.p, s->slots64.p, ns, s->tri.p, Q, nullptr, nq, nullptr, a2, W); break;
-      case 1: hipLaunchKernelGGL(k_reeval64<1>, dim3(g), dim3(256), 0, st, s->slots.p, s->slots64.p, ns, s->tri.p, Q, nullptr, nq, nullptr, a2, W); break;
-      default: hipLaunchKernelGGL(k_reeval64<2>, dim3(g), dim3(256), 0, st, s->slots.p, s->slots64.p, ns, s->tri.p, Q, nullptr, nq, nullptr, a2, W); break;
+      case 0: hipLaunchKernelGGL(k_reeval64<0>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, nullptr, nq, nullptr, a2, W); break;
+      case 1: hipLaunchKernelGGL(k_reeval64<1>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, nullptr, nq, nullptr, a2, W); break;
+      default: hipLaunchKernelGGL(k_reeval64<2>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, nullptr, nq, nullptr, a2, W); break;
     }
     check_launch("k_reeval64");
     return;
@@ -1387,9 +1455,9 @@ static void launch_walk_ring(const gwn_soup* s, const float* Q, int64_t nq, floa
   check_launch("k_walk_ring");
   if (mixed) {
     switch (s->order) {
-      case 0: hipLaunchKernelGGL(k_reeval64_band<0>, dim3(g), dim3(256), 0, st, s->slots.p, s->slots64.p, ns, s->tri.p, Q, nq, a2, band, W); break;
-      case 1: hipLaunchKernelGGL(k_reeval64_band<1>, dim3(g), dim3(256), 0, st, s->slots.p, s->slots64.p, ns, s->tri.p, Q, nq, a2, band, W); break;
-      default: hipLaunchKernelGGL(k_reeval64_band<2>, dim3(g), dim3(256), 0, st, s->slots.p, s->slots64.p, ns, s->tri.p, Q, nq, a2, band, W); break;
+      case 0: hipLaunchKernelGGL(k_reeval64_band<0>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, nq, a2, band, W); break;
+      case 1: hipLaunchKernelGGL(k_reeval64_band<1>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, nq, a2, band, W); break;
+      default: hipLaunchKernelGGL(k_reeval64_band<2>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, nq, a2, band, W); break;
     }
     check_launch("k_reeval64_band");
   }
@@ -1504,9 +1572,9 @@ void soup_query_device_ws(const gwn_soup* s, const float* Q, int64_t nq, float a
       const unsigned gr = dcount ? (unsigned)std::min<int64_t>(div_up(na64, 4), 2048) : (unsigned)div_up(na64, 4);
       ProfileScope prof("soup_reeval64", st, prof_on);
       switch (s->order) {
-        case 0: hipLaunchKernelGGL(k_reeval64<0>, dim3(gr), dim3(256), 0, st, s->slots.p, s->slots64.p, ns, s->tri.p, Q, amb, na64, dcount, a2, W); break;
-        case 1: hipLaunchKernelGGL(k_reeval64<1>, dim3(gr), dim3(256), 0, st, s->slots.p, s->slots64.p, ns, s->tri.p, Q, amb, na64, dcount, a2, W); break;
-        default: hipLaunchKernelGGL(k_reeval64<2>, dim3(gr), dim3(256), 0, st, s->slots.p, s->slots64.p, ns, s->tri.p, Q, amb, na64, dcount, a2, W); break;
+        case 0: hipLaunchKernelGGL(k_reeval64<0>, dim3(gr), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, amb, na64, dcount, a2, W); break;
+        case 1: hipLaunchKernelGGL(k_reeval64<1>, dim3(gr), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, amb, na64, dcount, a2, W); break;
+        default: hipLaunchKernelGGL(k_reeval64<2>, dim3(gr), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, amb, na64, dcount, a2, W); break;
       }
       check_launch("k_reeval64");
     }

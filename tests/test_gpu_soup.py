@@ -127,6 +127,37 @@ def test_ring_walk_and_sequential_walks_agree(order):
             assert np.array_equal(bvh.query(Q[:20000], beta, prec), Wsmall[:20000])
 
 
+@pytest.mark.parametrize("order", [0, 1, 2])
+@pytest.mark.parametrize("nq", [300, 65_541])
+def test_far_fields_that_overflow_are_descended(order, nq):
+    """A far field that is not finite is not taken: the walk descends, as the
+    reference's does.  A mesh scaled by 1e10 has order-2 moments (length^4)
+    beyond FP32 in its upper nodes; the walks that add first and ask at the
+    end start such a query again, so W equals the unscaled mesh's within the
+    truncation of one more level and the closed mesh classifies exactly.
+    Queries that are not finite give NaN and disturb no neighbour."""
+    V, F = D.bumpy_sphere(3, 8, 31)
+    rng = np.random.default_rng(31)
+    Q = rng.uniform(-1.4, 1.4, (nq, 3))
+    s = 1e10
+    big = gwn.FastWindingNumberBVH().build(V * s, F, order)
+    if order == 2:  # the upper nodes' moments do overflow
+        assert not np.isfinite(big.boxdata()[0, 64:]).all()
+    exact = gwn.winding_number_bruteforce(V, F, Q)
+    plain = gwn.FastWindingNumberBVH().build(V, F, order)
+    for prec in (gwn.PREC_FP32, gwn.PREC_MIXED, gwn.PREC_FP64):
+        W, W0 = big.query(Q * s, 4.0, prec), plain.query(Q, 4.0, prec)
+        bound = np.abs(W0 - exact).max() * 2 + 1e-5  # no worse than the truncation of the unscaled walk, twice
+        assert np.abs(W - exact).max() <= bound, (prec, np.abs(W - exact).max(), bound)
+        assert np.array_equal(W > 0.5, exact > 0.5)
+        Qn = Q.copy()
+        Qn[5], Qn[70, 1], Qn[71, 2] = np.nan, np.inf, -np.inf
+        Wn = plain.query(Qn, 4.0, prec)
+        assert np.isnan(Wn[[5, 70, 71]]).all()
+        keep = np.setdiff1d(np.arange(nq), [5, 70, 71])
+        assert np.array_equal(Wn[keep], W0[keep])
+
+
 def test_wave_walk_block_order_covers_every_query():
     """Batches of 65,536+ queries run their blocks of 256 costliest first (a
     per-XCD counting sort of costs read from a grid built with the tree).
