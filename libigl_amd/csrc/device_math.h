@@ -104,6 +104,14 @@ __device__ __forceinline__ void pack_far_field(const double* b, const double* q,
   r[19] = (T)g[9];           // f.w  xyz
 }
 
+// 1/sqrt(x) to FP64 rounding: the hardware estimate (about 2^-26 relative) and
+// one third-order step
+__device__ __forceinline__ double rsqrt64(double x) {
+  const double r = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * r), r, 1.0);
+  return fma(r * e, fma(0.375, e, 0.5), r);
+}
+
 // A running sum of angles atan2(y, x), kept as the product of the x + i y
 // scaled by powers of two and the number of full turns: the sum is
 // 2 pi turns + atan2(im, re).  A term costs a complex multiplication, a

@@ -363,8 +363,9 @@ __global__ void k_write_dbox(int64_t nn, const uint32_t* __restrict__ nodes, con
 
 // ---------------------------------------------------------------------------
 // exact triangle solid angle: UTsignedSolidAngleTri (6070-6110)
+// (not inlined: the sums below call it for few terms)
 template <typename T>
-__device__ __forceinline__ T tri_solid_angle(T ax, T ay, T az, T bx, T by, T bz, T cx, T cy, T cz, T qx, T qy,
+__device__ __attribute__((noinline)) T tri_solid_angle(T ax, T ay, T az, T bx, T by, T bz, T cx, T cy, T cz, T qx, T qy,
                                              T qz) {
   T a0 = ax - qx, a1 = ay - qy, a2 = az - qz;
   T b0 = bx - qx, b1 = by - qy, b2 = bz - qz;
@@ -419,13 +420,6 @@ struct D4 {
   double x, y, z, w;
 };
 
-// 1/sqrt(x) to FP64 rounding: the hardware estimate (about 2^-26 relative) and
-// one third-order step
-__device__ __forceinline__ double rsqrt64(double x) {
-  const double r = __builtin_amdgcn_rsq(x);
-  const double e = fma(-(x * r), r, 1.0);
-  return fma(r * e, fma(0.375, e, 0.5), r);
-}
 __device__ __forceinline__ float tri_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
 __device__ __forceinline__ double tri_rsqrt(double x) { return rsqrt64(x); }
 
@@ -456,14 +450,25 @@ struct SolidAngleSum {
     c0 *= rc; c1 *= rc; c2 *= rc;
     const T u0 = b0 - a0, u1 = b1 - a1, u2 = b2 - a2;
     const T w0 = c0 - a0, w1 = c1 - a1, w2 = c2 - a2;
-    const T k0 = fma(u1, w2, -(u2 * w1)), k1 = fma(u2, w0, -(u0 * w2)), k2 = fma(u0, w1, -(u1 * w0));
-    const T num = fma(a2, k2, fma(a1, k1, a0 * k0));
+    T num;
+    if constexpr (sizeof(T) == 4) {
+      const T k0 = fma(u1, w2, -(u2 * w1)), k1 = fma(u2, w0, -(u0 * w2)), k2 = fma(u0, w1, -(u1 * w0));
+      num = fma(a2, k2, fma(a1, k1, a0 * k0));
+    } else {
+      // rounded product by product, as tri_solid_angle: where products cancel
+      // (a query in the triangle's plane) the numerator is zero
+      num = a0 * (u1 * w2 - u2 * w1) + a1 * (u2 * w0 - u0 * w2) + a2 * (u0 * w1 - u1 * w0);
+    }
     if (num == T(0)) return;
     const T ab = fma(a2, b2, fma(a1, b1, a0 * b0));
     const T ac = fma(a2, c2, fma(a1, c1, a0 * c0));
     const T bc = fma(b2, c2, fma(b1, c1, b0 * c0));
     const T den = ((T(1) + ab) + ac) + bc;
-    if (!half.add(num, den)) extra += T(2) * atan2(num, den);
+    // FP64: where the angle hangs on the last bits (the query on an edge),
+    // the term is tri_solid_angle's
+    const bool fine = sizeof(T) == 4 || fmax(fabs(num), fabs(den)) > T(1e-9);
+    if (!fine || !half.add(num, den))
+      extra += tri_solid_angle<T>(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], qx, qy, qz);
   }
   __device__ __forceinline__ double total() const { return (double)extra + 2.0 * half.total(); }
 };

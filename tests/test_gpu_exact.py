@@ -166,3 +166,40 @@ def test_exact_2d_few_queries_many_edges():
         W = gwn.winding_number(V, E, Q)
         assert np.abs(W - Op.winding_number_2d(V, E, Q)).max() < 1e-12, nq
 
+
+
+def _cube(scale=1.0):
+    """An axis-aligned cube, two triangles a side, outward."""
+    V = np.array([[x, y, z] for x in (-1, 1) for y in (-1, 1) for z in (-1, 1)], np.float64) * 0.5 * scale
+    quads = [(0, 1, 3, 2), (4, 6, 7, 5), (0, 4, 5, 1), (2, 3, 7, 6), (0, 2, 6, 4), (1, 5, 7, 3)]
+    F = np.array([t for a, b, c, d in quads for t in ((a, b, c), (a, c, d))], np.int32)
+    return V, F
+
+
+@pytest.mark.parametrize("nq", [125, 65_541])
+def test_fp64_soup_exact_terms_on_edges_and_faces(nq):
+    """The FP64 walk with every triangle exact (accuracy_scale 1e3), queries on
+    a cube's corners, edges, diagonals and faces: UTsignedSolidAngleTri in FP64
+    (6070-6110) term by term, zero where the numerator or a length is zero."""
+    V, F = _cube()
+    g = np.linspace(-1.0, 1.0, 5)
+    Q = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+    ref = np.zeros(125)
+    for t in F:
+        d = V[t][None] - Q[:, None]  # 125 x 3 x 3
+        l = np.sqrt(d[..., 0] * d[..., 0] + d[..., 1] * d[..., 1] + d[..., 2] * d[..., 2])
+        ok = (l != 0).all(1)
+        d = d / np.where(l == 0, 1.0, l)[..., None]
+        a, b, c = d[:, 0], d[:, 1], d[:, 2]
+        u, w = b - a, c - a
+        num = (a[:, 0] * (u[:, 1] * w[:, 2] - u[:, 2] * w[:, 1]) + a[:, 1] * (u[:, 2] * w[:, 0] - u[:, 0] * w[:, 2])
+               + a[:, 2] * (u[:, 0] * w[:, 1] - u[:, 1] * w[:, 0]))
+
+        def dot(p, q):
+            return p[:, 0] * q[:, 0] + p[:, 1] * q[:, 1] + p[:, 2] * q[:, 2]
+        den = 1.0 + dot(a, b) + dot(a, c) + dot(b, c)
+        ref += np.where(ok & (num != 0), 2.0 * np.arctan2(num, den), 0.0)
+    Qn = np.tile(Q, (-(-nq // 125), 1))[:nq]
+    bvh = gwn.FastWindingNumberBVH().build(V, F, 2)
+    W = bvh.query(Qn, 1e3, gwn.PREC_FP64)
+    np.testing.assert_allclose(W, np.tile(ref / (4 * np.pi), -(-nq // 125))[:nq], rtol=0, atol=1e-12)
