@@ -9,11 +9,12 @@
 // in tiles of 256 (9 doubles each, 18 KB), so every triangle is read from
 // HBM once per block and broadcast from LDS to all lanes.  A small query set
 // also splits the triangles into chunks (grid.y) so that the GPU is full;
-// the chunk partials are then added in chunk order.  FP64 VALU bound.  atan2
-// terms are summed and divided by 2 pi once per query (the reference divides
-// each term; the difference is a few ulps of the FP64 result).
+// the chunk partials are then added in chunk order.  FP64 VALU bound.  The
+// angles are summed as one complex product (AngleSum) and divided by 2 pi once
+// per query; the reference takes an atan2 per triangle and divides each.
 #include <hip/hip_runtime.h>
 
+#include "device_math.h"
 #include "gwn_internal.h"
 #include "ring_walk.h"
 #include "wntree.h"
@@ -25,7 +26,9 @@ constexpr int EX_TILE = 256;
 constexpr int EX_QPT = 1;
 constexpr double EX_PI = 3.1415926535897932384626433832795;
 
-__device__ __forceinline__ double vos_atan2(const double* t, double px, double py, double pz) {
+// (not inlined: the sums below call it for few terms, and inlined it takes
+// 114 VGPRs where 75 do)
+__device__ __attribute__((noinline)) double vos_atan2(const double* t, double px, double py, double pz) {
   const double a0 = t[0] - px, a1 = t[1] - py, a2 = t[2] - pz;
   const double b0 = t[3] - px, b1 = t[4] - py, b2 = t[5] - pz;
   const double c0 = t[6] - px, c1 = t[7] - py, c2 = t[8] - pz;
@@ -39,6 +42,36 @@ __device__ __forceinline__ double vos_atan2(const double* t, double px, double p
   const double dab = a0 * b0 + a1 * b1 + a2 * b2;
   return atan2(det, la * lb * lc + dbc * la + dca * lb + dab * lc);
 }
+
+// Sum of vos_atan2 over triangles.  The determinant is the same, term for term
+// (a query in a triangle's plane gets the same zero, or the same sign); the
+// lengths come from the refined reciprocal square root and the rest uses
+// multiply-adds.  Where the angle hangs on the last bits (the query on an edge
+// or at a corner), and for a term the product does not take, vos_atan2 gives
+// it.  About 100 FP64 operations a triangle against 210 with a square root per
+// length and an atan2: 100,000 queries on 20,480 triangles 10.8 -> 6.4 ms.
+struct VosSum {
+  AngleSum<double> angles;
+  double extra = 0.0;
+
+  __device__ __forceinline__ void add(const double* t, double px, double py, double pz) {
+    const double a0 = t[0] - px, a1 = t[1] - py, a2 = t[2] - pz;
+    const double b0 = t[3] - px, b1 = t[4] - py, b2 = t[5] - pz;
+    const double c0 = t[6] - px, c1 = t[7] - py, c2 = t[8] - pz;
+    const double a = fma(a2, a2, fma(a1, a1, a0 * a0));
+    const double b = fma(b2, b2, fma(b1, b1, b0 * b0));
+    const double c = fma(c2, c2, fma(c1, c1, c0 * c0));
+    const double la = a * rsqrt64(a), lb = b * rsqrt64(b), lc = c * rsqrt64(c);
+    const double det = a0 * b1 * c2 + b0 * c1 * a2 + c0 * a1 * b2 - c0 * b1 * a2 - b0 * a1 * c2 - a0 * c1 * b2;
+    const double dbc = fma(b2, c2, fma(b1, c1, b0 * c0));
+    const double dca = fma(c2, a2, fma(c1, a1, c0 * a0));
+    const double dab = fma(a2, b2, fma(a1, b1, a0 * b0));
+    const double lll = la * lb * lc;
+    const double den = fma(dab, lc, fma(dca, lb, fma(dbc, la, lll)));
+    if (!(fmax(fabs(det), fabs(den)) > 1e-9 * lll) || !angles.add(det, den)) extra += vos_atan2(t, px, py, pz);
+  }
+  __device__ __forceinline__ double total() const { return extra + angles.total(); }
+};
 
 __global__ __launch_bounds__(EX_THREADS) void k_exact_gather(const double* __restrict__ V,
                                                                const int32_t* __restrict__ F, int64_t nf,
@@ -59,14 +92,14 @@ __global__ __launch_bounds__(EX_THREADS) void k_exact(const double* __restrict__
                                                        double* __restrict__ part, double* __restrict__ W) {
   __shared__ double tile[EX_TILE * 9];
   const int64_t q0 = ((int64_t)blockIdx.x * EX_THREADS) * EX_QPT + threadIdx.x;
-  double px[EX_QPT], py[EX_QPT], pz[EX_QPT], acc[EX_QPT];
+  double px[EX_QPT], py[EX_QPT], pz[EX_QPT];
+  VosSum acc[EX_QPT];
   for (int k = 0; k < EX_QPT; ++k) {
     const int64_t q = q0 + (int64_t)k * EX_THREADS;
     const bool ok = q < no;
     px[k] = ok ? O[3 * q] : 0.0;
     py[k] = ok ? O[3 * q + 1] : 0.0;
     pz[k] = ok ? O[3 * q + 2] : 0.0;
-    acc[k] = 0.0;
   }
   const int64_t fb = (int64_t)blockIdx.y * chunk;
   const int64_t fe = (fb + chunk) < nf ? (fb + chunk) : nf;
@@ -78,29 +111,27 @@ __global__ __launch_bounds__(EX_THREADS) void k_exact(const double* __restrict__
     for (int j = 0; j < cnt; ++j) {
       const double* t = tile + 9 * j;
 #pragma unroll
-      for (int k = 0; k < EX_QPT; ++k) acc[k] += vos_atan2(t, px[k], py[k], pz[k]);
+      for (int k = 0; k < EX_QPT; ++k) acc[k].add(t, px[k], py[k], pz[k]);
     }
   }
   for (int k = 0; k < EX_QPT; ++k) {
     const int64_t q = q0 + (int64_t)k * EX_THREADS;
     if (q < no) {
       if (part)
-        part[(int64_t)blockIdx.y * no + q] = acc[k];
+        part[(int64_t)blockIdx.y * no + q] = acc[k].total();
       else
-        W[q] = acc[k] / (2.0 * EX_PI);
+        W[q] = acc[k].total() / (2.0 * EX_PI);
     }
   }
 }
 
-// W[q] = the chunk partials of query q added in chunk order, divided by 2 pi
-// when the terms do not already carry it (3D)
-__global__ void k_exact_sum(const double* __restrict__ part, int64_t nchunks, int64_t no, bool div2pi,
-                            double* __restrict__ W) {
+// W[q] = the chunk partials of query q added in chunk order, over 2 pi
+__global__ void k_exact_sum(const double* __restrict__ part, int64_t nchunks, int64_t no, double* __restrict__ W) {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= no) return;
   double s = 0.0;
   for (int64_t c = 0; c < nchunks; ++c) s += part[c * no + q];
-  W[q] = div2pi ? s / (2.0 * EX_PI) : s;
+  W[q] = s / (2.0 * EX_PI);
 }
 
 // Triangle (or edge) chunks per launch: enough blocks for ~16 wavefronts per SIMD
@@ -114,11 +145,11 @@ static int64_t exact_chunks(int64_t nf, int64_t qblocks) {
 // ---- 2D: winding number of a curve of edges (winding_number.cpp:62-89 with
 // F.cols() == 2): W(o) = sum over edges (a,b) of signed_angle(a, b, o)
 // (signed_angle.cpp:8-41): -atan2(cross, dot) of the unit vectors from a and b
-// to o, each term divided by 2 pi.  Terms are summed in edge order within
-// each chunk of the edge list; when a small query set splits the edges into
-// chunks (exact_chunks), the chunk partials are then added in chunk order, so
-// the last bits can differ from the reference's single sum in edge order.
-__device__ __forceinline__ double signed_angle_2d(const double* e, double px, double py) {
+// to o, over 2 pi.  The angles are summed as one product (AngleSum) in edge
+// order within each chunk of the edge list; when a small query set splits the
+// edges into chunks (exact_chunks), the chunk partials are then added in chunk
+// order.  The last bits so differ from the reference's sum of its terms.
+__device__ __attribute__((noinline)) double signed_angle_2d(const double* e, double px, double py) {
   double ax = px - e[0], ay = py - e[1], bx = px - e[2], by = py - e[3];
   const double la = sqrt(ax * ax + ay * ay), lb = sqrt(bx * bx + by * by);
   if (la != 0.0) {
@@ -129,8 +160,25 @@ __device__ __forceinline__ double signed_angle_2d(const double* e, double px, do
     bx /= lb;
     by /= lb;
   }
-  return -atan2(bx * ay - by * ax, bx * ax + by * ay) / (2.0 * EX_PI);
+  return -atan2(bx * ay - by * ax, bx * ax + by * ay);
 }
+
+// Sum of signed_angle_2d over edges: the lengths do not change an angle, so
+// the product takes the unscaled cross and dot products.  A query (nearly) on
+// an edge, where the sign of the half turn hangs on the last bits, and a term
+// the product does not take are left to signed_angle_2d.  20,000 queries on
+// 26,214 edges, host arrays: 7.7 -> 0.9 ms.
+struct Edge2dSum {
+  AngleSum<double> angles;
+  double extra = 0.0;
+
+  __device__ __forceinline__ void add(const double* e, double px, double py) {
+    const double ax = px - e[0], ay = py - e[1], bx = px - e[2], by = py - e[3];
+    const double cross = bx * ay - by * ax, dot = bx * ax + by * ay;
+    if (!(fabs(cross) >= -1e-9 * dot) || !angles.add(cross, dot)) extra += signed_angle_2d(e, px, py);
+  }
+  __device__ __forceinline__ double total() const { return extra - angles.total(); }
+};
 
 __global__ __launch_bounds__(EX_THREADS) void k_exact2d_gather(const double* __restrict__ V,
                                                                  const int32_t* __restrict__ E, int64_t ne,
@@ -142,8 +190,7 @@ __global__ __launch_bounds__(EX_THREADS) void k_exact2d_gather(const double* __r
 }
 
 // Block (bx, by): queries of block bx against the edges of chunk by, as in
-// k_exact; the terms already carry the 1 / 2 pi, so the partials are summed
-// as they are.
+// k_exact.
 __global__ __launch_bounds__(EX_THREADS) void k_exact2d(const double* __restrict__ T, int64_t ne, int64_t chunk,
                                                          const double* __restrict__ O, int64_t no,
                                                          double* __restrict__ part, double* __restrict__ W) {
@@ -151,7 +198,7 @@ __global__ __launch_bounds__(EX_THREADS) void k_exact2d(const double* __restrict
   const int64_t q = (int64_t)blockIdx.x * EX_THREADS + threadIdx.x;
   const bool ok = q < no;
   const double px = ok ? O[2 * q] : 0.0, py = ok ? O[2 * q + 1] : 0.0;
-  double acc = 0.0;
+  Edge2dSum acc;
   const int64_t fb = (int64_t)blockIdx.y * chunk;
   const int64_t fe = (fb + chunk) < ne ? (fb + chunk) : ne;
   for (int64_t f0 = fb; f0 < fe; f0 += EX_TILE) {
@@ -159,13 +206,13 @@ __global__ __launch_bounds__(EX_THREADS) void k_exact2d(const double* __restrict
     __syncthreads();
     for (int e = threadIdx.x; e < cnt * 4; e += EX_THREADS) tile[e] = T[4 * f0 + e];
     __syncthreads();
-    for (int j = 0; j < cnt; ++j) acc += signed_angle_2d(tile + 4 * j, px, py);
+    for (int j = 0; j < cnt; ++j) acc.add(tile + 4 * j, px, py);
   }
   if (ok) {
     if (part)
-      part[(int64_t)blockIdx.y * no + q] = acc;
+      part[(int64_t)blockIdx.y * no + q] = acc.total();
     else
-      W[q] = acc;
+      W[q] = acc.total() / (2.0 * EX_PI);
   }
 }
 
@@ -192,7 +239,7 @@ void exact2d_device(const double* V, const int32_t* E, int64_t ne, const double*
                      O, no, part, W);
   check_launch("k_exact2d");
   if (part) {
-    hipLaunchKernelGGL(k_exact_sum, dim3(div_up(no, 256)), dim3(256), 0, st, part, nch, no, false, W);
+    hipLaunchKernelGGL(k_exact_sum, dim3(div_up(no, 256)), dim3(256), 0, st, part, nch, no, W);
     check_launch("k_exact_sum");
   }
 }
@@ -221,54 +268,58 @@ void exact_device(const double* V, int64_t nv, const int32_t* F, int64_t nf, con
                      O, no, part, W);
   check_launch("k_exact");
   if (part) {
-    hipLaunchKernelGGL(k_exact_sum, dim3(div_up(no, 256)), dim3(256), 0, st, part, nch, no, true, W);
+    hipLaunchKernelGGL(k_exact_sum, dim3(div_up(no, 256)), dim3(256), 0, st, part, nch, no, W);
     check_launch("k_exact_sum");
   }
 }
 
 
 // ---------------------------------------------------------------------------
-// The reference's hierarchy (wntree.cpp), one wavefront per query (queries in
-// Hilbert order when perm is given).  The wavefront walks the query's
-// pre-order records: inside an internal node's closed box it steps to the
-// first child; otherwise it sums the node's triangle list (inside a leaf: its
+// The reference's hierarchy (wntree.cpp), G lanes per query (queries in
+// Hilbert order when perm is given).  The lanes walk the query's pre-order
+// records together: inside an internal node's closed box they step to the
+// first child; otherwise they sum the node's triangle list (inside a leaf: its
 // faces; outside the box: its cap, or its faces when the cap is not smaller)
-// and jumps past the subtree.  The 64 lanes share each list, lane l taking
-// its triangles l, l+64, ...; each term is solid_angle(...) (solid_angle.cpp:
-// atan2 over 2 pi), and the lanes' FP64 partial sums are added in a fixed
-// order (wave_sum).  The reference adds a node's children's sums; the orders
-// agree to rounding.  A query's result does not depend on the batch it is in.
-// One query per lane, wave-coherent or not, ran 6x (100k queries) to 100x
-// (1,000 queries) longer: the lists run to dozens of triangles, which a lane
-// summed alone while the wavefront's other lanes waited.
+// and jump past the subtree.  They share each list, lane l taking its
+// triangles l, l+G, ...; each lane sums its angles as one product, and the
+// lanes' FP64 totals are added in a fixed order.  The reference adds a node's
+// children's sums; the orders agree to rounding.  A query's result depends on
+// the query and G only.
+// 20,480 triangles, 100,000 queries: 0.45 ms a call with an atan2 per triangle
+// and 64 lanes a query, 0.28 ms.
+template <int G>
 __global__ __launch_bounds__(256) void k_wn_tree_lanes(const WNRecord* __restrict__ rec, uint32_t nrec,
                                                         const double* __restrict__ tri,
                                                         const double* __restrict__ O,
                                                         const uint32_t* __restrict__ perm, int64_t no,
                                                         double* __restrict__ W) {
-  const int lane = threadIdx.x & 63;
-  const int64_t w = (int64_t)xcd_block() * 4 + (threadIdx.x >> 6);
+  const uint32_t lane = threadIdx.x % G;
+  const int64_t w = ((int64_t)xcd_block() * 256 + threadIdx.x) / G;
   if (w >= no) return;
   const int64_t q = perm ? (int64_t)perm[w] : w;
   const double px = O[3 * q], py = O[3 * q + 1], pz = O[3 * q + 2];
-  double part = 0.0;
-  uint32_t i = 0;
-  while (i < nrec) {
-    const WNRecord& r = rec[i];
-    const bool inside = !(px < r.lo[0] || px > r.hi[0] || py < r.lo[1] || py > r.hi[1] || pz < r.lo[2] ||
-                          pz > r.hi[2]);
-    if (inside && !r.leaf) {
-      ++i;
-      continue;
+  VosSum sum;
+  uint32_t i = 0, at = 0, end = 0;  // the next record; the rest of the list being summed (the same on the G lanes)
+  for (;;) {
+    while (at >= end && i < nrec) {  // to the next record with triangles for this query
+      const WNRecord& r = rec[i];
+      const bool inside = !(px < r.lo[0] || px > r.hi[0] || py < r.lo[1] || py > r.hi[1] || pz < r.lo[2] ||
+                            pz > r.hi[2]);
+      if (inside && !r.leaf) {
+        ++i;
+      } else {
+        at = inside ? r.in_start : r.out_start;
+        end = at + (inside ? r.in_count : r.out_count);
+        i = r.link;
+      }
     }
-    const uint32_t start = inside ? r.in_start : r.out_start;
-    const uint32_t count = inside ? r.in_count : r.out_count;
-    for (uint32_t k = (uint32_t)lane; k < count; k += 64)
-      part += vos_atan2(tri + 9 * (size_t)(start + k), px, py, pz) / (2.0 * EX_PI);
-    i = r.link;
+    if (at >= end) break;
+    if (lane < end - at) sum.add(tri + 9 * (size_t)(at + lane), px, py, pz);
+    at += G;
   }
-  const double sum = wave_sum(part);
-  if (lane == 0) W[q] = sum;
+  double v = sum.total();
+  for (int off = G / 2; off >= 1; off >>= 1) v = __dadd_rn(v, __shfl_xor(v, off, 64));
+  if (lane == 0) W[q] = v / (2.0 * EX_PI);
 }
 
 __global__ void k_wn_narrow(const double* __restrict__ O, int64_t n3, float* __restrict__ Of) {
@@ -286,6 +337,13 @@ void wntree_upload(const WNTreeHost& T, DevBuf<uint8_t>& rec, DevBuf<double>& tr
   GWN_HIP(hipStreamSynchronize(st));
 }
 
+// Batches below this take 64 lanes a query, larger ones 32.  Half the lanes
+// leave fewer of them idle at the ends of the lists, but a query then takes
+// twice as long: 20,480 triangles, 64 / 32 lanes: 35 / 50 us for 1,000
+// queries, 106 / 120 us for 10,000, 297 / 281 us for 100,000, 2.13 / 1.72 ms
+// for 1M.
+constexpr int64_t kWideLanesBelow = 65536;
+
 // O no x 3 and W no, device pointers; bbox: the root's box (query order)
 void wntree_query_device(const uint8_t* rec, int64_t nrec, const double* tri, const float* bbox, const double* O,
                          int64_t no, double* W, hipStream_t st) {
@@ -296,8 +354,11 @@ void wntree_query_device(const uint8_t* rec, int64_t nrec, const double* tri, co
   }
   uint32_t* perm = nullptr;
   // small batches walk in input order; larger ones along the Hilbert curve
-  // (neighbouring wavefronts then read the same records and triangles)
-  const bool sorted = no >= 4096;
+  // (neighbouring wavefronts then read the same records and triangles).  On
+  // 20,480 triangles the sort cost more than it saved up to 60,000 queries (209
+  // against 160 us) and as much at 100,000 (281 us); on 100,000 triangles it
+  // saved 65 us of 457 at 100,000 queries.
+  const bool sorted = no >= 65536;
   const size_t tb = sorted ? radix_sort_temp_bytes(no, false) : 0;
   Scratch ws(sorted ? scratch_bytes({12 * (size_t)no, 4 * (size_t)no, 4 * (size_t)no, tb}) : 1, st);
   if (sorted) {
@@ -311,8 +372,13 @@ void wntree_query_device(const uint8_t* rec, int64_t nrec, const double* tri, co
     radix_sort_u32(keys, perm, no, 30, tmp, tb, st);
   }
   ProfileScope prof("exact_tree", st);
-  hipLaunchKernelGGL(k_wn_tree_lanes, dim3(div_up(no, 4)), dim3(256), 0, st, reinterpret_cast<const WNRecord*>(rec),
-                     (uint32_t)nrec, tri, O, perm, no, W);
+  const WNRecord* r = reinterpret_cast<const WNRecord*>(rec);
+  if (no < kWideLanesBelow)
+    hipLaunchKernelGGL(k_wn_tree_lanes<64>, dim3(div_up(no, 4)), dim3(256), 0, st, r, (uint32_t)nrec, tri, O, perm, no,
+                       W);
+  else
+    hipLaunchKernelGGL(k_wn_tree_lanes<32>, dim3(div_up(no, 8)), dim3(256), 0, st, r, (uint32_t)nrec, tri, O, perm, no,
+                       W);
   check_launch("k_wn_tree_lanes");
 }
 

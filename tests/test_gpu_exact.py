@@ -177,6 +177,38 @@ def _cube(scale=1.0):
 
 
 @pytest.mark.parametrize("nq", [125, 65_541])
+def test_queries_on_vertices_edges_and_faces(nq):
+    """Queries at a cube's corners, on its edges, face diagonals and faces: the
+    terms there hang on the sign of a zero and on last bits (a half turn each
+    way), and the angle product leaves them to the per-triangle form, so the
+    sums equal the oracle's term by term sum."""
+    V, F = _cube()
+    g = np.linspace(-1.0, 1.0, 5)  # -1 -0.5 0 0.5 1: corners, edge and face midpoints, diagonals
+    Q = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+    Q = np.tile(Q, (-(-nq // Q.shape[0]), 1))[:nq]
+    Wo = O.winding_number_bf(V, F, Q[:125])
+    assert len(np.unique(np.round(Wo * 8))) > 3  # corners, edges and faces do differ
+    W = gwn.winding_number_bruteforce(V, F, Q)
+    np.testing.assert_allclose(W, np.tile(Wo, -(-nq // 125))[:nq], rtol=0, atol=1e-12)
+    P = np.array([[-0.5, -0.5], [0.5, -0.5], [0.5, 0.5], [-0.5, 0.5]])
+    E = np.array([[0, 1], [1, 2], [2, 3], [3, 0]], np.int32)
+    W2 = gwn.winding_number(P, E, Q[:, :2])
+    np.testing.assert_allclose(W2[:125], O.winding_number_2d(P, E, Q[:125, :2]), rtol=0, atol=1e-12)
+
+
+@pytest.mark.parametrize("nq", [1, 63, 65, 4097, 65_535, 65_536])
+def test_hierarchy_lanes_and_order_by_batch_size(nq):
+    """64 lanes a query in input order below 65,536 queries, 32 lanes and the
+    Hilbert order from there: both sum the reference's lists (leaves of up to
+    100 faces, caps of any length), which agree with the sum over every face
+    to rounding."""
+    V, F = D.noisy_sphere(4, 0.01, 5)
+    Q = np.random.default_rng(nq).uniform(-1.3, 1.3, (nq, 3))
+    W = gwn.WindingNumberAABB(V, F).winding_number(Q)
+    np.testing.assert_allclose(W, gwn.winding_number_bruteforce(V, F, Q), rtol=0, atol=1e-11)
+
+
+@pytest.mark.parametrize("nq", [125, 65_541])
 def test_fp64_soup_exact_terms_on_edges_and_faces(nq):
     """The FP64 walk with every triangle exact (accuracy_scale 1e3), queries on
     a cube's corners, edges, diagonals and faces: UTsignedSolidAngleTri in FP64
