@@ -288,6 +288,7 @@ struct gwn_soup {
   gwn::DevBuf<float> boxdata;   // nnodes x 92, reference BoxData order
   gwn::DevBuf<float4> slots;    // nslots x 6 (rope layout, FP32 moments)
   int64_t nslots = 0;
+  gwn::DevBuf<uint4> kids;      // nslots + 1: rope positions of each record's children, and of the root's
   gwn::DevBuf<double> slots64;  // nslots x 24 (FP64 moments), built with the tree
   gwn::DevBuf<double> V64;      // nv x 3, the vertices as given (closest-point queries)
   gwn::DevBuf<float4> dbox;     // nslots x 2 slot boxes for closest-point queries, built on first use

@@ -204,13 +204,28 @@ __device__ __forceinline__ void slot_far_field(const T* __restrict__ bd, int s, 
                         1.5 * s1 - 7.5 * czzy, -7.5 * (double)bd[BD_SP + s]};
   pack_far_field(b, q, g, r);
 }
+// Rope positions of a node's children, whose first record is `pos`; kNoKid
+// where there are fewer than four.
+__device__ __forceinline__ uint4 kid_positions(const uint32_t* __restrict__ nodes,
+                                               const uint32_t* __restrict__ nslots_sub, uint32_t node, uint32_t pos) {
+  uint32_t k[4] = {kNoKid, kNoKid, kNoKid, kNoKid};
+  for (int s = 0; s < 4; ++s) {
+    const uint32_t c = nodes[4 * (int64_t)node + s];
+    if (c == NODE_EMPTY) break;
+    k[s] = pos;
+    pos += (c & NODE_INTERNAL) ? 1 + nslots_sub[c & ~NODE_INTERNAL] : 1;
+  }
+  return make_uint4(k[0], k[1], k[2], k[3]);
+}
+
 __global__ void k_write_slots(int64_t nn, const uint32_t* __restrict__ nodes, const float* __restrict__ boxdata,
                               const uint32_t* __restrict__ nslots_sub, const uint32_t* __restrict__ first_slot,
-                              float4* __restrict__ slots) {
+                              uint32_t nslots, float4* __restrict__ slots, uint4* __restrict__ kids) {
   int64_t node = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (node >= nn) return;
   const float* bd = boxdata + 92 * node;
   uint32_t pos = first_slot[node];
+  if (node == 0) kids[nslots] = kid_positions(nodes, nslots_sub, 0, 0);
   for (int s = 0; s < 4; ++s) {
     const uint32_t c = nodes[4 * node + s];
     if (c == NODE_EMPTY) break;
@@ -218,9 +233,11 @@ __global__ void k_write_slots(int64_t nn, const uint32_t* __restrict__ nodes, co
     if (c & NODE_INTERNAL) {
       next = pos + 1 + nslots_sub[c & ~NODE_INTERNAL];
       link = next;
+      kids[pos] = kid_positions(nodes, nslots_sub, c & ~NODE_INTERNAL, pos + 1);
     } else {
       next = pos + 1;
       link = LINK_LEAF | c;
+      kids[pos] = make_uint4(kNoKid, kNoKid, kNoKid, kNoKid);
     }
     float4* r = slots + 6 * (int64_t)pos;
     float v[20];
@@ -732,19 +749,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
   W[qi] = finish_walk<MIXED>(sum, ex, L, tri, qx, qy, qz);
 }
 
-// FP64 term of record i for query q: adds a far-field or exact term to part
-// and ex and returns true, or returns false when the walk descends into the
-// record.  link: the record's link word.
-template <int ORDER>
-__device__ __forceinline__ bool record_term64(const double* __restrict__ s64, const float* __restrict__ tri,
-                                              uint32_t i, uint32_t& link, double qx, double qy, double qz,
-                                              double acc2, double& part, SolidAngleSum<double>& ex) {
+// FP64 far field of record i for query q: added to part when the query is
+// beyond the record's radius and the value is finite, else false.  link: the
+// record's link word.
+// descend() is called before the far field's part of the record is read
+// (or, where the value is not finite, after) when it returns false.
+template <int ORDER, typename Descend>
+__device__ __forceinline__ bool record_far64(const double* __restrict__ s64, uint32_t i, uint32_t& link, double qx,
+                                             double qy, double qz, double acc2, double& part, Descend&& descend) {
   const double* r = s64 + 24 * (size_t)i;
   const D4 b{r[4], r[5], r[6], r[7]};
   link = (uint32_t)__double_as_longlong(b.w);
   const double x = qx - r[0], y = qy - r[1], z = qz - r[2];
   const double l2 = x * x + y * y + z * z;
-  if (!(l2 <= r[3] * acc2)) {
+  const bool beyond = !(l2 <= r[3] * acc2);
+  if (!beyond) descend();
+  if (beyond) {
     const D4 c{r[8], r[9], r[10], r[11]}, d{r[12], r[13], r[14], r[15]}, e{r[16], r[17], r[18], r[19]},
         f{r[20], r[21], r[22], r[23]};
     const double m = rsqrt64(l2), m2 = __dmul_rn(m, m);
@@ -753,10 +773,9 @@ __device__ __forceinline__ bool record_term64(const double* __restrict__ s64, co
       part = fma(m2, o, part);
       return true;
     }
+    descend();
   }
-  if (!(link & LINK_LEAF)) return false;
-  ex.add(tri + 9 * (size_t)(link & ~LINK_LEAF), qx, qy, qz);
-  return true;
+  return false;
 }
 
 // all-FP64 form: FP64 moments, far field, atan2 and sum
@@ -818,8 +837,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     ex = SolidAngleSum<double>();
     for (uint32_t j = 0; j < nslots;) {
       uint32_t link;
-      const bool done = record_term64<ORDER>(s64, tri, j, link, qx, qy, qz, acc2, sum, ex);
-      j = (done && !(link & LINK_LEAF)) ? link : j + 1;
+      const bool far = record_far64<ORDER>(s64, j, link, qx, qy, qz, acc2, sum, [] {});
+      const bool leaf = (link & LINK_LEAF) != 0;
+      if (leaf && !far) ex.add(tri + 9 * (size_t)(link & ~LINK_LEAF), qx, qy, qz);
+      j = (far && !leaf) ? link : j + 1;
     }
   }
   W[qi] = (sum + ex.total()) / (4.0 * PI_D);
@@ -829,22 +850,61 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
 // A sequential walk is a chain of dependent record fetches as long as the
 // query's path (thousands on a large mesh): a pass over a few hundred queries
 // runs a handful of wavefronts for milliseconds.  Here the 64 lanes of a
-// wavefront share one query's walk (ring_walk, ring_walk.h).  The records
+// wavefront share one query's walk (frontier_walk, ring_walk.h).  The records
 // visited and the terms are those of the sequential walk (each record's
 // decision depends on the record and the query only); their FP64 sum is taken
 // per lane and then across lanes in a fixed order, so the result is
 // deterministic and differs from the sequential sum only by rounding.
 
-// FP64 ring walk of query q: W = sum / 4 pi, the same on every lane
+// Records first .. end - 1 in rope order, every angle a term of its own: what
+// a frontier walk whose ring is full leaves to one lane.
 template <int ORDER>
-__device__ __forceinline__ double ring_walk64(uint2* __restrict__ ring, int lane, const double* __restrict__ s64,
-                                              uint32_t nslots, const float* __restrict__ tri, double qx, double qy,
-                                              double qz, double acc2) {
+__device__ __attribute__((noinline)) double subtree64(const double* __restrict__ s64, const float* __restrict__ tri,
+                                                      uint32_t first, uint32_t end, double qx, double qy, double qz,
+                                                      double acc2) {
+  double sum = 0.0;
+  for (uint32_t j = first; j < end;) {
+    uint32_t link;
+    const bool far = record_far64<ORDER>(s64, j, link, qx, qy, qz, acc2, sum, [] {});
+    const bool leaf = (link & LINK_LEAF) != 0;
+    if (leaf && !far) {
+      const float* p = tri + 9 * (size_t)(link & ~LINK_LEAF);
+      sum = __dadd_rn(sum, tri_solid_angle<double>(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], qx, qy, qz));
+    }
+    j = (far && !leaf) ? link : j + 1;
+  }
+  return sum;
+}
+
+// LDS of one query's frontier walk
+struct FrontierLds {
+  uint32_t ring[kFrontier];
+  uint32_t far[kExactQueue];
+};
+
+// FP64 frontier walk of a query: W = sum / 4 pi, the same on every lane
+template <int ORDER>
+__device__ __forceinline__ double frontier_walk64(FrontierLds& lds, uint32_t lane, const double* __restrict__ s64,
+                                                  const uint4* __restrict__ kids, uint32_t nslots,
+                                                  const float* __restrict__ tri, double qx, double qy, double qz,
+                                                  double acc2) {
   double part = 0.0;
   SolidAngleSum<double> ex;
-  ring_walk(ring, lane, nslots, [&](uint32_t i, uint32_t& link) {
-    return record_term64<ORDER>(s64, tri, i, link, qx, qy, qz, acc2, part, ex);
-  });
+  const auto exact = [&](uint32_t t) { ex.add(tri + 9 * (size_t)t, qx, qy, qz); };
+  frontier_walk(
+      lds.ring, lds.far, nullptr, lane, kids, nslots,
+      [&](uint32_t i, uint4& k, uint32_t& link, uint32_t& t) {
+        const auto descend = [&] {
+          if (!(link & LINK_LEAF)) k = kids[i];
+        };
+        if (record_far64<ORDER>(s64, i, link, qx, qy, qz, acc2, part, descend)) return Visit::kDone;
+        t = link & ~LINK_LEAF;
+        return (link & LINK_LEAF) ? Visit::kExact : Visit::kDescend;
+      },
+      exact, exact,
+      [&](uint32_t first, uint32_t end) {
+        part = __dadd_rn(part, subtree64<ORDER>(s64, tri, first, end, qx, qy, qz, acc2));
+      });
   return wave_sum(part + ex.total()) / (4.0 * PI_D);
 }
 
@@ -852,17 +912,18 @@ __device__ __forceinline__ double ring_walk64(uint2* __restrict__ ring, int lane
 // given, else n): 4 queries per 256-thread block, one per wavefront,
 // grid-strided.
 template <int ORDER>
-__global__ __launch_bounds__(256) void k_reeval64(const double* __restrict__ s64, uint32_t nslots,
+__global__ __launch_bounds__(256) void k_reeval64(const double* __restrict__ s64, const uint4* __restrict__ kids,
+                                                  uint32_t nslots,
                                                   const float* __restrict__ tri,
                                                   const float* __restrict__ Q, const uint32_t* __restrict__ list,
                                                   int64_t n, const uint32_t* __restrict__ dcount, double acc2,
                                                   double* __restrict__ W) {
-  __shared__ uint2 ring_all[4][kReevalRing];
+  __shared__ FrontierLds lds[4];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t count = dcount ? (int64_t)*dcount : n;
   for (int64_t k = (int64_t)blockIdx.x * 4 + wv; k < count; k += (int64_t)gridDim.x * 4) {
     const int64_t qi = list ? (int64_t)list[k] : k;
-    const double w = ring_walk64<ORDER>(ring_all[wv], lane, s64, nslots, tri, Q[3 * qi], Q[3 * qi + 1],
+    const double w = frontier_walk64<ORDER>(lds[wv], lane, s64, kids, nslots, tri, Q[3 * qi], Q[3 * qi + 1],
                                         Q[3 * qi + 2], acc2);
     if (lane == 0) W[qi] = w;
   }
@@ -873,83 +934,126 @@ __global__ __launch_bounds__(256) void k_reeval64(const double* __restrict__ s64
 // and each lane's sequential walk is a chain of dependent record fetches as
 // long as its path: at accuracy_scale 4.9 on a 434k-triangle mesh a batch of
 // 1,000 queries takes 1.4 ms however few queries it has.  Here each query gets
-// a wavefront and the ring walk above, so a query takes depth-many rounds.
-// The records visited and each term are those of the sequential walk (FP32
-// decisions and terms with the reference's rounding, FP64 near triangles in
-// the mixed form); the sum is taken per lane and then across lanes in a fixed
-// order, so results are deterministic and differ from the sequential walks'
-// running sums only by rounding.  In the mixed form k_reeval64_band then
-// walks the queries whose W falls in the ambiguous band again in FP64, so the
-// batch needs no collection pass and no count.
-// Mixed form: a lane notes the near triangles it meets (up to kRingDefer, in
-// LDS) and sums their FP64 solid angles after the walk, keeping the FP64 code
-// out of the walk's registers; a query with more than kRingDefer on one lane
-// gets W = NaN, which k_reeval64_band walks again in FP64.
-constexpr int kRingDefer = 4;
+// a wavefront and the frontier walk (ring_walk.h), so a query takes about one
+// round per tree level and per 64 records.  The records visited and each term
+// are those of the sequential walk (FP32 decisions and terms with the
+// reference's rounding, FP64 near triangles in the mixed form); the sum is
+// taken per lane and then across lanes in a fixed order, so results are
+// deterministic and differ from the sequential walks' running sums only by
+// rounding.  In the mixed form k_reeval64_band then walks the queries whose W
+// falls in the ambiguous band again in FP64, so the batch needs no collection
+// pass and no count.
+//
+// Few queries wait for memory, many queries for the vector cache, which
+// serves one lane's 16 bytes a cycle where every lane reads another record.
+// EARLY (below kEarlyFetchBelow queries) requests the whole record and the
+// children's positions at once; otherwise the first 32 bytes decide what else
+// a lane reads (5 pieces of 16 bytes a record instead of 7).  81,920
+// triangles, early / as needed: 10.3 / 10.8 us (1,000 queries at
+// accuracy_scale 2), 34 / 39 us (1,000 at 4.9), 41.5 / 41.9 us (2,000 at 4.9),
+// 90 / 67 us (4,000 at 4.9).  Fetching records through LDS, eight lanes a
+// record, measured between the two: its 8 KiB a wavefront halve the
+// wavefronts in flight.  Against the walk by ranges of siblings with each
+// triangle evaluated where it was met: 1,000 queries at 2 25 -> 10 us, 20,000
+// at 2 108 -> 60 us, 60,000 at 3 399 -> 321 us; mixed form, 5,003 queries on
+// 119,000 triangles at 4.9 182 -> 138 us, 60,000 on 5,000 triangles at 3
+// 458 -> 171 us.
+constexpr int64_t kEarlyFetchBelow = 2048;
 
-// FP32 and mixed forms (the FP64 form is k_reeval64 over every query).  Held
-// to 8 wavefronts per SIMD: the walk fits in 64 VGPRs; the mixed form's FP64
-// tail would take more and keeps some of its values in scratch instead.
+// Records first .. end - 1 in rope order, the mixed form's near triangles in
+// FP64: what a frontier walk whose ring is full leaves to one lane.
 template <int ORDER, bool MIXED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_walk_ring(
-    const float4* __restrict__ slots, uint32_t nslots, const float* __restrict__ tri, const float* __restrict__ Q,
-    int64_t nq, float acc2f, float near_d, double* __restrict__ W) {
-  __shared__ uint2 ring_all[4][kReevalRing];
-  __shared__ uint32_t near_all[MIXED ? 4 * kRingDefer * 64 : 1];
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  uint2* ring = ring_all[wv];
-  uint32_t* near = near_all + (MIXED ? wv * kRingDefer * 64 + lane : 0);  // this lane's column
-  for (int64_t qi = (int64_t)blockIdx.x * 4 + wv; qi < nq; qi += (int64_t)gridDim.x * 4) {
-    const float qx = Q[3 * qi], qy = Q[3 * qi + 1], qz = Q[3 * qi + 2];
-    double w;
-    {
-      float p32 = 0.0f;
-      uint32_t nn = 0;  // near triangles noted (kRingDefer + 1 after an overflow)
-      ring_walk(ring, lane, nslots, [&](uint32_t i, uint32_t& link) {
-        const float4* r = slots + 6 * (size_t)i;
-        // the whole record in one round trip (loading the far-field part only
-        // where it is used measured no faster)
-        const float4 a = r[0], b = r[1], c = r[2], d = r[3], e = r[4], f = r[5];
-        link = __float_as_uint(b.w);
-        const bool leaf = (link & LINK_LEAF) != 0;
-        const float x = qx - a.x, y = qy - a.y, z = qz - a.z;
-        // rounded as the reference rounds it (no fused multiply-add)
-        const float l2 = __fadd_rn(__fadd_rn(__fmul_rn(x, x), __fmul_rn(y, y)), __fmul_rn(z, z));
-        if (!(l2 <= __fmul_rn(a.w, acc2f))) {
-          const float o = far_field_poly<ORDER>(x, y, z, l2, b, c, d, e, f);
-          if (isfinite(o)) {
-            p32 = __fadd_rn(p32, o);
-            return true;
-          }
-        }
-        if (!leaf) return false;
-        const uint32_t t = link & ~LINK_LEAF;
-        if (MIXED && near_triangle(a.w, l2, near_d)) {
-          if (nn < (uint32_t)kRingDefer) near[nn * 64] = t;
-          nn = nn < (uint32_t)kRingDefer ? nn + 1 : (uint32_t)kRingDefer + 1;
-        } else {
-          const float* p = tri + 9 * (size_t)t;
-          p32 = __fadd_rn(p32, tri_solid_angle_fast(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], qx, qy,
-                                                    qz));
-        }
-        return true;
-      });
-      const float s32 = wave_sum(p32);
-      if (!MIXED) {
-        w = (double)s32 / (4.0 * PI_D);
-      } else if (__ballot(nn > (uint32_t)kRingDefer) != 0) {
-        w = __longlong_as_double(0x7FF8000000000000ll);
-      } else {
-        double p64 = 0.0;
-        for (uint32_t k = 0; k < nn; ++k) {
-          const float* p = tri + 9 * (size_t)near[k * 64];
-          p64 = __dadd_rn(p64, tri_solid_angle<double>(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], qx, qy,
-                                                       qz));
-        }
-        w = ((double)s32 + wave_sum(p64)) / (4.0 * PI_D);
+__device__ __attribute__((noinline)) double subtree32(const float4* __restrict__ slots,
+                                                      const float* __restrict__ tri, uint32_t first, uint32_t end,
+                                                      float qx, float qy, float qz, float acc2, float near_d) {
+  float sum = 0.0f;
+  double sum64 = 0.0;
+  for (uint32_t j = first; j < end;) {
+    const float4* r = slots + 6 * (size_t)j;
+    const float4 a = r[0], b = r[1];
+    const uint32_t link = __float_as_uint(b.w);
+    const bool leaf = (link & LINK_LEAF) != 0;
+    const float x = qx - a.x, y = qy - a.y, z = qz - a.z;
+    const float l2 = __fadd_rn(__fadd_rn(__fmul_rn(x, x), __fmul_rn(y, y)), __fmul_rn(z, z));
+    if (!(l2 <= __fmul_rn(a.w, acc2))) {
+      const float o = far_field_poly<ORDER>(x, y, z, l2, b, r[2], r[3], r[4], r[5]);
+      if (isfinite(o)) {
+        sum = __fadd_rn(sum, o);
+        j = leaf ? j + 1 : link;
+        continue;
       }
     }
-    if (lane == 0) W[qi] = w;
+    if (leaf) {
+      const float* p = tri + 9 * (size_t)(link & ~LINK_LEAF);
+      if (MIXED && near_triangle(a.w, l2, near_d))
+        sum64 = __dadd_rn(sum64,
+                          tri_solid_angle<double>(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], qx, qy, qz));
+      else
+        sum = __fadd_rn(sum, tri_solid_angle_fast(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], qx, qy, qz));
+    }
+    ++j;
+  }
+  return (double)sum + sum64;
+}
+
+// FP32 and mixed forms (the FP64 form is k_reeval64 over every query).  FP32
+// fits 8 wavefronts per SIMD; the mixed form's FP64 terms spill outside the
+// walk at 8 and took 2 to 4% less time at 6 on batches of 60,000.
+template <int ORDER, bool MIXED, bool EARLY>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MIXED ? 6 : 8))) void k_walk_ring(
+    const float4* __restrict__ slots, const uint4* __restrict__ kids, uint32_t nslots, const float* __restrict__ tri,
+    const float* __restrict__ Q, int64_t nq, float acc2f, float near_d, double* __restrict__ W) {
+  __shared__ FrontierLds lds[4];
+  __shared__ uint32_t near_all[MIXED ? 4 * kExactQueue : 1];
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int64_t qi = (int64_t)blockIdx.x * 4 + wv; qi < nq; qi += (int64_t)gridDim.x * 4) {
+    const float qx = Q[3 * qi], qy = Q[3 * qi + 1], qz = Q[3 * qi + 2];
+    float p32 = 0.0f;
+    double rest = 0.0;
+    const auto exact = [&](uint32_t t) {
+      const float* p = tri + 9 * (size_t)t;
+      p32 = __fadd_rn(p32, tri_solid_angle_fast(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], qx, qy, qz));
+    };
+    const auto exact_near = [&](uint32_t t) {
+      const float* p = tri + 9 * (size_t)t;
+      if (MIXED)
+        rest = __dadd_rn(rest, tri_solid_angle<double>(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], qx, qy, qz));
+    };
+    frontier_walk(
+        lds[wv].ring, lds[wv].far, near_all + (MIXED ? wv * kExactQueue : 0), lane, kids, nslots,
+        [&](uint32_t i, uint4& k, uint32_t& link, uint32_t& t) {
+          const float4* r = slots + 6 * (size_t)i;
+          const float4 a = r[0], b = r[1];
+          float4 c, d, e, f;
+          if (EARLY) c = r[2], d = r[3], e = r[4], f = r[5], k = kids[i];
+          link = __float_as_uint(b.w);
+          const bool leaf = (link & LINK_LEAF) != 0;
+          const float x = qx - a.x, y = qy - a.y, z = qz - a.z;
+          // rounded as the reference rounds it (no fused multiply-add)
+          const float l2 = __fadd_rn(__fadd_rn(__fmul_rn(x, x), __fmul_rn(y, y)), __fmul_rn(z, z));
+          const bool beyond = !(l2 <= __fmul_rn(a.w, acc2f));
+          if (!EARLY && !beyond && !leaf) k = kids[i];  // on its way while the far fields are read
+          if (beyond) {
+            if (!EARLY) c = r[2], d = r[3], e = r[4], f = r[5];
+            const float o = far_field_poly<ORDER>(x, y, z, l2, b, c, d, e, f);
+            if (isfinite(o)) {
+              p32 = __fadd_rn(p32, o);
+              return Visit::kDone;
+            }
+            if (!EARLY && !leaf) k = kids[i];
+          }
+          if (!leaf) return Visit::kDescend;
+          t = link & ~LINK_LEAF;
+          return MIXED && near_triangle(a.w, l2, near_d) ? Visit::kExactNear : Visit::kExact;
+        },
+        exact, exact_near,
+        [&](uint32_t first, uint32_t end) {
+          rest = __dadd_rn(rest, subtree32<ORDER, MIXED>(slots, tri, first, end, qx, qy, qz, acc2f, near_d));
+        });
+    const float s32 = wave_sum(p32);
+    double w = (double)s32;
+    if (__ballot(rest != 0.0) != 0) w += wave_sum(rest);
+    if (lane == 0) W[qi] = w / (4.0 * PI_D);
   }
 }
 
@@ -958,14 +1062,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
 // A kernel of its own so that the FP64 walk's registers do not limit the
 // occupancy of the FP32 walk.
 template <int ORDER>
-__global__ __launch_bounds__(256) void k_reeval64_band(const double* __restrict__ s64, uint32_t nslots,
+__global__ __launch_bounds__(256) void k_reeval64_band(const double* __restrict__ s64, const uint4* __restrict__ kids,
+                                                  uint32_t nslots,
                                                        const float* __restrict__ tri, const float* __restrict__ Q,
                                                        int64_t nq, double acc2, double band, double* __restrict__ W) {
-  __shared__ uint2 ring_all[4][kReevalRing];
+  __shared__ FrontierLds lds[4];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   for (int64_t qi = (int64_t)blockIdx.x * 4 + wv; qi < nq; qi += (int64_t)gridDim.x * 4) {
-    if (fabs(W[qi] - 0.5) >= band) continue;  // wave-uniform; NaN (near-list overflow) is walked again
-    const double w = ring_walk64<ORDER>(ring_all[wv], lane, s64, nslots, tri, Q[3 * qi], Q[3 * qi + 1],
+    if (fabs(W[qi] - 0.5) >= band) continue;  // wave-uniform; NaN is walked again
+    const double w = frontier_walk64<ORDER>(lds[wv], lane, s64, kids, nslots, tri, Q[3 * qi], Q[3 * qi + 1],
                                         Q[3 * qi + 2], acc2);
     if (lane == 0) W[qi] = w;
   }
@@ -1147,8 +1252,9 @@ void soup_finish_build(gwn_soup* s, hipStream_t st) {
   GWN_HIP(hipStreamSynchronize(st));
   s->nslots = total;
   s->slots.alloc(6 * (size_t)total);
+  s->kids.alloc((size_t)total + 1);
   hipLaunchKernelGGL(k_write_slots, dim3(div_up(nn, 256)), dim3(256), 0, st, nn, s->nodes.p, s->boxdata.p, nsub.p,
-                     first.p, s->slots.p);
+                     first.p, total, s->slots.p, s->kids.p);
   check_launch("k_write_slots");
   build_fp64_moments(s, L, st);
   build_cost_grid(s, st);
@@ -1441,15 +1547,23 @@ static void launch_walk_ring(const gwn_soup* s, const float* Q, int64_t nq, floa
   ProfileScope prof("soup_walk_ring", st, prof_on);
   if (precision == GWN_PREC_FP64) {
     switch (s->order) {
-      case 0: hipLaunchKernelGGL(k_reeval64<0>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, nullptr, nq, nullptr, a2, W); break;
-      case 1: hipLaunchKernelGGL(k_reeval64<1>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, nullptr, nq, nullptr, a2, W); break;
-      default: hipLaunchKernelGGL(k_reeval64<2>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, nullptr, nq, nullptr, a2, W); break;
+      case 0: hipLaunchKernelGGL(k_reeval64<0>, dim3(g), dim3(256), 0, st, s->slots64.p, s->kids.p, ns, s->tri.p, Q, nullptr, nq, nullptr, a2, W); break;
+      case 1: hipLaunchKernelGGL(k_reeval64<1>, dim3(g), dim3(256), 0, st, s->slots64.p, s->kids.p, ns, s->tri.p, Q, nullptr, nq, nullptr, a2, W); break;
+      default: hipLaunchKernelGGL(k_reeval64<2>, dim3(g), dim3(256), 0, st, s->slots64.p, s->kids.p, ns, s->tri.p, Q, nullptr, nq, nullptr, a2, W); break;
     }
     check_launch("k_reeval64");
     return;
   }
-#define GWN_LAUNCH_R(O, M)                                                                                      \
-  hipLaunchKernelGGL((k_walk_ring<O, M>), dim3(g), dim3(256), 0, st, s->slots.p, ns, s->tri.p, Q, nq, acc2, nd, W)
+  const bool early = nq < kEarlyFetchBelow;
+#define GWN_LAUNCH_R(O, M)                                                                                          \
+  do {                                                                                                              \
+    if (early)                                                                                                      \
+      hipLaunchKernelGGL((k_walk_ring<O, M, true>), dim3(g), dim3(256), 0, st, s->slots.p, s->kids.p, ns, s->tri.p, \
+                         Q, nq, acc2, nd, W);                                                                       \
+    else                                                                                                            \
+      hipLaunchKernelGGL((k_walk_ring<O, M, false>), dim3(g), dim3(256), 0, st, s->slots.p, s->kids.p, ns,          \
+                         s->tri.p, Q, nq, acc2, nd, W);                                                             \
+  } while (0)
   const bool mixed = precision == GWN_PREC_MIXED;
   switch (s->order) {
     case 0: if (mixed) GWN_LAUNCH_R(0, true); else GWN_LAUNCH_R(0, false); break;
@@ -1460,9 +1574,9 @@ static void launch_walk_ring(const gwn_soup* s, const float* Q, int64_t nq, floa
   check_launch("k_walk_ring");
   if (mixed) {
     switch (s->order) {
-      case 0: hipLaunchKernelGGL(k_reeval64_band<0>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, nq, a2, band, W); break;
-      case 1: hipLaunchKernelGGL(k_reeval64_band<1>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, nq, a2, band, W); break;
-      default: hipLaunchKernelGGL(k_reeval64_band<2>, dim3(g), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, nq, a2, band, W); break;
+      case 0: hipLaunchKernelGGL(k_reeval64_band<0>, dim3(g), dim3(256), 0, st, s->slots64.p, s->kids.p, ns, s->tri.p, Q, nq, a2, band, W); break;
+      case 1: hipLaunchKernelGGL(k_reeval64_band<1>, dim3(g), dim3(256), 0, st, s->slots64.p, s->kids.p, ns, s->tri.p, Q, nq, a2, band, W); break;
+      default: hipLaunchKernelGGL(k_reeval64_band<2>, dim3(g), dim3(256), 0, st, s->slots64.p, s->kids.p, ns, s->tri.p, Q, nq, a2, band, W); break;
     }
     check_launch("k_reeval64_band");
   }
@@ -1577,9 +1691,9 @@ void soup_query_device_ws(const gwn_soup* s, const float* Q, int64_t nq, float a
       const unsigned gr = dcount ? (unsigned)std::min<int64_t>(div_up(na64, 4), 2048) : (unsigned)div_up(na64, 4);
       ProfileScope prof("soup_reeval64", st, prof_on);
       switch (s->order) {
-        case 0: hipLaunchKernelGGL(k_reeval64<0>, dim3(gr), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, amb, na64, dcount, a2, W); break;
-        case 1: hipLaunchKernelGGL(k_reeval64<1>, dim3(gr), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, amb, na64, dcount, a2, W); break;
-        default: hipLaunchKernelGGL(k_reeval64<2>, dim3(gr), dim3(256), 0, st, s->slots64.p, ns, s->tri.p, Q, amb, na64, dcount, a2, W); break;
+        case 0: hipLaunchKernelGGL(k_reeval64<0>, dim3(gr), dim3(256), 0, st, s->slots64.p, s->kids.p, ns, s->tri.p, Q, amb, na64, dcount, a2, W); break;
+        case 1: hipLaunchKernelGGL(k_reeval64<1>, dim3(gr), dim3(256), 0, st, s->slots64.p, s->kids.p, ns, s->tri.p, Q, amb, na64, dcount, a2, W); break;
+        default: hipLaunchKernelGGL(k_reeval64<2>, dim3(gr), dim3(256), 0, st, s->slots64.p, s->kids.p, ns, s->tri.p, Q, amb, na64, dcount, a2, W); break;
       }
       check_launch("k_reeval64");
     }

@@ -127,6 +127,29 @@ def test_ring_walk_and_sequential_walks_agree(order):
             assert np.array_equal(bvh.query(Q[:20000], beta, prec), Wsmall[:20000])
 
 
+@pytest.mark.parametrize("ntri", [1, 2, 3, 5, 17, 5120])
+@pytest.mark.parametrize("nq", [1, 2047, 2048])
+def test_frontier_walk_at_its_edges(ntri, nq):
+    """The one-wavefront walk against the wave-coherent one on the same queries:
+    trees whose root has 1 to 4 children, records fetched whole (below 2,048
+    queries) or as needed, and at accuracy_scale 1e3, where nothing is far, a
+    frontier of more records than the ring holds (5,120 triangles) and triangle
+    queues that fill many times."""
+    V, F = D.bumpy_sphere(4, 16, 57)
+    F = F[:ntri]
+    rng = np.random.default_rng(57)
+    near = D.near_surface_queries(V, F, nq - nq // 2, 5e-4, rng)  # within near_dist: FP64 terms in the mixed form
+    Q = np.concatenate([near, rng.uniform(-1.4, 1.4, (nq // 2, 3))])
+    fill = rng.uniform(-1.4, 1.4, (65_536 - nq, 3))
+    bvh = gwn.FastWindingNumberBVH().build(V, F, 2)
+    for beta in (2.0, 1e3):
+        for prec, tol in ((gwn.PREC_FP32, 1e-5), (gwn.PREC_MIXED, 1e-5), (gwn.PREC_FP64, 1e-12)):
+            W = bvh.query(Q, beta, prec)
+            Wwave = bvh.query(np.concatenate([Q, fill]), beta, prec)[:nq]
+            assert np.abs(W - Wwave).max() <= tol, (beta, prec)
+            assert np.array_equal(W[:1], bvh.query(Q[:1], beta, prec))
+
+
 @pytest.mark.parametrize("order", [0, 1, 2])
 @pytest.mark.parametrize("nq", [300, 65_541])
 def test_far_fields_that_overflow_are_descended(order, nq):
