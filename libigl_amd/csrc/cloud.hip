@@ -619,9 +619,18 @@ __global__ void k_rec_write(int64_t ncells, const int32_t* __restrict__ CH, cons
 // with E1[u][v] = EC[3 + u + 3v] and E2[i][u][v] = EC[12 + 9i + u + 3v].  This
 // is exact algebra; only the rounding of the far field changes (~1e-7
 // relative), and the near/far decisions do not use it.
+//
+// The record's free word holds the square of the cell's radius for the far
+// test of k_cloud_traverse; NaN where FP32 does not hold it to rounding or a
+// caller's radius is negative, which leaves the test to its exact form.
+__device__ __forceinline__ float square_for_test(float r) {
+  const float r2 = r * r;
+  return r == 0.0f || (r > 0.0f && r2 >= 1e-30f && r2 <= 1e37f) ? r2 : __builtin_nanf("");
+}
+
 template <int NT>
 __global__ void k_rec_poly(uint32_t nrec, const uint2* __restrict__ meta, const float* __restrict__ EC,
-                           float4* __restrict__ poly) {
+                           const float* __restrict__ R, float4* __restrict__ poly) {
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= nrec) return;
   const uint2 m = meta[p];
@@ -684,7 +693,7 @@ __global__ void k_rec_poly(uint32_t nrec, const uint2* __restrict__ meta, const 
   float v[20];
   pack_far_field(b, q, g, v);
   float4* r = poly + 5 * (size_t)p;  // b, c, d, e, f of far_field_bracket
-  r[0] = make_float4(v[0], v[1], v[2], 0.0f);
+  r[0] = make_float4(v[0], v[1], v[2], square_for_test(R[m.y]));
   for (int j = 1; j < 5; ++j) r[j] = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
 }
 
@@ -705,6 +714,10 @@ __device__ __forceinline__ float dipole(float lx, float ly, float lz, float ax, 
 // walk in order (results independent of the other queries in its wave) while
 // every record, leaf point and coefficient a wave reads is the same for all
 // its lanes and is fetched once through the scalar cache.
+// Bound by VALU issue, as the soup's walk: the conditions are scalar lane
+// masks, and the test by squares takes 4 instructions where the root, two
+// conversions and a double product took 17.  2M points, 4.1M queries: 1.24 ->
+// 1.05 ms.
 template <int NT>
 __global__ __launch_bounds__(256) void k_cloud_traverse(const float4* __restrict__ head, const uint2* __restrict__ meta,
                                                         uint32_t nrec, const float4* __restrict__ poly,
@@ -723,6 +736,13 @@ __global__ __launch_bounds__(256) void k_cloud_traverse(const float4* __restrict
     for (int64_t j = 0; j < npts; ++j)
       wn += dipole(Ps[3 * j] - qx, Ps[3 * j + 1] - qy, Ps[3 * j + 2] - qz, NAs[3 * j], NAs[3 * j + 1], NAs[3 * j + 2]);
   } else {
+    // The reference's test is sqrt(l2) > beta R, the root a float and the
+    // product a double.  Compared as squares, l2 and beta^2 R^2 decide it
+    // wherever they are apart by more than the roundings (3e-7 at most); only
+    // a lane in between takes the root.
+    const float b2 = (float)(beta * beta);
+    const bool plain = beta >= 1e-3 && beta <= 1e6;
+    const float far2 = plain ? b2 * (1.0f + 1e-6f) : __builtin_nanf(""), near2 = plain ? b2 * (1.0f - 1e-6f) : far2;
     uint32_t i = 0, skip = 0;
     while (i < nrec) {
       const uint2 m = meta[i];
@@ -733,28 +753,32 @@ __global__ __launch_bounds__(256) void k_cloud_traverse(const float4* __restrict
       // (the compiler would otherwise wait for meta, then for the decision,
       // before requesting the rest; measured 1.84 -> 1.72 ms on 4.1M queries)
       asm volatile("" ::"s"(m.x), "s"(m.y), "s"(h.x), "s"(h.w), "s"(r0.x), "s"(r2.x), "s"(r4.w));
-      const bool leaf = (m.x & REC_LEAF) != 0;
-      if (skip == i) {
-        skip = i + 1;
-        if (leaf) {
+      const uint64_t part = lanes_at_most(skip, i);
+      if ((m.x & REC_LEAF) != 0) {
+        // a lane that sums the leaf's points leaves skip at i, below i + 1
+        if (lane_in(part)) {
           const int64_t s = m.x & ~REC_LEAF;
           for (uint32_t j = 0; j < m.y; ++j) {
             const int64_t k = s + j;
             wn += dipole(Ps[3 * k] - qx, Ps[3 * k + 1] - qy, Ps[3 * k + 2] - qz, NAs[3 * k], NAs[3 * k + 1],
                          NAs[3 * k + 2]);
           }
-        } else {
-          const float lx = h.x - qx, ly = h.y - qy, lz = h.z - qz;
-          const float l2 = lx * lx + ly * ly + lz * lz;
-          if ((double)sqrtf(l2) > beta * (double)h.w) {
-            constexpr int ORDER = NT == 3 ? 0 : NT == 12 ? 1 : 2;
-            wn += far_field_poly<ORDER>(lx, ly, lz, l2, r0, r1, r2, r3, r4);
-            skip = m.x;
-          }
         }
+        i = __builtin_amdgcn_readfirstlane(i + 1);
+        continue;
       }
-      const bool step = leaf || __ballot(skip == i + 1) != 0;
-      i = __builtin_amdgcn_readfirstlane(step ? i + 1 : m.x);
+      const float lx = h.x - qx, ly = h.y - qy, lz = h.z - qz;
+      const float l2 = lx * lx + ly * ly + lz * lz;
+      uint64_t far = part & lanes_above(l2, r0.w * far2);
+      if ((part & ~far & ~lanes_below_value(l2, r0.w * near2)) != 0)
+        far = part & __builtin_amdgcn_fcmp((double)sqrtf(l2), beta * (double)h.w, 2);  // FCMP_OGT
+      if (lane_in(far)) {
+        constexpr int ORDER = NT == 3 ? 0 : NT == 12 ? 1 : 2;
+        const float k = __builtin_amdgcn_rsqf(l2);
+        wn = fmaf(k * k, far_field_bracket<ORDER>(lx, ly, lz, k, r0, r1, r2, r3, r4), wn);
+        skip = m.x;
+      }
+      i = __builtin_amdgcn_readfirstlane((part & ~far) != 0 ? i + 1 : m.x);
     }
   }
   WN[qi] = wn;
@@ -1006,11 +1030,14 @@ static void rope_records(gwn_cloud* c, const SplitCell* all, const std::vector<u
   c->poly.alloc(5 * (size_t)c->nrec);
   const unsigned gp = (unsigned)div_up(c->nrec, 256);
   if (c->nterms == 3)
-    hipLaunchKernelGGL(k_rec_poly<3>, dim3(gp), dim3(256), 0, st, (uint32_t)c->nrec, c->meta.p, c->EC.p, c->poly.p);
+    hipLaunchKernelGGL(k_rec_poly<3>, dim3(gp), dim3(256), 0, st, (uint32_t)c->nrec, c->meta.p, c->EC.p,
+                       c->R.p, c->poly.p);
   else if (c->nterms == 12)
-    hipLaunchKernelGGL(k_rec_poly<12>, dim3(gp), dim3(256), 0, st, (uint32_t)c->nrec, c->meta.p, c->EC.p, c->poly.p);
+    hipLaunchKernelGGL(k_rec_poly<12>, dim3(gp), dim3(256), 0, st, (uint32_t)c->nrec, c->meta.p, c->EC.p,
+                       c->R.p, c->poly.p);
   else
-    hipLaunchKernelGGL(k_rec_poly<39>, dim3(gp), dim3(256), 0, st, (uint32_t)c->nrec, c->meta.p, c->EC.p, c->poly.p);
+    hipLaunchKernelGGL(k_rec_poly<39>, dim3(gp), dim3(256), 0, st, (uint32_t)c->nrec, c->meta.p, c->EC.p,
+                       c->R.p, c->poly.p);
   check_launch("k_rec_poly");
   GWN_HIP(hipStreamSynchronize(st));
 }

@@ -4,6 +4,21 @@
 
 namespace gwn {
 
+// Lane masks of a wavefront held in scalar registers.  (A condition kept as a
+// bool and balloted later costs two VALU instructions more.)
+__device__ __forceinline__ uint64_t lanes_at_most(uint32_t v, uint32_t i) {
+  return __builtin_amdgcn_uicmp(v, i, 37);  // ICMP_ULE
+}
+__device__ __forceinline__ uint64_t lanes_beyond(float l2, float r2) {
+  return __builtin_amdgcn_fcmpf(l2, r2, 10);  // FCMP_UGT: !(l2 <= r2)
+}
+__device__ __forceinline__ uint64_t lanes_beyond(double l2, double r2) { return __builtin_amdgcn_fcmp(l2, r2, 10); }
+__device__ __forceinline__ uint64_t lanes_above(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 2); }  // OGT
+__device__ __forceinline__ uint64_t lanes_below_value(float a, float b) {
+  return __builtin_amdgcn_fcmpf(a, b, 4);  // OLT
+}
+__device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+
 // atan on [0,1] as a * P(a^2), P of degree 8: a weighted least-squares /
 // Lawson fit to atan(x)/x on 4000 Chebyshev nodes (computed for this
 // library); max error 1.2e-8 in exact arithmetic, ~1e-7 rad when evaluated in

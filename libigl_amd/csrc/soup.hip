@@ -632,17 +632,6 @@ __device__ __forceinline__ float in_vgpr(float x) {
   return v;
 }
 
-// Lane masks of a wavefront held in scalar registers.  (A condition kept as a
-// bool and balloted later costs two VALU instructions more.)
-__device__ __forceinline__ uint64_t lanes_at_most(uint32_t v, uint32_t i) {
-  return __builtin_amdgcn_uicmp(v, i, 37);  // ICMP_ULE
-}
-__device__ __forceinline__ uint64_t lanes_beyond(float l2, float r2) {
-  return __builtin_amdgcn_fcmpf(l2, r2, 10);  // FCMP_UGT: !(l2 <= r2)
-}
-__device__ __forceinline__ uint64_t lanes_beyond(double l2, double r2) { return __builtin_amdgcn_fcmp(l2, r2, 10); }
-__device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
-
 // HANDOVER: a wavefront whose lanes have stopped sharing records (fewer than
 // 16 lanes per step on average over a window of 256 steps: the union of their
 // paths exceeds the longest by far, as on fans of thin triangles) hands over

@@ -249,3 +249,33 @@ def test_from_octree_rejects_bad_trees():
     o = O.Octree(P, np.float32)
     assert np.array_equal(CH2, o.CH) and np.array_equal(CN2, o.CN) and np.array_equal(W2, o.W)
     assert all(pi[k] == o.point_indices(k).tolist() for k in range(len(pi)))
+
+
+@pytest.mark.parametrize("radius", [1.0, 0.0, -1.0, 1e-20, 1e25])
+@pytest.mark.parametrize("beta", [1e-4, 2.0, 1e7])
+def test_far_test_by_squares(radius, beta):
+    """The far test compares squares where FP32 holds them and takes the root
+    otherwise.  A caller's radii times `radius`: as they are, zero, negative,
+    and with squares outside FP32's range; beta inside and outside the plain
+    range; queries at cell centres and at the threshold to a last bit either
+    way.  The decisions are the oracle's, which takes the root and the double
+    product everywhere: a wrong one would show as a whole cell's error."""
+    P, N, A = _cloud(5000, seed=29)
+    o = O.Octree(P, np.float32)
+    lists = _lists(o)
+    CM, R, EC, _ = O.cloud_over(P, N, A, O.Octree.from_lists(o.CH, lists, np.float32), 2)
+    R = (R * np.float32(radius)).astype(np.float32)
+    *_, ev = O.cloud_over(P, N, A, O.Octree.from_lists(o.CH, lists, np.float32), 2, CM=CM, R=R, EC=EC)
+    rng = np.random.default_rng(29)
+    k = rng.integers(0, CM.shape[0], 400)
+    k = k[o.cell_count[k] > 0]
+    with np.errstate(over="ignore", invalid="ignore"):
+        edge = CM[k] + np.stack([np.float64(beta) * R[k]] + [np.zeros(k.size)] * 2, 1).astype(np.float32)
+    edge = edge[np.isfinite(edge).all(1) & (np.abs(edge) < 1e6).all(1)]
+    Q = np.concatenate([edge, np.nextafter(edge, np.float32(9)), np.nextafter(edge, np.float32(-9)), CM[k],
+                        rng.uniform(-1.3, 1.3, (500, 3))]).astype(np.float32)
+    W, Wo = gwn.fast_winding_number(P, N, A, lists, o.CH, CM, R, EC, Q, beta), ev(Q, beta)
+    ok = np.isfinite(Wo) & (np.abs(Wo) < 1e3)  # not at a centre taken for far
+    assert ok.sum() > 500
+    d = np.abs(W - Wo)[ok] / np.maximum(1.0, np.abs(Wo[ok]))
+    assert (d <= 2e-4).all(), (d.max(), int((d > 2e-4).sum()))
