@@ -15,19 +15,25 @@
 //              sorted; each run of equal keys sums to the edge's net count;
 //              non-zero nets become segments oriented so the weight is > 0
 //   frac       per query, the boundary sum in FP64 (segments staged in LDS)
-//   crossings  all rays share the direction x0, so the queries are taken in
-//              Hilbert order and a wavefront walks the soup's rope of slot
-//              boxes coherently (as the closest-point search does): a lane
-//              enters a slot whose box its ray meets (FP64 slab test on boxes
-//              rounded outward) and counts its triangle with the watertight
-//              ray-triangle test of Woop, Benthin and Wald (JCGT 2013) in FP64.
+//   crossings  all rays share the direction x0, so the tree and its slot boxes
+//              are built over the mesh in a frame (u, v, w) whose w axis is x0:
+//              a ray is then a point of the (u, v) plane and meets a box when
+//              it lies in the box's rectangle and starts below the box's top,
+//              five FP32 comparisons.  The queries are taken along a Hilbert
+//              curve of that plane, so a wavefront's 64 rays pass through
+//              nearly the same boxes, and walk the rope coherently (as the
+//              closest-point search does).  The boxes only cull: each triangle
+//              left is counted with the watertight ray-triangle test of Woop,
+//              Benthin and Wald (JCGT 2013) in FP64, in the mesh's own frame.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
 #include <vector>
 
+#include "device_math.h"
 #include "gwn_internal.h"
+#include "ring_walk.h"
 
 namespace gwn {
 namespace {
@@ -128,38 +134,45 @@ __global__ void k_ap_zero(double* __restrict__ W, int64_t n) {
   if (i < n) W[i] = 0.0;
 }
 
-__global__ void k_ap_narrow(const double* __restrict__ O, int64_t n, float* __restrict__ Of) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < 3 * n) Of[i] = (float)O[i];
-}
-
 // ---------------- signed crossings ----------------
 struct Ray {
   double d[3];    // direction x0
-  double inv[3];  // 1 / d (unused on an axis where d is 0)
   int kx, ky, kz; // watertight shear: kz the dominant axis
   double sx, sy, sz;
 };
 
-// does the ray o + t d, t >= 0, meet the box?  (boxes are rounded outward)
-__device__ __forceinline__ bool ap_box(const Ray& r, const double* o, const float4& lo, const float4& hi) {
-  const double l[3] = {lo.x, lo.y, lo.z}, h[3] = {hi.x, hi.y, hi.z};
-  double tmin = 0.0, tmax = INFINITY;
-  for (int a = 0; a < 3; ++a) {
-    if (r.d[a] == 0.0) {
-      if (o[a] < l[a] || o[a] > h[a]) return false;
-    } else {
-      double t0 = (l[a] - o[a]) * r.inv[a], t1 = (h[a] - o[a]) * r.inv[a];
-      if (t0 > t1) {
-        const double t = t0;
-        t0 = t1;
-        t1 = t;
-      }
-      tmin = t0 > tmin ? t0 : tmin;
-      tmax = t1 < tmax ? t1 : tmax;
-    }
-  }
-  return tmin <= tmax;
+// Frame of the rays: rows u, v, w (w = d / |d|), and the size of the mesh.
+struct RayFrame {
+  double m[3][3];
+  double reach;  // largest coordinate of the mesh in magnitude
+};
+
+// the largest float not above x, the smallest not below it
+__device__ __forceinline__ float ap_down(double x) {
+  const float f = (float)x;
+  return (double)f > x ? nextafterf(f, -INFINITY) : f;
+}
+__device__ __forceinline__ float ap_up(double x) {
+  const float f = (float)x;
+  return (double)f < x ? nextafterf(f, INFINITY) : f;
+}
+
+// Query order: the origins' (u, v), narrowed.
+__global__ void k_ap_plane(const double* __restrict__ O, int64_t n, RayFrame f, float* __restrict__ Of) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double x = O[3 * i], y = O[3 * i + 1], z = O[3 * i + 2];
+  Of[3 * i] = (float)(f.m[0][0] * x + f.m[0][1] * y + f.m[0][2] * z);
+  Of[3 * i + 1] = (float)(f.m[1][0] * x + f.m[1][1] * y + f.m[1][2] * z);
+  Of[3 * i + 2] = 0.0f;
+}
+
+// The corners of each face, 9 doubles (one run of scalar loads a triangle).
+__global__ void k_ap_corners(const double* __restrict__ V, const int32_t* __restrict__ F, int64_t nf,
+                             double* __restrict__ T) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= 3 * nf) return;
+  for (int a = 0; a < 3; ++a) T[3 * i + a] = V[3 * (int64_t)F[i] + a];
 }
 
 // +1 / -1 for a crossing of triangle (A, B, C) at t >= 0, 0 for none
@@ -183,39 +196,103 @@ __device__ __forceinline__ int ap_cross(const Ray& r, const double* o, const dou
   return (r.d[0] * n[0] + r.d[1] * n[1]) + r.d[2] * n[2] > 0.0 ? 1 : -1;
 }
 
+// A ray in the frame, widened by more than the roundings of the rotation (of
+// its origin here and of the vertices under the boxes), and outward to float.
+struct FlatRay {
+  float u0, u1, v0, v1, w0;
+};
+__device__ __forceinline__ FlatRay flat_ray(const RayFrame& f, const double* o) {
+  const double margin = 1e-14 * (f.reach + fabs(o[0]) + fabs(o[1]) + fabs(o[2]));
+  const double u = f.m[0][0] * o[0] + f.m[0][1] * o[1] + f.m[0][2] * o[2];
+  const double v = f.m[1][0] * o[0] + f.m[1][1] * o[1] + f.m[1][2] * o[2];
+  const double w = f.m[2][0] * o[0] + f.m[2][1] * o[1] + f.m[2][2] * o[2];
+  return {ap_down(u - margin), ap_up(u + margin), ap_down(v - margin), ap_up(v + margin), ap_down(w - margin)};
+}
+// An infinite origin meets no box (a NaN one meets every box).
+__device__ __forceinline__ bool no_ray(const double* o) { return isinf(o[0]) || isinf(o[1]) || isinf(o[2]); }
+
+__device__ __forceinline__ int tri_cross(const Ray& r, const double* o, const double* __restrict__ p) {
+  const double A[3] = {p[0], p[1], p[2]}, B[3] = {p[3], p[4], p[5]}, C[3] = {p[6], p[7], p[8]};
+  return ap_cross(r, o, A, B, C);
+}
+
+// One step is 10 VALU instructions (45 with the FP64 slab test of boxes in the
+// mesh's frame, and more steps: rays ordered by their origins share fewer
+// boxes).  81,920 triangles, 1M queries: 2.03 -> 0.28 ms a call; with w in the
+// rays' order 0.74 ms.
 __global__ __launch_bounds__(256) void k_ap_crossings(const float4* __restrict__ dbox, uint32_t nslots,
-                                                      const double* __restrict__ V, const int32_t* __restrict__ F,
-                                                      const double* __restrict__ O, const uint32_t* __restrict__ perm,
-                                                      int64_t no, Ray r, double* __restrict__ W) {
+                                                      const double* __restrict__ tri, const double* __restrict__ O,
+                                                      const uint32_t* __restrict__ perm, int64_t no, Ray r,
+                                                      RayFrame f, double* __restrict__ W) {
   const int64_t t = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
   if (t >= no) return;
   const int64_t qi = perm[t];
   const double o[3] = {O[3 * qi], O[3 * qi + 1], O[3 * qi + 2]};
+  const FlatRay q = flat_ray(f, o);
   int count = 0;
-  uint32_t skip = 0, i = 0;
+  uint32_t i = 0, skip = no_ray(o) ? nslots : 0;
   while (i < nslots) {
     const float4 lo = dbox[2 * (size_t)i], hi = dbox[2 * (size_t)i + 1];
     // the whole 32-byte record in one scalar-cache round trip, not the link
     // first and the box after it
     asm volatile("" ::"s"(lo.x), "s"(lo.w), "s"(hi.z));
     const uint32_t link = __float_as_uint(lo.w);
-    const bool leaf = (link & AP_LEAF) != 0;
-    if (skip == i) {
-      skip = i + 1;
-      if (!ap_box(r, o, lo, hi)) {
-        if (!leaf) skip = link;
-      } else if (leaf) {
-        const int32_t* tf = F + 3 * (size_t)(link & ~AP_LEAF);
-        const double A[3] = {V[3 * (int64_t)tf[0]], V[3 * (int64_t)tf[0] + 1], V[3 * (int64_t)tf[0] + 2]};
-        const double B[3] = {V[3 * (int64_t)tf[1]], V[3 * (int64_t)tf[1] + 1], V[3 * (int64_t)tf[1] + 2]};
-        const double C[3] = {V[3 * (int64_t)tf[2]], V[3 * (int64_t)tf[2] + 1], V[3 * (int64_t)tf[2] + 2]};
-        count += ap_cross(r, o, A, B, C);
-      }
+    // the lanes that need this record, and of them those whose ray meets the
+    // box (all of them but on a comparison that holds); a lane that does
+    // leaves skip at i, below the record it needs next
+    const uint64_t part = lanes_at_most(skip, i);
+    const uint64_t miss = lanes_below_value(q.u1, lo.x) | lanes_above(q.u0, hi.x) | lanes_below_value(q.v1, lo.y) |
+                          lanes_above(q.v0, hi.y) | lanes_above(q.w0, hi.z);
+    const uint64_t meet = part & ~miss;
+    if ((link & AP_LEAF) != 0) {
+      if (meet != 0 && lane_in(meet)) count += tri_cross(r, o, tri + 9 * (size_t)(link & ~AP_LEAF));
+      i = __builtin_amdgcn_readfirstlane(i + 1);
+    } else {
+      if (lane_in(part & miss)) skip = link;
+      i = __builtin_amdgcn_readfirstlane(meet != 0 ? i + 1 : link);
     }
-    const bool step = leaf || __ballot(skip == i + 1) != 0;
-    i = __builtin_amdgcn_readfirstlane(step ? i + 1 : link);
   }
   W[qi] = W[qi] + (double)count;  // frac + c (WindingNumberAntipodalScene.h:104)
+}
+
+// The same count with one wavefront per ray (frontier_walk), in input order:
+// a wavefront of 64 rays that lie far apart walks the union of their boxes.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_ap_crossings_ring(
+    const float4* __restrict__ dbox, const uint4* __restrict__ kids, uint32_t nslots, const double* __restrict__ tri,
+    const double* __restrict__ O, int64_t no, Ray r, RayFrame f, double* __restrict__ W) {
+  __shared__ uint32_t ring[4][kFrontier], queue[4][kExactQueue];
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t qi = (int64_t)blockIdx.x * 4 + wv;
+  if (qi >= no) return;
+  const double o[3] = {O[3 * qi], O[3 * qi + 1], O[3 * qi + 2]};
+  if (no_ray(o)) return;
+  const FlatRay q = flat_ray(f, o);
+  int count = 0;
+  const auto meets = [&](uint32_t i, uint32_t& link) {
+    const float4 lo = dbox[2 * (size_t)i], hi = dbox[2 * (size_t)i + 1];
+    link = __float_as_uint(lo.w);
+    return !(q.u1 < lo.x || q.u0 > hi.x || q.v1 < lo.y || q.v0 > hi.y || q.w0 > hi.z);
+  };
+  const auto cross = [&](uint32_t t) { count += tri_cross(r, o, tri + 9 * (size_t)t); };
+  frontier_walk(
+      ring[wv], queue[wv], nullptr, lane, kids, nslots,
+      [&](uint32_t i, uint4& k, uint32_t& link, uint32_t& t) {
+        k = kids[i];
+        if (!meets(i, link)) return Visit::kDone;
+        t = link & ~AP_LEAF;
+        return (link & AP_LEAF) ? Visit::kExact : Visit::kDescend;
+      },
+      cross, cross,
+      [&](uint32_t first, uint32_t end) {
+        for (uint32_t j = first; j < end;) {
+          uint32_t link;
+          const bool in = meets(j, link), leaf = (link & AP_LEAF) != 0;
+          if (in && leaf) cross(link & ~AP_LEAF);
+          j = in || leaf ? j + 1 : link;
+        }
+      });
+  for (int off = 32; off >= 1; off >>= 1) count += __shfl_xor(count, off, 64);
+  if (lane == 0) W[qi] = W[qi] + (double)count;
 }
 
 }  // namespace
@@ -271,10 +348,46 @@ void antipodal_build(gwn_antipodal* a, const double* V, int64_t nv, const int32_
   GWN_CHECK(std::isfinite(a->x0[0]) && std::isfinite(a->x0[1]) && std::isfinite(a->x0[2]) &&
                 (a->x0[0] != 0.0 || a->x0[1] != 0.0 || a->x0[2] != 0.0),
             GWN_ERR_INVALID, "x0 must be a finite non-zero direction");
-  soup_build_into(&a->soup, V, nv, F, nf, GWN_TREE_LBVH);
+  GWN_CHECK(nv == 0 || V != nullptr, GWN_ERR_INVALID, "null vertices");
+  // the frame of the rays: w along x0, u and v any two axes across it
+  const double* x = a->x0;
+  const double len = std::sqrt((x[0] * x[0] + x[1] * x[1]) + x[2] * x[2]);
+  int k0 = 0;  // the axis least along x0
+  for (int k = 1; k < 3; ++k)
+    if (std::fabs(x[k]) < std::fabs(x[k0])) k0 = k;
+  double(&m)[3][3] = a->frame;
+  for (int k = 0; k < 3; ++k) m[2][k] = x[k] / len;
+  const double dot = m[2][k0], across = std::sqrt(1.0 - dot * dot);
+  for (int k = 0; k < 3; ++k) m[0][k] = ((k == k0 ? 1.0 : 0.0) - dot * m[2][k]) / across;
+  for (int k = 0; k < 3; ++k) m[1][k] = m[2][(k + 1) % 3] * m[0][(k + 2) % 3] - m[2][(k + 2) % 3] * m[0][(k + 1) % 3];
+  std::vector<double> turned(3 * (size_t)nv);
+  a->reach = 0.0;
+  for (int64_t i = 0; i < nv; ++i)
+    for (int k = 0; k < 3; ++k) {
+      turned[3 * i + k] = m[k][0] * V[3 * i] + m[k][1] * V[3 * i + 1] + m[k][2] * V[3 * i + 2];
+      if (std::isfinite(V[3 * i + k]) && std::fabs(V[3 * i + k]) > a->reach) a->reach = std::fabs(V[3 * i + k]);
+    }
+  a->soup.boxes_only = true;
+  soup_build_into(&a->soup, turned.data(), nv, F, nf, GWN_TREE_LBVH);
   if (nf > 0) soup_ensure_dist(&a->soup, st);
-  a->nseg = ap_boundary(a->soup.V64.p, a->soup.F.p, nf, a->seg, st);
+  DevBuf<double> dV(3 * (size_t)nv);
+  if (nv > 0) GWN_HIP(hipMemcpyAsync(dV.p, V, sizeof(double) * 3 * (size_t)nv, hipMemcpyHostToDevice, st));
+  a->tri.alloc(9 * (size_t)nf);
+  if (nf > 0) {
+    hipLaunchKernelGGL(k_ap_corners, dim3(div_up(3 * nf, 256)), dim3(256), 0, st, dV.p, a->soup.F.p, nf, a->tri.p);
+    check_launch("k_ap_corners");
+  }
+  a->nseg = ap_boundary(dV.p, a->soup.F.p, nf, a->seg, st);
+  GWN_HIP(hipStreamSynchronize(st));
 }
+
+// Batches below this, and up to kRingRaysMost those of fewer than two rays per
+// triangle, take a wavefront per ray: 64 rays further apart than the triangles share few boxes.  Ring /
+// wave: 1,000 rays on 81,920 triangles 18 / 466 us, 65,001 on 20,480 101 / 149
+// us, 200,000 on 100,000 347 / 521 us, 400,000 on 100,000 680 / 483 us,
+// 100,000 on 1,000 117 / 98 us; on 1.31M triangles 262,144 0.54 / 1.10 ms, 1M
+// 1.99 / 0.90 ms.
+constexpr int64_t kRingRaysBelow = 65536, kRingRaysMost = 262144;
 
 // WindingNumberAntipodalScene.h:82-150: O no x 3, W no (device, FP64)
 void antipodal_query_device(const gwn_antipodal* a, const double* O, int64_t no, double* W, hipStream_t st) {
@@ -291,38 +404,45 @@ void antipodal_query_device(const gwn_antipodal* a, const double* O, int64_t no,
   }
   const gwn_soup* s = &a->soup;
   if (s->nf == 0 || s->nslots == 0) return;
+  const bool ring = no < kRingRaysBelow || no < std::min<int64_t>(2 * s->nf, kRingRaysMost);
   const size_t tb = radix_sort_temp_bytes(no, false);
-  Scratch ws(scratch_bytes({12 * (size_t)no, 4 * (size_t)no, 4 * (size_t)no, tb}), st);
-  float* Of = ws.take_n<float>(3 * (size_t)no);
-  uint32_t* keys = ws.take_n<uint32_t>((size_t)no);
-  uint32_t* perm = ws.take_n<uint32_t>((size_t)no);
-  void* tmp = ws.take(tb);
-  hipLaunchKernelGGL(k_ap_narrow, dim3(div_up(3 * no, 256)), dim3(256), 0, st, O, no, Of);
-  check_launch("k_ap_narrow");
-  hilbert_keys(Of, no, s->bbox, keys, perm, st);
-  radix_sort_u32(keys, perm, no, 30, tmp, tb, st);
+  Scratch ws(ring ? 1 : scratch_bytes({12 * (size_t)no, 4 * (size_t)no, 4 * (size_t)no, tb}), st);
+  RayFrame f;
+  for (int i = 0; i < 3; ++i)
+    for (int k = 0; k < 3; ++k) f.m[i][k] = a->frame[i][k];
+  f.reach = a->reach;
   Ray r;
   int kz = 0;
   for (int k = 1; k < 3; ++k)
     if (std::fabs(a->x0[k]) > std::fabs(a->x0[kz])) kz = k;
   int kx = (kz + 1) % 3, ky = (kx + 1) % 3;
   if (a->x0[kz] < 0.0) std::swap(kx, ky);  // keeps the winding of the projected triangle
-  for (int k = 0; k < 3; ++k) {
-    r.d[k] = a->x0[k];
-    r.inv[k] = a->x0[k] != 0.0 ? 1.0 / a->x0[k] : 0.0;
-  }
+  for (int k = 0; k < 3; ++k) r.d[k] = a->x0[k];
   r.kx = kx;
   r.ky = ky;
   r.kz = kz;
   r.sx = a->x0[kx] / a->x0[kz];
   r.sy = a->x0[ky] / a->x0[kz];
   r.sz = 1.0 / a->x0[kz];
-  {
+  if (ring) {
     ProfileScope prof("antipodal_crossings", st);
-    hipLaunchKernelGGL(k_ap_crossings, dim3(g), dim3(256), 0, st, s->dbox.p, (uint32_t)s->nslots, s->V64.p, s->F.p,
-                       O, perm, no, r, W);
-    check_launch("k_ap_crossings");
+    hipLaunchKernelGGL(k_ap_crossings_ring, dim3(div_up(no, 4)), dim3(256), 0, st, s->dbox.p, s->kids.p,
+                       (uint32_t)s->nslots, a->tri.p, O, no, r, f, W);
+    check_launch("k_ap_crossings_ring");
+    return;
   }
+  float* Of = ws.take_n<float>(3 * (size_t)no);
+  uint32_t* keys = ws.take_n<uint32_t>((size_t)no);
+  uint32_t* perm = ws.take_n<uint32_t>((size_t)no);
+  void* tmp = ws.take(tb);
+  hipLaunchKernelGGL(k_ap_plane, dim3(div_up(no, 256)), dim3(256), 0, st, O, no, f, Of);
+  check_launch("k_ap_plane");
+  hilbert_keys(Of, no, s->bbox, keys, perm, st);
+  radix_sort_u32(keys, perm, no, 30, tmp, tb, st);
+  ProfileScope prof("antipodal_crossings", st);
+  hipLaunchKernelGGL(k_ap_crossings, dim3(g), dim3(256), 0, st, s->dbox.p, (uint32_t)s->nslots, a->tri.p, O, perm, no,
+                     r, f, W);
+  check_launch("k_ap_crossings");
 }
 
 }  // namespace gwn

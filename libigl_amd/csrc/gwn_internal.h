@@ -300,6 +300,7 @@ struct gwn_soup {
   // bbox (records visited at accuracy scale 2, as a log-scale byte), built
   // with the tree: the wave walks start their costliest blocks first.
   gwn::DevBuf<uint8_t> cost_grid;
+  bool boxes_only = false;  // set before the build: no FP64 moments, no cost grid (not for queries)
   // After the build a handle is read-only to queries, except for dbox and the
   // pseudonormals, which the first query that needs them builds under
   // dist_mu / pn_mu (dist_ready / pn_ready set after).
@@ -324,10 +325,13 @@ struct gwn_curve {
   int64_t nslots = 0;
 };
 
-// Antipodal-method scene: the soup's triangles, tree and slot boxes for the
-// rays, and the weighted open-boundary segments.
+// Antipodal-method scene: the tree and slot boxes of the mesh turned into the
+// rays' frame, the triangles as given, and the weighted open-boundary segments.
 struct gwn_antipodal {
-  gwn_soup soup;
+  gwn_soup soup;            // over the turned vertices
+  gwn::DevBuf<double> tri;  // nf x 9: the faces' corners as given
+  double frame[3][3] = {};  // rows u, v, w (w along x0): turned = frame * vertex
+  double reach = 0.0;       // largest coordinate of V in magnitude
   gwn::DevBuf<double> seg;  // nseg x 8: a.xyz, b.xyz, w, 0
   int64_t nseg = 0;
   double x0[3] = {0, 0, 0};

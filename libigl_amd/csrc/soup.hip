@@ -1245,8 +1245,10 @@ void soup_finish_build(gwn_soup* s, hipStream_t st) {
   hipLaunchKernelGGL(k_write_slots, dim3(div_up(nn, 256)), dim3(256), 0, st, nn, s->nodes.p, s->boxdata.p, nsub.p,
                      first.p, total, s->slots.p, s->kids.p);
   check_launch("k_write_slots");
-  build_fp64_moments(s, L, st);
-  build_cost_grid(s, st);
+  if (!s->boxes_only) {
+    build_fp64_moments(s, L, st);
+    build_cost_grid(s, st);
+  }
   GWN_HIP(hipStreamSynchronize(st));
 }
 

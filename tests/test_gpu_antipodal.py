@@ -98,3 +98,28 @@ def test_large_mesh_and_edge_cases():
     # empty mesh and no queries
     assert np.all(gwn.winding_number_antipodal(V, F[:0], Q[:5]) == 0)
     assert gwn.WindingNumberAntipodalScene(V, F).winding_number(np.zeros((0, 3))).shape == (0,)
+
+
+@pytest.mark.parametrize("x0", [None, [0, 0, 1], [1, 1, 0], [-3, 1e-9, 2]])
+@pytest.mark.parametrize("shift,scale", [(0.0, 1.0), (1e4, 1.0), (-3.0, 1e-6)])
+def test_turned_boxes_and_both_walks(x0, shift, scale):
+    """The rays' boxes lie in a frame turned so that its w axis is x0 and are
+    widened by more than the turn's roundings, also far from the origin: counts
+    equal the exact winding number of a closed mesh on either side of 65,536
+    rays (one wavefront a ray below, 64 rays a wavefront from there), bit for
+    bit the same.  A NaN or infinite origin disturbs no other."""
+    V, F = D.bumpy_sphere(3, 8, 77)
+    rng = np.random.default_rng(77)
+    Q = np.concatenate([rng.uniform(-1.4, 1.4, (60_000, 3)), D.near_surface_queries(V, F, 6_000, 1e-3, rng)])
+    exact = np.round(gwn.winding_number_bruteforce(V, F, Q))
+    s = gwn.WindingNumberAntipodalScene(V * scale + shift, F, None if x0 is None else np.asarray(x0, float))
+    Qs = Q * scale + shift
+    Qs[[3, 40_000]] = np.nan
+    Qs[50_000, 1] = np.inf
+    keep = np.setdiff1d(np.arange(Q.shape[0]), [3, 40_000, 50_000])
+    W = s.winding_number(Qs)
+    assert np.abs(W[keep] - exact[keep]).max() < 1e-9
+    for part in (slice(0, 1), slice(0, 65_535), slice(0, 65_536)):
+        k = keep[(keep >= part.start) & (keep < part.stop)]
+        assert np.array_equal(s.winding_number(Qs[part])[k - part.start], W[k])
+    assert W[50_000] == 0.0
