@@ -396,7 +396,7 @@ int gwn_soup_get_info(const gwn_soup* s, gwn_soup_info* info) {
     info->depth = s->depth;
     info->device_bytes = (int64_t)(s->U.bytes() + s->F.bytes() + s->tri.bytes() + s->boxes.bytes() +
                                    s->nodes.bytes() + s->boxdata.bytes() + s->slots.bytes() + s->slots64.bytes() +
-                                   s->kids.bytes() + s->V64.bytes() + s->dbox.bytes());
+                                   s->kids.bytes() + s->V64.bytes() + s->dbox.bytes() + s->planes.bytes());
     std::memcpy(info->bbox, s->bbox, sizeof(s->bbox));
   });
 }

@@ -292,6 +292,8 @@ struct gwn_soup {
   gwn::DevBuf<double> slots64;  // nslots x 24 (FP64 moments), built with the tree
   gwn::DevBuf<double> V64;      // nv x 3, the vertices as given (closest-point queries)
   gwn::DevBuf<float4> dbox;     // nslots x 2 slot boxes for closest-point queries, built on first use
+  gwn::DevBuf<float4> planes;   // nf x 4: plane and edge planes of each face about `centre` (k_face_planes), with dbox
+  float centre[3] = {0, 0, 0};
   // pseudonormal sign: face normals nf x 3, angle-weighted vertex normals
   // nv x 3, edge normals per face and corner nf x 3 x 3; built on first use
   gwn::DevBuf<double> pn_face, pn_vertex, pn_edge;

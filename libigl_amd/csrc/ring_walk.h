@@ -1,15 +1,10 @@
 // ring_walk.h -- one query's walk of a rope-ordered tree shared by the 64
-// lanes of a wavefront: by ranges of siblings (ring_walk), or by nodes whose
-// children's positions are known (frontier_walk).
+// lanes of a wavefront (frontier_walk).
 //
 // A sequential walk is a chain of dependent record fetches as long as the
-// query's path.  In ring_walk the wavefront keeps a ring of pending (first record,
-// end) ranges of sibling records in LDS; each round every lane takes one
-// range, evaluates its first record, and pushes the record's child range
-// [i+1, link) if the walk descends there and the rest of the range (from i+1
-// after a leaf, from link after an internal record) if not empty, so a round
-// needs no fetch beyond the record itself.  When the ring is full a lane walks
-// its ranges sequentially instead.  Every record the sequential walk would
+// query's path.  Here the wavefront keeps a ring of pending records in LDS;
+// each round every lane takes one, evaluates it and, if the walk descends
+// there, pushes the record's children.  Every record the sequential walk would
 // decide on is decided on here too, each by one lane.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -18,7 +13,6 @@
 
 namespace gwn {
 
-constexpr int kReevalRing = 512;            // ranges per wavefront (4 KiB of LDS)
 constexpr uint32_t kRopeLeaf = 0x80000000u;  // link word of a leaf record
 
 __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
@@ -32,65 +26,11 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The ring walk of one query by the calling wavefront (ring: its kReevalRing
-// entries of LDS).  visit(i, link) evaluates record i for the query, adds its
-// term (if any) to the lane's own partial sums, sets link to the record's link
-// word and returns false when the walk descends into the record.
-template <typename Visit>
-__device__ __forceinline__ void ring_walk(uint2* __restrict__ ring, int lane, uint32_t nslots, Visit&& visit) {
-  if (lane == 0) ring[0] = make_uint2(0u, nslots);
-  uint32_t head = 0, tail = 1;  // wave-uniform ring positions
-  wave_lds_sync();
-  while (head != tail) {
-    const uint32_t take = min(tail - head, 64u);
-    const bool have = (uint32_t)lane < take;
-    uint2 it = make_uint2(0u, 0u);
-    if (have) it = ring[(head + lane) % kReevalRing];
-    head += take;
-    uint2 push0 = make_uint2(0u, 0u), push1 = make_uint2(0u, 0u);
-    uint32_t np = 0;
-    if (have) {
-      const uint32_t i = it.x;
-      uint32_t link;
-      const bool done = visit(i, link);
-      const uint32_t next = (link & kRopeLeaf) ? i + 1 : link;
-      if (!done) push0 = make_uint2(i + 1, link), np = 1;  // child range
-      if (next < it.y) {
-        if (np) push1 = make_uint2(next, it.y);
-        else push0 = make_uint2(next, it.y);
-        ++np;
-      }
-    }
-    const uint64_t b0 = __ballot(np & 1u), b1 = __ballot(np >> 1);
-    const uint32_t below = lanes_below(b0) + 2u * lanes_below(b1);
-    const uint32_t room = kReevalRing - (tail - head);
-    const bool fits = below + np <= room;
-    if (fits) {
-      if (np > 0) ring[(tail + below) % kReevalRing] = push0;
-      if (np > 1) ring[(tail + below + 1) % kReevalRing] = push1;
-    } else {
-      // ring full: walk the ranges sequentially (rope order)
-      for (uint32_t m = 0; m < np; ++m) {
-        const uint2 rg = m ? push1 : push0;
-        uint32_t i = rg.x;
-        while (i < rg.y) {
-          uint32_t link;
-          const bool done = visit(i, link);
-          i = (done && !(link & kRopeLeaf)) ? link : i + 1;
-        }
-      }
-    }
-    // lanes that fit are a prefix in lane order: their ranges are contiguous
-    tail += (uint32_t)__popcll(__ballot(fits && (np & 1u))) + 2u * (uint32_t)__popcll(__ballot(fits && (np >> 1)));
-    wave_lds_sync();
-  }
-}
-
-// The frontier walk: as ring_walk, but a node's children enter the ring
-// together (their positions in the rope are kept per record, kids), so a
-// query takes about as many rounds as the tree has levels, plus one per 64
-// records: 7.5 rounds where the ring walk took 21.4 (81,920 triangles,
-// accuracy_scale 2), 20.6 against 28.7 at 4.9.  Exact triangles go to a queue
+// A node's children enter the ring together (their positions in the rope are
+// kept per record, kids), so a query takes about as many rounds as the tree
+// has levels, plus one per 64 records: 7.5 rounds where pushing ranges of
+// siblings, one sibling a round, took 21.4 (81,920 triangles, accuracy_scale
+// 2), 20.6 against 28.7 at 4.9.  Exact triangles go to a queue
 // and are evaluated 64 at a time by the whole wavefront, where evaluating
 // each where it is met keeps the lanes that found none idle.
 constexpr int kFrontier = 1024;                // records per wavefront (4 KiB of LDS)
@@ -108,10 +48,10 @@ struct ExactQueue {
     if (mine) q[(head + n + lanes_below(m)) % kExactQueue] = t;
     n += (uint32_t)__popcll(m);
   }
-  // evaluates up to 64 of them, when there are as many or no more will come
-  template <typename Exact>
+  // evaluates up to 64 of them, when there are BATCH or no more will come
+  template <int BATCH, typename Exact>
   __device__ __forceinline__ void serve(uint32_t lane, bool last, Exact&& exact) {
-    if (n >= 64 || (last && n > 0)) {
+    if (n >= BATCH || (last && n > 0)) {
       const uint32_t cnt = min(n, 64u);
       if (lane < cnt) exact(q[(head + lane) % kExactQueue]);
       head += cnt;
@@ -131,7 +71,7 @@ struct ExactQueue {
 // kExact and kExactNear.  exact(t) and exact_near(t) add a
 // triangle to the calling lane's own sums; subtree(first, end) adds records
 // first .. end - 1, which a full ring has no room for.
-template <typename VisitFn, typename Exact, typename ExactNear, typename Subtree>
+template <int BATCH = 64, typename VisitFn, typename Exact, typename ExactNear, typename Subtree>
 __device__ __forceinline__ void frontier_walk(uint32_t* __restrict__ ring, uint32_t* __restrict__ q,
                                               uint32_t* __restrict__ qn, uint32_t lane,
                                               const uint4* __restrict__ kids, uint32_t nslots, VisitFn&& visit,
@@ -174,8 +114,8 @@ __device__ __forceinline__ void frontier_walk(uint32_t* __restrict__ ring, uint3
     near.push(what == Visit::kExactNear, t);
     wave_lds_sync();
     const bool last = head == tail;
-    far.serve(lane, last, exact);
-    near.serve(lane, last, exact_near);
+    far.serve<BATCH>(lane, last, exact);
+    near.serve<BATCH>(lane, last, exact_near);
     if (last && far.n + near.n == 0) break;
   }
 }

@@ -378,6 +378,45 @@ __global__ void k_write_dbox(int64_t nn, const uint32_t* __restrict__ nodes, con
   }
 }
 
+// Planes of a face for a lower bound of its distance (k_closest): the unit
+// normal's plane and, through each edge, the plane across the face with the
+// unit normal pointing out of it, as (n, d) with n.(p - centre) + d the signed
+// distance.  Zero where an edge or the normal has no direction, which bounds
+// nothing.
+__global__ void k_face_planes(const double* __restrict__ V, const int32_t* __restrict__ F, int64_t nf, float cx,
+                              float cy, float cz, float4* __restrict__ planes) {
+  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (f >= nf) return;
+  double v[3][3], n[3];
+  const double c[3] = {cx, cy, cz};
+  for (int k = 0; k < 3; ++k)
+    for (int a = 0; a < 3; ++a) v[k][a] = V[3 * (int64_t)F[3 * f + k] + a] - c[a];
+  const auto cross = [](const double* x, const double* y, double* z) {
+    for (int a = 0; a < 3; ++a) z[a] = x[(a + 1) % 3] * y[(a + 2) % 3] - x[(a + 2) % 3] * y[(a + 1) % 3];
+  };
+  const auto plane = [&](const double* dir, const double* at) {
+    const double l = sqrt(dir[0] * dir[0] + dir[1] * dir[1] + dir[2] * dir[2]);
+    if (!(l > 1e-150 && l < 1e150)) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const double u[3] = {dir[0] / l, dir[1] / l, dir[2] / l};
+    return make_float4((float)u[0], (float)u[1], (float)u[2], (float)-(u[0] * at[0] + u[1] * at[1] + u[2] * at[2]));
+  };
+  double e[3][3];
+  for (int k = 0; k < 3; ++k)
+    for (int a = 0; a < 3; ++a) e[k][a] = v[(k + 1) % 3][a] - v[k][a];
+  cross(e[0], e[1], n);
+  // a sliver's normal is mostly rounding: bound nothing with it
+  const double l0 = e[0][0] * e[0][0] + e[0][1] * e[0][1] + e[0][2] * e[0][2];
+  const double l1 = e[1][0] * e[1][0] + e[1][1] * e[1][1] + e[1][2] * e[1][2];
+  const double nn = n[0] * n[0] + n[1] * n[1] + n[2] * n[2];
+  const bool flat = nn > 1e-14 * l0 * l1;
+  planes[4 * f] = flat ? plane(n, v[0]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (int k = 0; k < 3; ++k) {
+    double out[3];
+    cross(e[k], n, out);
+    planes[4 * f + 1 + k] = flat ? plane(out, v[k]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // exact triangle solid angle: UTsignedSolidAngleTri (6070-6110)
 // (not inlined: the sums below call it for few terms)
@@ -1286,8 +1325,20 @@ void soup_ensure_dist(gwn_soup* s, hipStream_t st) {
   hipLaunchKernelGGL(k_write_dbox, dim3(div_up(nn, 256)), dim3(256), 0, st, nn, s->nodes.p, nbox.p, s->V64.p,
                      s->F.p, first.p, s->slots.p, db.p);
   check_launch("k_write_dbox");
+  DevBuf<float4> planes;
+  for (int k = 0; k < 3; ++k) {
+    const float c = 0.5f * s->bbox[k] + 0.5f * s->bbox[3 + k];
+    s->centre[k] = std::isfinite(c) ? c : 0.0f;
+  }
+  if (!s->boxes_only) {
+    planes.alloc(4 * (size_t)s->nf);
+    hipLaunchKernelGGL(k_face_planes, dim3(div_up(s->nf, 256)), dim3(256), 0, st, s->V64.p, s->F.p, s->nf,
+                       s->centre[0], s->centre[1], s->centre[2], planes.p);
+    check_launch("k_face_planes");
+  }
   GWN_HIP(hipStreamSynchronize(st));
   s->dbox = std::move(db);
+  s->planes = std::move(planes);
   s->dist_ready.store(true, std::memory_order_release);
 }
 

@@ -171,3 +171,47 @@ def test_signed_distance_large_batch():
     S1, I1, C1 = bvh.signed_distance(Q[12345:12346], gwn.SIGN_FAST_WINDING_NUMBER)
     assert I1[0] == I[12345] and np.array_equal(C1[0], C[12345])
     assert abs(S1[0] - S[12345]) <= 2e-5 * np.linalg.norm(C1[0] - Q[12345])
+
+
+@pytest.mark.parametrize("shift", [0.0, 1e4])
+def test_both_closest_point_walks_agree(shift):
+    """One wavefront a point below 131,072 points; from there 64 points a
+    wavefront, which hands over what takes it too long.  Same face, distance
+    and closest point bit for bit, for points deep inside (handed over), near
+    the surface, on vertices and edge midpoints (ties between faces), far away
+    and not finite, and with coordinates far larger than the mesh (the FP32
+    tests' allowances grow with them)."""
+    V, F, Q = D.soup_workload(nq=4000)
+    rng = np.random.default_rng(23)
+    d = rng.normal(size=(600, 3))
+    deep = d / np.linalg.norm(d, axis=1)[:, None] * rng.uniform(0, 0.3, (600, 1))
+    mids = 0.5 * (V[F[:300, 0]] + V[F[:300, 1]])
+    odd = np.array([[np.nan, 0, 0], [np.inf, 0, 0], [0, -np.inf, np.nan], [1e3, 0, 0], [0, 1e30, 0]])
+    P = np.concatenate([deep, Q, V[:300], mids, odd]) + shift
+    fill = rng.uniform(-1, 1, (131_072 - P.shape[0], 3)) * 0.4 + shift  # interior: many are handed over
+    bvh = gwn.FastWindingNumberBVH().build(V + shift, F, 2)
+    small = bvh.signed_distance(P, gwn.SIGN_UNSIGNED)
+    large = bvh.signed_distance(np.concatenate([P, fill]), gwn.SIGN_UNSIGNED)
+    for a, b in zip(small, large):
+        assert np.array_equal(a, b[:P.shape[0]], equal_nan=True)
+    sub = np.concatenate([np.arange(0, P.shape[0], 7), np.arange(P.shape[0] - 5, P.shape[0])])
+    So, Io, Co = O.signed_distance(V + shift, F, P[sub], gwn.SIGN_UNSIGNED)
+    ok = np.isfinite(So)
+    np.testing.assert_allclose(small[0][sub][ok], So[ok], rtol=1e-12, atol=1e-12 * (1 + shift))
+    assert np.array_equal(np.isfinite(small[0][sub]), ok)
+
+
+def test_closest_point_on_slivers_and_points():
+    """Faces without a plane (repeated vertices, collinear corners, slivers of
+    1e-9) among ordinary ones: their planes bound nothing, so they are found."""
+    rng = np.random.default_rng(31)
+    V = rng.uniform(-1, 1, (3000, 3))
+    F = rng.permutation(3000).reshape(-1, 3).astype(np.int32)
+    F[::5, 1] = F[::5, 0]                                   # a segment
+    F[::10, 2] = F[::10, 0]                                 # a point
+    V[F[1::5, 2]] = 0.5 * (V[F[1::5, 0]] + V[F[1::5, 1]])   # collinear
+    V[F[2::5, 2]] = V[F[2::5, 0]] + 1e-9 * rng.normal(size=V[F[2::5, 2]].shape)
+    P = np.concatenate([rng.uniform(-1.2, 1.2, (2000, 3)), V[F[:, 0]] + 1e-4])
+    S, I, C = gwn.signed_distance(P, V, F, gwn.SIGN_UNSIGNED)
+    So, Io, Co = O.signed_distance(V, F, P, gwn.SIGN_UNSIGNED)
+    np.testing.assert_allclose(S, So, rtol=1e-9, atol=1e-12)
