@@ -89,16 +89,38 @@ __device__ __forceinline__ int oct_lcp(uint64_t h0, uint64_t l0, uint64_t h1, ui
 }
 
 // lcp[a] for boundary a (between sorted points a and a+1), a in [0, n-1);
-// opens[a] = number of split cells whose first point is a.
-__global__ void k_oct_lcp(const uint64_t* __restrict__ hi, const uint64_t* __restrict__ lo, int64_t n,
-                          int32_t* __restrict__ lcp, uint32_t* __restrict__ opens) {
+// opens[a] = number of split cells whose first point is a.  They lie at the
+// depths prev+1 .. top, and point a is in a split cell down to the larger of
+// its two boundaries: `sizes` collects both by depth, as differences from one
+// depth to the next, so that the levels' cells and points are known before
+// the first level is split (a copy back per level took 2 ms of 32 ms at
+// 500,000 points).
+constexpr int OCT_SIZES = OCT_MAX_SPLIT_DEPTH + 2;
+__global__ __launch_bounds__(256) void k_oct_lcp(const uint64_t* __restrict__ hi, const uint64_t* __restrict__ lo,
+                                                 int64_t n, int32_t* __restrict__ lcp, uint32_t* __restrict__ opens,
+                                                 uint32_t* __restrict__ sizes) {
+  __shared__ uint32_t h[2 * OCT_SIZES];
+  for (int t = threadIdx.x; t < 2 * OCT_SIZES; t += 256) h[t] = 0;
+  __syncthreads();
   const int64_t a = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= n - 1) return;
-  const int cur = oct_lcp(hi[a], lo[a], hi[a + 1], lo[a + 1]);
-  const int prev = a == 0 ? -1 : oct_lcp(hi[a - 1], lo[a - 1], hi[a], lo[a]);
-  lcp[a] = cur;
-  const int top = cur < OCT_MAX_SPLIT_DEPTH ? cur : OCT_MAX_SPLIT_DEPTH;
-  opens[a] = top > prev ? (uint32_t)(top - prev) : 0u;
+  if (a < n) {
+    const int cur = a < n - 1 ? oct_lcp(hi[a], lo[a], hi[a + 1], lo[a + 1]) : -1;
+    const int prev = a == 0 ? -1 : oct_lcp(hi[a - 1], lo[a - 1], hi[a], lo[a]);
+    const int top = cur < OCT_MAX_SPLIT_DEPTH ? cur : OCT_MAX_SPLIT_DEPTH;
+    if (a < n - 1) {
+      lcp[a] = cur;
+      opens[a] = top > prev ? (uint32_t)(top - prev) : 0u;
+    }
+    if (top > prev) {
+      atomicAdd(&h[prev + 1], 1u);
+      atomicAdd(&h[top + 1], ~0u);
+    }
+    const int before = prev < OCT_MAX_SPLIT_DEPTH ? prev : OCT_MAX_SPLIT_DEPTH;
+    atomicAdd(&h[OCT_SIZES + 1 + (top > before ? top : before)], 1u);  // ends after that depth
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < 2 * OCT_SIZES; t += 256)
+    if (h[t]) atomicAdd(&sizes[t], h[t]);
 }
 
 __device__ __forceinline__ uint32_t oct_digit(const uint64_t* hi, const uint64_t* lo, int64_t k, int d) {
@@ -118,36 +140,62 @@ __device__ __forceinline__ uint32_t split_rank(const int32_t* lcp, const uint32_
   return open_scan[s] + (uint32_t)(d - prev - 1);
 }
 
-__global__ void k_oct_level(const SplitCell* __restrict__ cur, uint32_t ncur, const uint64_t* __restrict__ hi,
-                            const uint64_t* __restrict__ lo, const int32_t* __restrict__ lcp,
-                            const uint32_t* __restrict__ open_scan, int32_t* __restrict__ CH, float* __restrict__ CN,
-                            float* __restrict__ Wd, int64_t* __restrict__ cstart, int32_t* __restrict__ ccount,
-                            SplitCell* __restrict__ next, uint32_t* __restrict__ nnext, uint32_t next_cap,
-                            int64_t ncells, uint32_t* __restrict__ err) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= ncur) return;
-  const SplitCell sc = cur[t];
-  const float c0 = CN[3 * (int64_t)sc.cell], c1 = CN[3 * (int64_t)sc.cell + 1], c2 = CN[3 * (int64_t)sc.cell + 2];
-  const float h = Wd[sc.cell] / 2;
-  const float hh = h / 2;
-  int64_t s = sc.start;
-  for (uint32_t o = 0; o < 8; ++o) {
-    // first point of the range whose digit at this depth exceeds o
-    int64_t a = s, b = sc.end;
-    while (a < b) {
-      const int64_t m = (a + b) >> 1;
-      if (oct_digit(hi, lo, m, sc.depth) <= o)
-        a = m + 1;
-      else
-        b = m;
+// Eight lanes per split cell, one per child: each finds where its octant ends
+// (one thread that found the eight ends in turn took 106, 223 and 134 us on the
+// widest levels of 500,000 points, a chain of up to 8 x 19 dependent loads).
+// The children to split next are counted per block, so that the one counter
+// sees an atomic per 1,024 children: with one per wavefront it bound the
+// levels, 204 us on the widest, now 29.
+constexpr int OCT_THREADS = 1024;
+__global__ __launch_bounds__(OCT_THREADS) void k_oct_level(
+    const SplitCell* __restrict__ cur, const uint32_t* __restrict__ ncur, uint32_t most,
+    const uint64_t* __restrict__ hi, const uint64_t* __restrict__ lo, const int32_t* __restrict__ lcp,
+    const uint32_t* __restrict__ open_scan, int32_t* __restrict__ CH, float* __restrict__ CN, float* __restrict__ Wd,
+    int64_t* __restrict__ cstart, int32_t* __restrict__ ccount, SplitCell* __restrict__ next,
+    uint32_t* __restrict__ nnext, uint32_t next_cap, int64_t ncells, uint32_t* __restrict__ err) {
+  __shared__ uint32_t base[OCT_THREADS / 64];
+  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t o = (uint32_t)(t & 7);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  bool have = t / 8 < (*ncur < most ? *ncur : most);  // (whole groups of eight lanes)
+  SplitCell sc{};
+  if (have) sc = cur[t / 8];
+  // first point of the range whose digit at this depth exceeds o
+  int64_t a = sc.start, b = sc.end;
+  while (a < b) {
+    const int64_t m = (a + b) >> 1;
+    if (oct_digit(hi, lo, m, sc.depth) <= o)
+      a = m + 1;
+    else
+      b = m;
+  }
+  const int64_t e = a;
+  const int64_t before = __shfl_up(e, 1, 8);
+  const int64_t s = o == 0 ? sc.start : before;
+  const int64_t child64 = 1 + 8 * (int64_t)sc.rank + o;
+  if (have && child64 >= ncells) {  // inconsistent ranks: report, never write out of range
+    atomicOr(err, 1u);
+    have = false;
+  }
+  const int32_t child = (int32_t)child64;
+  const bool split = have && e - s >= 2 && sc.depth + 1 <= OCT_MAX_SPLIT_DEPTH;
+  const uint64_t splits = __ballot(split);
+  if (lane == 0) base[wave] = (uint32_t)__popcll(splits);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t sum = 0;
+    for (int w = 0; w < OCT_THREADS / 64; ++w) {
+      const uint32_t k = base[w];
+      base[w] = sum;
+      sum += k;
     }
-    const int64_t e = a;
-    const int64_t child64 = 1 + 8 * (int64_t)sc.rank + o;
-    if (child64 >= ncells) {  // inconsistent ranks: report, never write out of range
-      atomicOr(err, 1u);
-      return;
-    }
-    const int32_t child = (int32_t)child64;
+    const uint32_t at = sum ? atomicAdd(nnext, sum) : 0u;
+    for (int w = 0; w < OCT_THREADS / 64; ++w) base[w] += at;
+  }
+  if (have) {
+    const float c0 = CN[3 * (int64_t)sc.cell], c1 = CN[3 * (int64_t)sc.cell + 1], c2 = CN[3 * (int64_t)sc.cell + 2];
+    const float h = Wd[sc.cell] / 2;
+    const float hh = h / 2;
     CH[8 * (int64_t)sc.cell + o] = child;
     CN[3 * (int64_t)child] = c0 + ((o & 1) ? hh : -hh);
     CN[3 * (int64_t)child + 1] = c1 + ((o & 2) ? hh : -hh);
@@ -155,21 +203,21 @@ __global__ void k_oct_level(const SplitCell* __restrict__ cur, uint32_t ncur, co
     Wd[child] = h;
     cstart[child] = s;
     ccount[child] = (int32_t)(e - s);
-    if (e - s >= 2 && sc.depth + 1 <= OCT_MAX_SPLIT_DEPTH) {
-      SplitCell nc;
-      nc.cell = child;
-      nc.depth = sc.depth + 1;
-      nc.start = s;
-      nc.end = e;
-      nc.rank = split_rank(lcp, open_scan, s, sc.depth + 1);
-      nc.pad = 0;
-      const uint32_t slot = atomicAdd(nnext, 1u);
-      if (slot < next_cap)
-        next[slot] = nc;
-      else
-        atomicOr(err, 2u);
-    }
-    s = e;
+  }
+  __syncthreads();
+  if (split) {
+    SplitCell nc;
+    nc.cell = child;
+    nc.depth = sc.depth + 1;
+    nc.start = s;
+    nc.end = e;
+    nc.rank = split_rank(lcp, open_scan, s, sc.depth + 1);
+    nc.pad = 0;
+    const uint32_t slot = base[wave] + (uint32_t)__popcll(splits & ((1ull << lane) - 1));
+    if (slot < next_cap)
+      next[slot] = nc;
+    else
+      atomicOr(err, 2u);
   }
 }
 
@@ -200,30 +248,60 @@ __global__ void k_permute_points(const float* __restrict__ P, const float* __res
 // ---------------- precompute ----------------
 // Centre of mass of split cells, summed as the reference sums it: FP32,
 // sequentially, over the cell's points in ascending index order
-// (fast_winding_number.cpp:60-73).  Per level, the (cell, point) pairs are
-// sorted by (cell ordinal, point index), the terms are laid out in that
-// order, and each cell's four sums are folded in it: a wavefront per cell on
-// levels of few (large) cells, a thread per cell on levels of many.
-// Block (j, y): cell j's pairs y * 64 + lane, stepping by gridDim.y * 64, so
-// that a level of few large cells still spreads over many blocks.
-__global__ void k_lvl_emit(const SplitCell* __restrict__ lvl, const uint32_t* __restrict__ off,
-                           const int32_t* __restrict__ perm, uint64_t* __restrict__ keys) {
+// (fast_winding_number.cpp:60-73).  Per level, the points in index order take
+// their cell's ordinal as key and are sorted by it, stably, so that each
+// cell's points follow one another in index order; the terms are laid out in
+// that order, and each cell's four sums are folded in it: a wavefront per cell
+// on levels of few (large) cells, a thread per cell on levels of many.
+// Sorting 32-bit ordinals takes one to three passes a level; sorting
+// (ordinal, index) as one 64-bit key out of octree order took five to seven,
+// 5.7 ms of launches, gaps and copies at 500,000 points.
+//
+// Block (j, y): cell j's points y * 64 + lane, stepping by gridDim.y * 64, so
+// that a level of few large cells still spreads over many blocks.  cell_of[i]
+// becomes the split cell of point i, counted over all levels: points in no
+// split cell of this level keep an earlier level's.
+__global__ void k_lvl_mark(const SplitCell* __restrict__ lvl, uint32_t base, const int32_t* __restrict__ perm,
+                           uint32_t* __restrict__ cell_of) {
   const uint32_t j = blockIdx.x;
   const SplitCell sc = lvl[j];
   const int64_t cnt = sc.end - sc.start;
-  const uint32_t o = off[j];
   const int64_t step = (int64_t)gridDim.y * blockDim.x;
   for (int64_t t = (int64_t)blockIdx.y * blockDim.x + threadIdx.x; t < cnt; t += step)
-    keys[o + t] = ((uint64_t)j << 32) | (uint32_t)perm[sc.start + t];
+    cell_of[perm[sc.start + t]] = base + j;
 }
 
-// The terms the reference adds for a cell, in key order: a, a*x, a*y, a*z
+// Entry k of the point list (all points where `list` is null): its ordinal in
+// the level, m for a point that is in none of the level's cells.
+__global__ void k_lvl_keys(const uint32_t* __restrict__ list, int64_t count, const uint32_t* __restrict__ cell_of,
+                           uint32_t base, uint32_t m, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= count) return;
+  const uint32_t i = list ? list[k] : (uint32_t)k;
+  const uint32_t v = cell_of[i];
+  keys[k] = v >= base ? v - base : m;
+  vals[k] = i;
+}
+
+// the list without the points that are in none of the level's cells
+__global__ void k_lvl_flags(const uint32_t* __restrict__ list, int64_t count, const uint32_t* __restrict__ cell_of,
+                            uint32_t base, uint32_t* __restrict__ flags) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < count) flags[k] = cell_of[list ? list[k] : (uint32_t)k] >= base ? 1u : 0u;
+}
+__global__ void k_lvl_compact(const uint32_t* __restrict__ list, int64_t count, const uint32_t* __restrict__ flags,
+                              const uint32_t* __restrict__ pos, uint32_t* __restrict__ out) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < count && flags[k]) out[pos[k]] = list ? list[k] : (uint32_t)k;
+}
+
+// The terms the reference adds for a cell, in sorted order: a, a*x, a*y, a*z
 // (FP32 products, fast_winding_number.cpp:64-66).
-__global__ void k_lvl_terms(int64_t T, const uint64_t* __restrict__ keys, const float* __restrict__ P,
+__global__ void k_lvl_terms(int64_t T, const uint32_t* __restrict__ order, const float* __restrict__ P,
                             const float* __restrict__ A, float4* __restrict__ terms) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= T) return;
-  const int64_t i = (int64_t)(keys[t] & 0xFFFFFFFFull);
+  const int64_t i = order[t];
   const float a = A[i];
   terms[t] = make_float4(a, a * P[3 * i], a * P[3 * i + 1], a * P[3 * i + 2]);
 }
@@ -235,7 +313,7 @@ __global__ void k_lvl_fold(const SplitCell* __restrict__ lvl, uint32_t ncell, co
   if (j >= ncell) return;
   const SplitCell sc = lvl[j];
   const int64_t cnt = sc.end - sc.start;
-  const float4* v = terms + off[j];
+  const float4* v = terms + (off[j] - off[0]);  // (the offsets run over all levels, modulo 2^32)
   float at = 0.0f, m0 = 0.0f, m1 = 0.0f, m2 = 0.0f;
   for (int64_t t = 0; t < cnt; ++t) {
     const float4 q = v[t];
@@ -250,69 +328,83 @@ __global__ void k_lvl_fold(const SplitCell* __restrict__ lvl, uint32_t ncell, co
 }
 
 constexpr int FOLD_CHUNK = 512;   // terms staged in LDS per round
-constexpr int FOLD_GROUP = 16;    // float4 LDS reads in flight per lane
+constexpr int FOLD_GROUP = 16;    // float4 LDS reads of one group: 64 terms
+constexpr int FOLD_ROW = FOLD_CHUNK + 4;  // the four sums' rows start four banks apart
 
-// s + b[0] + b[1] + ... + b[n-1], added in that order (FP32).  The lane reads
-// 64 of its terms from LDS before adding them, so the LDS latency is paid
-// once per 64 dependent adds, not once per 4.
-__device__ __forceinline__ float fold_in_order(const float* b, int n, float s) {
-  const float4* b4 = reinterpret_cast<const float4*>(b);
-  const int n4 = n >> 2;
-  int g = 0;
-  for (; g + FOLD_GROUP <= n4; g += FOLD_GROUP) {
-    float4 q[FOLD_GROUP];
+__device__ __forceinline__ void fold_read(const float4* b4, float4 (&q)[FOLD_GROUP]) {
 #pragma unroll
-    for (int k = 0; k < FOLD_GROUP; ++k) q[k] = b4[g + k];
+  for (int k = 0; k < FOLD_GROUP; ++k) q[k] = b4[k];
+}
+__device__ __forceinline__ float fold_add(const float4 (&q)[FOLD_GROUP], float s) {
 #pragma unroll
-    for (int k = 0; k < FOLD_GROUP; ++k) {
-      s += q[k].x;
-      s += q[k].y;
-      s += q[k].z;
-      s += q[k].w;
-    }
+  for (int k = 0; k < FOLD_GROUP; ++k) {
+    s += q[k].x;
+    s += q[k].y;
+    s += q[k].z;
+    s += q[k].w;
   }
-  for (int e = 4 * g; e < n; ++e) s += b[e];
   return s;
 }
 
-// One wavefront per cell (levels of few, large cells).  The lanes stage
-// FOLD_CHUNK terms at a time in LDS, the next FOLD_CHUNK already in flight,
-// and lanes 0-3 each fold one of the four running sums in order: the same
-// sequential FP32 sums, one add per term and lane.
-__global__ __launch_bounds__(64) void k_lvl_fold_wave(const SplitCell* __restrict__ lvl,
-                                                      const uint32_t* __restrict__ off,
-                                                      const float4* __restrict__ terms, float* __restrict__ CM) {
-  __shared__ __align__(16) float buf[4][FOLD_CHUNK];
-  const SplitCell sc = lvl[blockIdx.x];
-  const int64_t cnt = sc.end - sc.start;
-  const float4* v = terms + off[blockIdx.x];
-  const int lane = threadIdx.x;
+// A cell's four sums a, a*x, a*y, a*z over its `cnt` terms, each in order in
+// FP32; lane l returns the sum of its row l & 3.  term(e) gives term e < cnt.
+// The lanes stage FOLD_CHUNK terms at a time in LDS, the next FOLD_CHUNK
+// already in flight, and every lane folds its row.  What remains is the chain
+// of dependent adds: each group of 64 terms is read from LDS while the one
+// before it is added (without that the LDS latency stood between groups: a
+// root of 500,000 points took 3.75 ms, now 1.80 ms, 3.6 ns an add).  Terms past the end are
+// -0, which leaves any sum as it is, so groups are always whole.
+template <typename Term>
+__device__ __forceinline__ float fold_cell(float (&buf)[4][FOLD_ROW], int64_t cnt, int lane, Term&& term) {
   constexpr int PER = FOLD_CHUNK / 64;
   float4 r[PER];
+  auto fetch = [&](int64_t base) {
 #pragma unroll
-  for (int u = 0; u < PER; ++u)
-    if (lane + 64 * u < cnt) r[u] = v[lane + 64 * u];
+    for (int u = 0; u < PER; ++u) {
+      const int64_t e = base + lane + 64 * u;
+      r[u] = make_float4(-0.0f, -0.0f, -0.0f, -0.0f);
+      if (e < cnt) r[u] = term(e);
+    }
+  };
+  fetch(0);
   float s = 0.0f;
+  const float4* b4 = reinterpret_cast<const float4*>(buf[lane & 3]);
   for (int64_t base = 0; base < cnt; base += FOLD_CHUNK) {
     const int n = (int)(cnt - base < FOLD_CHUNK ? cnt - base : FOLD_CHUNK);
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
       const int e = lane + 64 * u;
-      if (e < n) {
-        buf[0][e] = r[u].x;
-        buf[1][e] = r[u].y;
-        buf[2][e] = r[u].z;
-        buf[3][e] = r[u].w;
-      }
+      buf[0][e] = r[u].x;
+      buf[1][e] = r[u].y;
+      buf[2][e] = r[u].z;
+      buf[3][e] = r[u].w;
     }
     __syncthreads();
-    const int64_t nb = base + FOLD_CHUNK;
-#pragma unroll
-    for (int u = 0; u < PER; ++u)
-      if (nb + lane + 64 * u < cnt) r[u] = v[nb + lane + 64 * u];
-    if (lane < 4) s = fold_in_order(buf[lane], n, s);
+    if (base + FOLD_CHUNK < cnt) fetch(base + FOLD_CHUNK);
+    const int groups = (n + 63) / 64;
+    float4 q0[FOLD_GROUP], q1[FOLD_GROUP];
+    fold_read(b4, q0);
+    for (int g = 0; g < groups; g += 2) {  // (a chunk holds an even number of groups)
+      fold_read(b4 + (g + 1) * FOLD_GROUP, q1);
+      s = fold_add(q0, s);
+      if (g + 1 == groups) break;
+      if (g + 2 < groups) fold_read(b4 + (g + 2) * FOLD_GROUP, q0);
+      s = fold_add(q1, s);
+    }
     __syncthreads();
   }
+  return s;
+}
+
+// One wavefront per cell (levels of few, large cells).
+__global__ __launch_bounds__(64) void k_lvl_fold_wave(const SplitCell* __restrict__ lvl,
+                                                      const uint32_t* __restrict__ off,
+                                                      const float4* __restrict__ terms, float* __restrict__ CM) {
+  __shared__ __align__(16) float buf[4][FOLD_ROW];
+  const SplitCell sc = lvl[blockIdx.x];
+  const float4* v = terms + (off[blockIdx.x] - off[0]);
+  const int lane = threadIdx.x;
+  const float s = fold_cell(buf, sc.end - sc.start, lane, [&](int64_t e) { return v[e]; });
   const float at = __shfl(s, 0);
   if (lane >= 1 && lane <= 3) CM[3 * (int64_t)sc.cell + lane - 1] = s / at;
 }
@@ -402,42 +494,16 @@ __global__ __launch_bounds__(64) void k_cm_fold_wave(const int32_t* __restrict__
                                                      const int32_t* __restrict__ ccount, const float* __restrict__ P,
                                                      const float* __restrict__ A, const int32_t* __restrict__ perm,
                                                      float* __restrict__ CM) {
-  __shared__ __align__(16) float buf[4][FOLD_CHUNK];
+  __shared__ __align__(16) float buf[4][FOLD_ROW];
   const int32_t c = cells[blockIdx.x];
   if (fold_cm && CH[8 * (int64_t)c] >= 0) return;  // uniform over the block
   const int64_t s0 = cstart[c];
-  const int64_t cnt = ccount[c];
   const int lane = threadIdx.x;
-  constexpr int PER = FOLD_CHUNK / 64;
-  float4 r[PER];
-  auto gather = [&](int64_t base) {
-#pragma unroll
-    for (int u = 0; u < PER; ++u)
-      if (base + lane + 64 * u < cnt) {
-        const int64_t p = perm[s0 + base + lane + 64 * u];
-        const float a = A[p];
-        r[u] = make_float4(a, a * P[3 * p], a * P[3 * p + 1], a * P[3 * p + 2]);
-      }
-  };
-  gather(0);
-  float s = 0.0f;
-  for (int64_t base = 0; base < cnt; base += FOLD_CHUNK) {
-    const int n = (int)(cnt - base < FOLD_CHUNK ? cnt - base : FOLD_CHUNK);
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int e = lane + 64 * u;
-      if (e < n) {
-        buf[0][e] = r[u].x;
-        buf[1][e] = r[u].y;
-        buf[2][e] = r[u].z;
-        buf[3][e] = r[u].w;
-      }
-    }
-    __syncthreads();
-    gather(base + FOLD_CHUNK);
-    if (lane < 4) s = fold_in_order(buf[lane], n, s);
-    __syncthreads();
-  }
+  const float s = fold_cell(buf, ccount[c], lane, [&](int64_t e) {
+    const int64_t p = perm[s0 + e];
+    const float a = A[p];
+    return make_float4(a, a * P[3 * p], a * P[3 * p + 1], a * P[3 * p + 2]);
+  });
   const float at = __shfl(s, 0);
   if (lane >= 1 && lane <= 3) CM[3 * (int64_t)c + lane - 1] = s / at;
 }
@@ -528,13 +594,24 @@ __global__ void k_large_counts(const int32_t* __restrict__ cells, uint32_t count
   if (t < count) out[t] = ccount[cells[t]];
 }
 
-__global__ void k_cell_empty(int64_t ncells, const int32_t* __restrict__ ccount, int nt, float* __restrict__ CM,
-                             float* __restrict__ R, float* __restrict__ EC) {
+// A wavefront takes 64 cells and writes the moments of the empty ones a cell
+// at a time (a thread per cell, 39 strided stores each, took 361 us at 500,000
+// points).
+__global__ __launch_bounds__(256) void k_cell_empty(int64_t ncells, const int32_t* __restrict__ ccount, int nt,
+                                                    float* __restrict__ CM, float* __restrict__ R,
+                                                    float* __restrict__ EC) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncells || ccount[c] > 0) return;
+  const int lane = threadIdx.x & 63;
+  const bool empty = c < ncells && ccount[c] <= 0;
+  uint64_t todo = __ballot(empty);
+  while (todo) {
+    const int j = __ffsll((unsigned long long)todo) - 1;
+    todo &= todo - 1;
+    if (lane < nt) EC[nt * (c - lane + j) + lane] = 0.0f;
+  }
+  if (!empty) return;
   for (int d = 0; d < 3; ++d) CM[3 * c + d] = __int_as_float(0x7FC00000);  // NaN, as the reference
   R[c] = 0.0f;
-  for (int k = 0; k < nt; ++k) EC[nt * c + k] = 0.0f;
 }
 
 // classify non-empty cells into small / large lists: flags, scans, scatter
@@ -815,8 +892,9 @@ __global__ __launch_bounds__(256) void k_cloud_brute(const float* __restrict__ P
 // octree take their centres from the per-level folds (their point lists are
 // ranges of the key order, the reference sums in ascending index order);
 // otherwise each cell sums its centre over its own list, in list order.
+// lvl_points: points in the split cells of each level (with fold_cm).
 static void cell_moments(gwn_cloud* c, bool fold_cm, const SplitCell* all, const std::vector<uint32_t>& lvl_off,
-                         hipStream_t st) {
+                         const std::vector<uint32_t>& lvl_points, hipStream_t st) {
   const int64_t ncells = c->ncells;
   const int nt = c->nterms;
   c->CM.alloc(3 * (size_t)ncells);
@@ -843,45 +921,62 @@ static void cell_moments(gwn_cloud* c, bool fold_cm, const SplitCell* all, const
                        c->R.p, c->EC.p);
     check_launch("k_cell_empty");
     // split-cell centres, level by level.  The work buffers are allocated
-    // once for the largest level: a level's cells are disjoint ranges of the
-    // points, so it has at most n (cell, point) pairs.
-    uint32_t maxm = 0;
-    for (size_t d = 0; d + 1 < lvl_off.size(); ++d) maxm = std::max(maxm, lvl_off[d + 1] - lvl_off[d]);
-    const bool any_level = fold_cm && maxm > 0;
-    const int64_t np = c->n;
-    DevBuf<uint32_t> cnt(any_level ? maxm : 0), off(any_level ? maxm : 0), tot(any_level ? 1 : 0);
-    DevBuf<uint8_t> sct(any_level ? scan_temp_bytes(maxm) : 0);
-    DevBuf<uint64_t> keys(any_level ? np : 0);
-    DevBuf<uint32_t> dummy(any_level ? np : 0);
-    DevBuf<float4> terms(any_level ? np : 0);
-    const size_t tb = any_level ? radix_sort_temp_bytes(np, true) : 0;
-    DevBuf<uint8_t> tmp(tb);
-    for (size_t d = 0; any_level && d + 1 < lvl_off.size(); ++d) {
-      const uint32_t b = lvl_off[d], e = lvl_off[d + 1];
-      if (e == b) continue;
-      const uint32_t m = e - b;
-      hipLaunchKernelGGL(k_split_counts, dim3(div_up(m, 256)), dim3(256), 0, st, all + b, m, cnt.p);
+    // once: a level's cells are disjoint ranges of the points, so it has at
+    // most n (cell, point) pairs.
+    const uint32_t nsplit = lvl_off.empty() ? 0 : lvl_off.back();
+    if (fold_cm && nsplit > 0) {
+      const int64_t np = c->n;
+      DevBuf<uint32_t> cnt(nsplit), off(nsplit), cell_of(np), keys(np), vals(np), list[2];
+      DevBuf<uint8_t> sct(scan_temp_bytes(std::max<int64_t>(nsplit, np)));
+      DevBuf<float4> terms(np);
+      const size_t tb = radix_sort_temp_bytes(np, false);
+      DevBuf<uint8_t> tmp(tb);
+      hipLaunchKernelGGL(k_split_counts, dim3(div_up(nsplit, 256)), dim3(256), 0, st, all, nsplit, cnt.p);
       check_launch("k_split_counts");
-      exclusive_scan_u32(cnt.p, off.p, m, tot.p, sct.p, st);
-      uint32_t T = 0;
-      GWN_HIP(hipMemcpyAsync(&T, tot.p, 4, hipMemcpyDeviceToHost, st));
-      GWN_HIP(hipStreamSynchronize(st));
-      GWN_CHECK((int64_t)T <= np, GWN_ERR_INVALID, "cloud build: a level holds more pairs than points");
-      const unsigned ysplit = m < 4096 ? (unsigned)div_up(4096, m) : 1u;
-      hipLaunchKernelGGL(k_lvl_emit, dim3(m, ysplit), dim3(64), 0, st, all + b, off.p, c->perm.p, keys.p);
-      check_launch("k_lvl_emit");
-      int obits = 1;
-      while ((1u << obits) < m) ++obits;
-      radix_sort_u64(keys.p, dummy.p, T, 32 + obits, tmp.p, tb, st);
-      hipLaunchKernelGGL(k_lvl_terms, dim3(div_up(T, 256)), dim3(256), 0, st, (int64_t)T, keys.p, c->P.p, c->A.p,
-                         terms.p);
-      check_launch("k_lvl_terms");
-      if (m <= 65536) {
-        hipLaunchKernelGGL(k_lvl_fold_wave, dim3(m), dim3(64), 0, st, all + b, off.p, terms.p, c->CM.p);
-        check_launch("k_lvl_fold_wave");
-      } else {
-        hipLaunchKernelGGL(k_lvl_fold, dim3(div_up(m, 64)), dim3(64), 0, st, all + b, m, off.p, terms.p, c->CM.p);
-        check_launch("k_lvl_fold");
+      exclusive_scan_u32(cnt.p, off.p, nsplit, nullptr, sct.p, st);
+      const uint32_t* active = nullptr;  // null: every point, in index order
+      int64_t nactive = np;
+      int spare = 0;
+      for (size_t d = 0; d + 1 < lvl_off.size(); ++d) {
+        const uint32_t b = lvl_off[d], e = lvl_off[d + 1];
+        if (e == b) continue;
+        const uint32_t m = e - b, T = lvl_points[d];
+        const unsigned ysplit = m < 4096 ? (unsigned)div_up(4096, m) : 1u;
+        hipLaunchKernelGGL(k_lvl_mark, dim3(m, ysplit), dim3(64), 0, st, all + b, b, c->perm.p, cell_of.p);
+        check_launch("k_lvl_mark");
+        // points once in no split cell are in none further down: the list is
+        // cut when half of it has gone (five launches, a few sorts' worth)
+        if (T <= nactive / 2) {
+          if (!list[spare].p) list[spare].alloc((size_t)T);
+          const unsigned ga = (unsigned)div_up(nactive, 256);
+          hipLaunchKernelGGL(k_lvl_flags, dim3(ga), dim3(256), 0, st, active, nactive, cell_of.p, b, keys.p);
+          check_launch("k_lvl_flags");
+          exclusive_scan_u32(keys.p, vals.p, nactive, nullptr, sct.p, st);
+          hipLaunchKernelGGL(k_lvl_compact, dim3(ga), dim3(256), 0, st, active, nactive, keys.p, vals.p,
+                             list[spare].p);
+          check_launch("k_lvl_compact");
+          active = list[spare].p;
+          nactive = T;
+          spare ^= 1;
+        }
+        hipLaunchKernelGGL(k_lvl_keys, dim3(div_up(nactive, 256)), dim3(256), 0, st, active, nactive, cell_of.p, b, m,
+                           keys.p, vals.p);
+        check_launch("k_lvl_keys");
+        const uint32_t most = T < nactive ? m : m - 1;
+        int bits = 0;
+        while (bits < 32 && (most >> bits) != 0) ++bits;
+        const uint32_t* order = radix_sort_u32_values(keys.p, vals.p, nactive, bits, tmp.p, tb, st);
+        hipLaunchKernelGGL(k_lvl_terms, dim3(div_up(T, 256)), dim3(256), 0, st, (int64_t)T, order, c->P.p, c->A.p,
+                           terms.p);
+        check_launch("k_lvl_terms");
+        if (m <= 65536) {
+          hipLaunchKernelGGL(k_lvl_fold_wave, dim3(m), dim3(64), 0, st, all + b, off.p + b, terms.p, c->CM.p);
+          check_launch("k_lvl_fold_wave");
+        } else {
+          hipLaunchKernelGGL(k_lvl_fold, dim3(div_up(m, 64)), dim3(64), 0, st, all + b, m, off.p + b, terms.p,
+                             c->CM.p);
+          check_launch("k_lvl_fold");
+        }
       }
       GWN_HIP(hipStreamSynchronize(st));
     }
@@ -1080,16 +1175,18 @@ void cloud_build_device(gwn_cloud* c, hipStream_t st, bool moments) {
     return;
   }
   // root cube: bbox centre and longest side (octree.cpp:139-150), in float
-  std::vector<float> hp(3 * (size_t)n);
-  GWN_HIP(hipMemcpyAsync(hp.data(), c->P.p, sizeof(float) * hp.size(), hipMemcpyDeviceToHost, st));
-  GWN_HIP(hipStreamSynchronize(st));
-  float mn[3] = {hp[0], hp[1], hp[2]}, mx[3] = {hp[0], hp[1], hp[2]};
-  for (int64_t i = 1; i < n; ++i)
-    for (int d = 0; d < 3; ++d) {
-      const float v = hp[3 * i + d];
-      if (v < mn[d]) mn[d] = v;
-      if (v > mx[d]) mx[d] = v;
-    }
+  // (on the card: the copy to the host and the loop there took 2.5 ms at
+  // 500,000 points)
+  float first[3], mn[3], mx[3], bb[6];
+  GWN_HIP(hipMemcpyAsync(first, c->P.p, sizeof(first), hipMemcpyDeviceToHost, st));
+  points_bbox(c->P.p, n, bb, st);
+  // minima and maxima that start from the first point: a NaN there stays, and
+  // where all are zeros its sign does
+  for (int d = 0; d < 3; ++d) {
+    const bool keep = std::isnan(first[d]) || bb[d] == bb[3 + d];
+    mn[d] = keep ? first[d] : bb[d];
+    mx[d] = keep ? first[d] : bb[3 + d];
+  }
   float ctr[3];
   for (int d = 0; d < 3; ++d) ctr[d] = (mn[d] + mx[d]) / 2.0f;
   float w0 = mx[0] - mn[0];
@@ -1131,14 +1228,16 @@ void cloud_build_device(gwn_cloud* c, hipStream_t st, bool moments) {
   // split-cell ranks
   const int64_t nb = n - 1;
   DevBuf<int32_t> lcp(nb > 0 ? nb : 1);
-  DevBuf<uint32_t> opens(nb > 0 ? nb : 1), oscan(nb > 0 ? nb : 1), total(1);
-  uint32_t S = 0;
+  DevBuf<uint32_t> opens(nb > 0 ? nb : 1), oscan(nb > 0 ? nb : 1), total(1), sizes(2 * OCT_SIZES);
+  uint32_t S = 0, hsizes[2 * OCT_SIZES];
   if (nb > 0) {
-    hipLaunchKernelGGL(k_oct_lcp, dim3(div_up(nb, 256)), dim3(256), 0, st, HS, LS, n, lcp.p, opens.p);
+    GWN_HIP(hipMemsetAsync(sizes.p, 0, sizeof(hsizes), st));
+    hipLaunchKernelGGL(k_oct_lcp, dim3(g), dim3(256), 0, st, HS, LS, n, lcp.p, opens.p, sizes.p);
     check_launch("k_oct_lcp");
     DevBuf<uint8_t> sc(scan_temp_bytes(nb));
     exclusive_scan_u32(opens.p, oscan.p, nb, total.p, sc.p, st);
     GWN_HIP(hipMemcpyAsync(&S, total.p, 4, hipMemcpyDeviceToHost, st));
+    GWN_HIP(hipMemcpyAsync(hsizes, sizes.p, sizeof(hsizes), hipMemcpyDeviceToHost, st));
     GWN_HIP(hipStreamSynchronize(st));
   }
   const int64_t ncells = 1 + 8 * (int64_t)S;
@@ -1160,31 +1259,39 @@ void cloud_build_device(gwn_cloud* c, hipStream_t st, bool moments) {
   }
   // level-synchronous split; all split cells kept, level by level
   DevBuf<SplitCell> all(S > 0 ? S : 1);
-  DevBuf<uint32_t> cntd(1), errd(1);
-  GWN_HIP(hipMemsetAsync(errd.p, 0, 4, st));
-  std::vector<uint32_t> lvl_off{0};
+  std::vector<uint32_t> lvl_off{0}, lvl_points;
   if (S > 0) {
-    SplitCell root{0, 0, 0, n, 0, 0};
-    GWN_HIP(hipMemcpyAsync(all.p, &root, sizeof(root), hipMemcpyHostToDevice, st));
-    lvl_off.push_back(1);
+    // levels' cells and points from their differences by depth
+    uint32_t cells = 0, points = (uint32_t)n;
     for (int d = 0; d <= OCT_MAX_SPLIT_DEPTH; ++d) {
-      const uint32_t b = lvl_off[d], e = lvl_off[d + 1];
-      if (e == b) break;
-      GWN_CHECK(e <= S, GWN_ERR_INVALID, "octree split count mismatch");
-      GWN_HIP(hipMemsetAsync(cntd.p, 0, 4, st));
-      hipLaunchKernelGGL(k_oct_level, dim3(div_up(e - b, 128)), dim3(128), 0, st, all.p + b, e - b, HS, LS, lcp.p,
-                         oscan.p, c->CH.p, c->CN.p, c->Wd.p, c->cstart.p, c->ccount.p, all.p + e, cntd.p, S - e,
-                         ncells, errd.p);
-      check_launch("k_oct_level");
-      uint32_t nn = 0, ef = 0;
-      GWN_HIP(hipMemcpyAsync(&nn, cntd.p, 4, hipMemcpyDeviceToHost, st));
-      GWN_HIP(hipMemcpyAsync(&ef, errd.p, 4, hipMemcpyDeviceToHost, st));
-      GWN_HIP(hipStreamSynchronize(st));
-      GWN_CHECK(ef == 0, GWN_ERR_INVALID, "octree build: split ranks out of range");
-      GWN_CHECK(e + nn <= S, GWN_ERR_INVALID, "octree split count mismatch");
-      lvl_off.push_back(e + nn);
+      cells += hsizes[d];
+      points -= hsizes[OCT_SIZES + d];
+      if (cells == 0) break;
+      lvl_off.push_back(lvl_off.back() + cells);
+      lvl_points.push_back(points);
     }
     GWN_CHECK(lvl_off.back() == S, GWN_ERR_INVALID, "octree split cells != scan total");
+    const size_t nlev = lvl_points.size();
+    DevBuf<uint32_t> made(nlev + 2);  // cells made at each level, and the error word
+    GWN_HIP(hipMemsetAsync(made.p, 0, 4 * (nlev + 2), st));
+    SplitCell root{0, 0, 0, n, 0, 0};
+    const uint32_t one = 1;
+    GWN_HIP(hipMemcpyAsync(all.p, &root, sizeof(root), hipMemcpyHostToDevice, st));
+    GWN_HIP(hipMemcpyAsync(made.p, &one, 4, hipMemcpyHostToDevice, st));
+    for (size_t d = 0; d < nlev; ++d) {
+      const uint32_t b = lvl_off[d], e = lvl_off[d + 1];
+      hipLaunchKernelGGL(k_oct_level, dim3(div_up(8 * (int64_t)(e - b), OCT_THREADS)), dim3(OCT_THREADS), 0, st, all.p + b, made.p + d, e - b,
+                         HS, LS, lcp.p, oscan.p, c->CH.p, c->CN.p, c->Wd.p, c->cstart.p, c->ccount.p, all.p + e,
+                         made.p + d + 1, S - e, ncells, made.p + nlev + 1);
+    }
+    check_launch("k_oct_level");
+    std::vector<uint32_t> hm(nlev + 2);
+    GWN_HIP(hipMemcpyAsync(hm.data(), made.p, 4 * hm.size(), hipMemcpyDeviceToHost, st));
+    GWN_HIP(hipStreamSynchronize(st));
+    GWN_CHECK(hm[nlev + 1] == 0, GWN_ERR_INVALID, "octree build: split ranks out of range");
+    for (size_t d = 0; d < nlev; ++d)
+      GWN_CHECK(hm[d] == lvl_off[d + 1] - lvl_off[d], GWN_ERR_INVALID, "octree split count mismatch");
+    GWN_CHECK(hm[nlev] == 0, GWN_ERR_INVALID, "octree split count mismatch");
   }
 
   c->root_leaf = S == 0;
@@ -1195,7 +1302,7 @@ void cloud_build_device(gwn_cloud* c, hipStream_t st, bool moments) {
     GWN_HIP(hipStreamSynchronize(st));
     return;
   }
-  cell_moments(c, true, all.p, lvl_off, st);
+  cell_moments(c, true, all.p, lvl_off, lvl_points, st);
   rope_records(c, all.p, lvl_off, c->cstart.p, st);
   build_cloud_cost_grid(c, st);
   GWN_HIP(hipStreamSynchronize(st));
@@ -1315,7 +1422,7 @@ void cloud_build_from_octree_device(gwn_cloud* c, const int32_t* hCH, int64_t nc
     GWN_HIP(hipMemcpyAsync(c->EC.p, hEC, 4 * (size_t)c->nterms * ncells, hipMemcpyHostToDevice, st));
   } else {
     GWN_CHECK(!hCM && !hR && !hEC, GWN_ERR_INVALID, "give all of CM, R, EC or none");
-    cell_moments(c, false, all.p, lvl_off, st);
+    cell_moments(c, false, all.p, lvl_off, {}, st);
   }
   DevBuf<int64_t> dls(ncells);
   GWN_HIP(hipMemcpyAsync(dls.p, lstart.data(), 8 * (size_t)ncells, hipMemcpyHostToDevice, st));

@@ -185,6 +185,12 @@ void sah4_build(const float* boxes, uint32_t nboxes, std::vector<uint32_t>& node
 size_t radix_sort_temp_bytes(int64_t n, bool key64);
 void radix_sort_u32(uint32_t* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes,
                     hipStream_t st);
+// sorts by the low `bits` of the keys (none: as they are) and returns where
+// the values lie then, in `vals` or in `tmp`; the keys are not kept
+const uint32_t* radix_sort_u32_values(uint32_t* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes,
+                                      hipStream_t st);
+// min and max of n points' coordinates (bb: 3 + 3), NaN left out
+void points_bbox(const float* P, int64_t n, float* bb, hipStream_t st);
 void radix_sort_u64(uint64_t* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes,
                     hipStream_t st);
 

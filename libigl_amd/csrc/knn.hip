@@ -751,7 +751,7 @@ struct KnnTree {
   DevBuf<float4> rec;
 };
 
-static void knn_bbox(const float* Cf, int64_t n, float* bb, hipStream_t st) {
+void points_bbox(const float* Cf, int64_t n, float* bb, hipStream_t st) {
   const int g = (int)std::min<int64_t>(1024, std::max<int64_t>(1, div_up(n, 256)));
   DevBuf<float> part(6 * (size_t)g);
   hipLaunchKernelGGL(k_kn_bbox, dim3(g), dim3(256), 0, st, Cf, n, part.p);
@@ -782,7 +782,7 @@ static void knn_build(const double* V, int64_t nv, const int32_t* cand, int64_t 
   GWN_HIP(hipStreamSynchronize(st));
   GWN_CHECK(nbad[1] == 0, GWN_ERR_INVALID, "knn: a candidate index lies outside V");
   GWN_CHECK(nbad[0] == 0, GWN_ERR_INVALID, "knn: points must be finite");
-  knn_bbox(Cf.p, nc, T.bbox, st);
+  points_bbox(Cf.p, nc, T.bbox, st);
   DevBuf<uint32_t> order(nc);
   T.codes.alloc((size_t)nc);
   morton_keys(Cf.p, nc, T.bbox, T.codes.p, order.p, st);
@@ -914,7 +914,7 @@ void point_areas_device(const double* P, int64_t n, const int32_t* I, int64_t k,
     hipLaunchKernelGGL(k_kn_narrow, dim3(div_up(3 * n, 256)), dim3(256), 0, st, P, n, Pf.p, bad.p);
     check_launch("k_kn_narrow");
     float bb[6];
-    knn_bbox(Pf.p, n, bb, st);
+    points_bbox(Pf.p, n, bb, st);
     morton_keys(Pf.p, n, bb, keys.p, order.p, st);
     const size_t tb = radix_sort_temp_bytes(n, false);
     DevBuf<uint8_t> tmp(tb);

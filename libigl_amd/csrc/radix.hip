@@ -260,9 +260,11 @@ size_t radix_sort_temp_bytes(int64_t n, bool key64) {
          align256(4 * 256);
 }
 
+// Returns the sorted values, in `vals` or (after an odd number of passes) in
+// `tmp`; with `in_place` keys and values are copied back instead.
 template <typename K>
-static void radix_sort(K* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes, hipStream_t st) {
-  if (n <= 1) return;
+static const uint32_t* radix_sort(bool in_place, K* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes, hipStream_t st) {
+  if (n <= 1) return vals;
   GWN_CHECK(tmp_bytes >= radix_sort_temp_bytes(n, sizeof(K) == 8), GWN_ERR_INVALID, "radix sort temp too small");
   GWN_CHECK(n < ((int64_t)1 << 32), GWN_ERR_INVALID, "radix sort: more than 2^32 - 1 keys");
   const int64_t nt = div_up(n, RS_TILE);
@@ -291,19 +293,25 @@ static void radix_sort(K* keys, uint32_t* vals, int64_t n, int bits, void* tmp, 
     std::swap(va, vb);
     ++passes;
   }
-  if (passes & 1) {
+  if (in_place && (passes & 1)) {
     GWN_HIP(hipMemcpyAsync(keys, ka, sizeof(K) * (size_t)n, hipMemcpyDeviceToDevice, st));
     GWN_HIP(hipMemcpyAsync(vals, va, sizeof(uint32_t) * (size_t)n, hipMemcpyDeviceToDevice, st));
+    return vals;
   }
+  return va;
 }
 
 void radix_sort_u32(uint32_t* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes,
                     hipStream_t st) {
-  radix_sort<uint32_t>(keys, vals, n, bits, tmp, tmp_bytes, st);
+  radix_sort<uint32_t>(true, keys, vals, n, bits, tmp, tmp_bytes, st);
+}
+const uint32_t* radix_sort_u32_values(uint32_t* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes,
+                                      hipStream_t st) {
+  return radix_sort<uint32_t>(false, keys, vals, n, bits, tmp, tmp_bytes, st);
 }
 void radix_sort_u64(uint64_t* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes,
                     hipStream_t st) {
-  radix_sort<uint64_t>(keys, vals, n, bits, tmp, tmp_bytes, st);
+  radix_sort<uint64_t>(true, keys, vals, n, bits, tmp, tmp_bytes, st);
 }
 
 }  // namespace gwn

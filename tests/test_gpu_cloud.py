@@ -279,3 +279,54 @@ def test_far_test_by_squares(radius, beta):
     assert ok.sum() > 500
     d = np.abs(W - Wo)[ok] / np.maximum(1.0, np.abs(Wo[ok]))
     assert (d <= 2e-4).all(), (d.max(), int((d > 2e-4).sum()))
+
+
+def _clusters(sizes, copies):
+    rng = np.random.default_rng(len(sizes) + copies)
+    parts = [rng.uniform(-1, 1, (n, 3)) * 40.0 ** -k + [0.3, -0.2, 0.1] for k, n in enumerate(sizes)]
+    parts.append(np.repeat([[0.25, 0.5, -0.75]], copies, axis=0))
+    P = np.concatenate(parts)
+    P = P[rng.permutation(len(P))].astype(np.float32)
+    return P, rng.normal(size=P.shape).astype(np.float32), rng.uniform(0.5, 2.0, len(P)).astype(np.float32)
+
+
+@pytest.mark.parametrize("sizes", [(2,), (64, 3), (513, 130, 40, 9, 4), (5000, 2000, 700, 129, 2, 2), (66000, 512)])
+def test_levels_of_few_points(sizes):
+    # clusters inside clusters: most points leave the split cells from one
+    # level to the next, in rows of 64 and 512 terms and past them; octree, CM
+    # and R are bit-identical
+    P, N, A = _clusters(sizes, 0)
+    c = gwn.PointCloudFWN(P, N, A, 2)
+    oc = O.Cloud(P, N, A, 2, np.float32)
+    CH, CN, W, _, cc, _ = c.octree()
+    assert np.array_equal(CH, oc.oct.CH) and np.array_equal(CN, oc.oct.CN) and np.array_equal(W, oc.oct.W)
+    assert np.array_equal(cc, oc.oct.cell_count)
+    CM, R, EC = c.expansion()
+    ne = cc > 0
+    assert np.array_equal(CM[ne], oc.CM[ne]) and np.array_equal(R[ne], oc.R[ne])
+    assert np.isnan(CM[~ne]).all() and np.all(EC[~ne] == 0) and np.all(R[~ne] == 0)
+
+
+@pytest.mark.parametrize("copies", [2, 33, 70, 600])
+def test_centres_with_points_that_no_level_tells_apart(copies):
+    # every centre is the FP32 sum over its cell's points in index order
+    P, N, A = _clusters((513, 130, 9), copies)
+    c = gwn.PointCloudFWN(P, N, A, 0)
+    _, _, _, cs, cc, pl = c.octree()
+    CM, _, _ = c.expansion()
+    for cell in np.flatnonzero(cc):
+        i = np.sort(pl[cs[cell]:cs[cell] + cc[cell]])
+        m = np.cumsum(A[i, None] * P[i], axis=0, dtype=np.float32)[-1] / np.cumsum(A[i], dtype=np.float32)[-1]
+        assert np.array_equal(CM[cell], m)
+
+
+@pytest.mark.parametrize("first", [0.0, -0.0])
+def test_flat_cloud_keeps_its_signs(first):
+    # a cloud in the plane z = 0: the root's centre is what minima and maxima
+    # that start from the first point give
+    P = np.random.default_rng(5).uniform(-1, 1, (1000, 3)).astype(np.float32)
+    P[:, 2] = -first
+    P[0, 2] = first
+    _, CN, _, _, _, _ = gwn.PointCloudFWN(P, np.ones_like(P), np.ones(1000, np.float32), 0).octree()
+    o = O.Octree(P, np.float32)
+    assert np.array_equal(CN, o.CN) and np.array_equal(np.signbit(CN[0]), np.signbit(o.CN[0]))
