@@ -31,8 +31,8 @@ inline uint32_t closest_budget(int64_t nslots) {
 // Batches below this take one wavefront per point: a wavefront of 64 points
 // walks the union of their boxes one record at a time, up to its budget, and
 // few of them do not fill the GPU meanwhile.  Per point / by 64, whole signed
-// distance calls: 1,000 points on 5,000 triangles 45 / 735 us, 10,000 on
-// 100,000 0.95 / 1.58 ms, 100,000 on 20,480 0.81 / 1.34 ms, 325,392 on 1,063
+// distance calls: 1,000 points on 5,000 triangles 43 / 735 us, 10,000 on
+// 100,000 0.34 / 1.58 ms, 100,000 on 20,480 0.92 / 1.34 ms, 325,392 on 1,063
 // 1.41 / 0.59 ms, 1M on 81,920 10.2 / 4.1 ms.
 constexpr int64_t kRingPointsBelow = 131072;
 constexpr int kStarts = 16;  // greedy descents of k_closest_ring below the root's
