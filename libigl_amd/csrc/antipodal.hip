@@ -437,8 +437,8 @@ void antipodal_query_device(const gwn_antipodal* a, const double* O, int64_t no,
   void* tmp = ws.take(tb);
   hipLaunchKernelGGL(k_ap_plane, dim3(div_up(no, 256)), dim3(256), 0, st, O, no, f, Of);
   check_launch("k_ap_plane");
-  hilbert_keys(Of, no, s->bbox, keys, perm, st);
-  radix_sort_u32(keys, perm, no, 30, tmp, tb, st);
+  hilbert_keys(Of, no, s->bbox, keys, perm, tmp, st);
+  radix_sort_counted_u32(keys, perm, no, 30, tmp, tb, st);
   ProfileScope prof("antipodal_crossings", st);
   hipLaunchKernelGGL(k_ap_crossings, dim3(g), dim3(256), 0, st, s->dbox.p, (uint32_t)s->nslots, a->tri.p, O, perm, no,
                      r, f, W);

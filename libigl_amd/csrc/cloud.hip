@@ -1450,8 +1450,8 @@ void cloud_query_device(const gwn_cloud* c, const float* Q, int64_t nq, double b
   uint32_t* keys = ws.take_n<uint32_t>((size_t)nq);
   uint32_t* perm = ws.take_n<uint32_t>((size_t)nq);
   void* tmp = ws.take(tb);
-  hilbert_keys(Q, nq, c->bbox, keys, perm, st);
-  radix_sort_u32(keys, perm, nq, 30, tmp, tb, st);
+  hilbert_keys(Q, nq, c->bbox, keys, perm, tmp, st);
+  radix_sort_counted_u32(keys, perm, nq, 30, tmp, tb, st);
   const bool rl = c->root_leaf;
   // the sort keys are spent: their space holds the block order (g entries)
   // and the block costs (g bytes)

@@ -680,8 +680,8 @@ void signed_distance_device(gwn_soup* s, const double* P, int64_t np, int sign_t
                        (const uint32_t*)nullptr, np, up2, best, face, cl);
     check_launch("k_closest_ring");
   } else {
-    hilbert_keys(Pf, np, s->bbox, keys, perm, st);
-    radix_sort_u32(keys, perm, np, 30, tmp, tb, st);
+    hilbert_keys(Pf, np, s->bbox, keys, perm, tmp, st);
+    radix_sort_counted_u32(keys, perm, np, 30, tmp, tb, st);
     ProfileScope prof("closest_point", st);
     // the sort keys are spent: their space holds the handed-over queries
     uint32_t* deferred = keys;

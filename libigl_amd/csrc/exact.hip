@@ -368,8 +368,8 @@ void wntree_query_device(const uint8_t* rec, int64_t nrec, const double* tri, co
     void* tmp = ws.take(tb);
     hipLaunchKernelGGL(k_wn_narrow, dim3(div_up(3 * no, 256)), dim3(256), 0, st, O, 3 * no, Of);
     check_launch("k_wn_narrow");
-    hilbert_keys(Of, no, bbox, keys, perm, st);
-    radix_sort_u32(keys, perm, no, 30, tmp, tb, st);
+    hilbert_keys(Of, no, bbox, keys, perm, tmp, st);
+    radix_sort_counted_u32(keys, perm, no, 30, tmp, tb, st);
   }
   ProfileScope prof("exact_tree", st);
   const WNRecord* r = reinterpret_cast<const WNRecord*>(rec);

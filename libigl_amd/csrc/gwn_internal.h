@@ -185,6 +185,13 @@ void sah4_build(const float* boxes, uint32_t nboxes, std::vector<uint32_t>& node
 size_t radix_sort_temp_bytes(int64_t n, bool key64);
 void radix_sort_u32(uint32_t* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes,
                     hipStream_t st);
+// The sort of keys made by k_rs_keys (radix_keys.h) with this tmp's count table
+// (radix_counts_u32, radix_tiles(n) blocks); the values become the keys'
+// positions, bits >= 1.
+uint32_t* radix_counts_u32(void* tmp, int64_t n);
+int64_t radix_tiles(int64_t n);
+void radix_sort_counted_u32(uint32_t* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes,
+                            hipStream_t st);
 // sorts by the low `bits` of the keys (none: as they are) and returns where
 // the values lie then, in `vals` or in `tmp`; the keys are not kept
 const uint32_t* radix_sort_u32_values(uint32_t* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes,
@@ -223,8 +230,11 @@ void soup_ensure_dist(gwn_soup* s, hipStream_t st);
 // .off / .obj file as a triangle mesh (polygons split into fans)
 void read_triangle_mesh(const char* path, std::vector<double>& V, std::vector<int32_t>& F);
 void morton_keys(const float* Q, int64_t nq, const float* bbox, uint32_t* keys, uint32_t* vals, hipStream_t st);
-// 30-bit Hilbert keys (10 bits per axis over bbox) + identity values: query order for the tree walks
-void hilbert_keys(const float* Q, int64_t nq, const float* bbox, uint32_t* keys, uint32_t* vals, hipStream_t st);
+// The queries' order along a 30-bit Hilbert curve (10 bits per axis over bbox),
+// in which the tree walks take them: keys for radix_sort_counted_u32 with the
+// same tmp (radix_sort_temp_bytes(nq, false))
+void hilbert_keys(const float* Q, int64_t nq, const float* bbox, uint32_t* keys, uint32_t* vals, void* tmp,
+                  hipStream_t st);
 // Costliest-first order of the blocks of 256 sorted queries (perm) within
 // each XCD's range of logical blocks, block costs read from a kCostGrid^3
 // grid of log-scale walk costs over bbox: order ceil(nq/256) entries and

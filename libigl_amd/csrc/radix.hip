@@ -1,6 +1,7 @@
 // radix.hip -- stable LSD radix sort (8-bit digits) and exclusive scan.
 //
-// One pass = three kernels, none waiting on another block:
+// One pass = three kernels (two for the first pass over keys made by k_rs_keys,
+// radix_keys.h), none waiting on another block:
 //   k_rs_tile_hist    each 256-thread block counts the digits of its 2048-key
 //                     tile in LDS and writes them digit-major:
 //                     counts[d * ntiles + tile]
@@ -22,12 +23,10 @@
 #include <algorithm>
 
 #include "gwn_internal.h"
+#include "radix_keys.h"
 
 namespace gwn {
 
-constexpr int RS_THREADS = 256;
-constexpr int RS_ITEMS = 8;
-constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
 constexpr int RS_WAVES = RS_THREADS / 64;
 
 template <typename K>
@@ -118,7 +117,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const K* __restrict__
     const int64_t i = wbase + r * 64 + lane;
     const bool valid = i < n;
     key[r] = valid ? kin[i] : K(0);
-    val[r] = valid ? vin[i] : 0u;
+    val[r] = !valid ? 0u : vin ? vin[i] : (uint32_t)i;  // (no values: each key's own position)
   }
 #pragma unroll
   for (int r = 0; r < RS_ITEMS; ++r) {
@@ -261,9 +260,11 @@ size_t radix_sort_temp_bytes(int64_t n, bool key64) {
 }
 
 // Returns the sorted values, in `vals` or (after an odd number of passes) in
-// `tmp`; with `in_place` keys and values are copied back instead.
+// `tmp`; with `in_place` keys and values are copied back instead.  `counted`:
+// the keys come from k_rs_keys, their first counts are made and the values
+// are to be the keys' positions.
 template <typename K>
-static const uint32_t* radix_sort(bool in_place, K* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes, hipStream_t st) {
+static const uint32_t* radix_sort(bool in_place, bool counted, K* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes, hipStream_t st) {
   if (n <= 1) return vals;
   GWN_CHECK(tmp_bytes >= radix_sort_temp_bytes(n, sizeof(K) == 8), GWN_ERR_INVALID, "radix sort temp too small");
   GWN_CHECK(n < ((int64_t)1 << 32), GWN_ERR_INVALID, "radix sort: more than 2^32 - 1 keys");
@@ -282,11 +283,15 @@ static const uint32_t* radix_sort(bool in_place, K* keys, uint32_t* vals, int64_
   uint32_t* vb = v2;
   int passes = 0;
   for (int shift = 0; shift < bits; shift += 8) {
-    hipLaunchKernelGGL(k_rs_tile_hist<K>, dim3((unsigned)nt), dim3(RS_THREADS), 0, st, ka, n, shift, counts, nt);
-    check_launch("k_rs_tile_hist");
+    const bool first = counted && shift == 0;
+    if (!first) {
+      hipLaunchKernelGGL(k_rs_tile_hist<K>, dim3((unsigned)nt), dim3(RS_THREADS), 0, st, ka, n, shift, counts, nt);
+      check_launch("k_rs_tile_hist");
+    }
     hipLaunchKernelGGL(k_rs_digit_scan, dim3(256), dim3(256), 0, st, counts, nt, totals);
     check_launch("k_rs_digit_scan");
-    hipLaunchKernelGGL(k_rs_scatter<K>, dim3((unsigned)nt), dim3(RS_THREADS), 0, st, ka, va, kb, vb, n, shift, counts,
+    hipLaunchKernelGGL(k_rs_scatter<K>, dim3((unsigned)nt), dim3(RS_THREADS), 0, st, ka,
+                       first ? nullptr : va, kb, vb, n, shift, counts,
                        totals, nt);
     check_launch("k_rs_scatter");
     std::swap(ka, kb);
@@ -303,15 +308,23 @@ static const uint32_t* radix_sort(bool in_place, K* keys, uint32_t* vals, int64_
 
 void radix_sort_u32(uint32_t* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes,
                     hipStream_t st) {
-  radix_sort<uint32_t>(true, keys, vals, n, bits, tmp, tmp_bytes, st);
+  radix_sort<uint32_t>(true, false, keys, vals, n, bits, tmp, tmp_bytes, st);
 }
 const uint32_t* radix_sort_u32_values(uint32_t* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes,
                                       hipStream_t st) {
-  return radix_sort<uint32_t>(false, keys, vals, n, bits, tmp, tmp_bytes, st);
+  return radix_sort<uint32_t>(false, false, keys, vals, n, bits, tmp, tmp_bytes, st);
+}
+uint32_t* radix_counts_u32(void* tmp, int64_t n) {
+  return (uint32_t*)((uint8_t*)tmp + 2 * align256(4 * (size_t)n));
+}
+int64_t radix_tiles(int64_t n) { return div_up(n > 0 ? n : 1, RS_TILE); }
+void radix_sort_counted_u32(uint32_t* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes,
+                            hipStream_t st) {
+  radix_sort<uint32_t>(true, true, keys, vals, n, bits, tmp, tmp_bytes, st);
 }
 void radix_sort_u64(uint64_t* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes,
                     hipStream_t st) {
-  radix_sort<uint64_t>(true, keys, vals, n, bits, tmp, tmp_bytes, st);
+  radix_sort<uint64_t>(true, false, keys, vals, n, bits, tmp, tmp_bytes, st);
 }
 
 }  // namespace gwn

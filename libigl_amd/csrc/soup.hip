@@ -13,7 +13,7 @@
 //                   in the rope (skip-pointer) layout
 //   k_write_slots   one 96-byte record per non-empty child slot
 //
-// Query (gwn_soup_query*): k_hilbert_q + radix sort orders queries along a
+// Query (gwn_soup_query*): k_rs_keys + radix sort orders queries along a
 // Hilbert curve so a wavefront's 64 queries walk similar paths; k_traverse walks
 // the rope layout with no stack: a far child slot (|q-P|^2 > maxP2*beta^2 and
 // a finite Taylor value) adds its order-0/1/2 term and jumps to its skip
@@ -30,6 +30,7 @@
 
 #include "device_math.h"
 #include "gwn_internal.h"
+#include "radix_keys.h"
 #include "ring_walk.h"
 #include "soup_moments.h"
 
@@ -1172,17 +1173,17 @@ __device__ __forceinline__ uint32_t hilbert3_10(uint32_t x0, uint32_t x1, uint32
   for (int b = 9; b >= 0; --b) h = (h << 3) | (((X[0] >> b) & 1u) << 2) | (((X[1] >> b) & 1u) << 1) | ((X[2] >> b) & 1u);
   return h;
 }
-__global__ void k_hilbert_q(const float* __restrict__ Q, int64_t nq, float lx, float ly, float lz, float sx,
-                            float sy, float sz, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nq) return;
-  float fx = (Q[3 * i] - lx) * sx, fy = (Q[3 * i + 1] - ly) * sy, fz = (Q[3 * i + 2] - lz) * sz;
-  fx = fminf(fmaxf(fx, 0.0f), 1023.0f);
-  fy = fminf(fmaxf(fy, 0.0f), 1023.0f);
-  fz = fminf(fmaxf(fz, 0.0f), 1023.0f);
-  keys[i] = hilbert3_10((uint32_t)fx, (uint32_t)fy, (uint32_t)fz);
-  vals[i] = (uint32_t)i;
-}
+struct HilbertKey {
+  const float* Q;
+  float lx, ly, lz, sx, sy, sz;
+  __device__ __forceinline__ uint32_t operator()(int64_t i) const {
+    float fx = (Q[3 * i] - lx) * sx, fy = (Q[3 * i + 1] - ly) * sy, fz = (Q[3 * i + 2] - lz) * sz;
+    fx = fminf(fmaxf(fx, 0.0f), 1023.0f);
+    fy = fminf(fmaxf(fy, 0.0f), 1023.0f);
+    fz = fminf(fmaxf(fz, 0.0f), 1023.0f);
+    return hilbert3_10((uint32_t)fx, (uint32_t)fy, (uint32_t)fz);
+  }
+};
 
 // ---------------------------------------------------------------------------
 // host orchestration
@@ -1482,14 +1483,17 @@ void block_order(const uint8_t* grid, const float* bb, const float* Q, const uin
   check_launch("k_block_order");
 }
 
-// 30-bit Hilbert keys of the queries over a box (clamped to it) and the
-// identity permutation: the order in which the tree walks take their queries
-void hilbert_keys(const float* Q, int64_t nq, const float* bb, uint32_t* keys, uint32_t* vals, hipStream_t st) {
+// 30-bit Hilbert keys of the queries over a box (clamped to it): the order in
+// which the tree walks take their queries
+void hilbert_keys(const float* Q, int64_t nq, const float* bb, uint32_t* keys, uint32_t* vals, void* tmp,
+                  hipStream_t st) {
   const float ex = std::max(bb[3] - bb[0], 1e-30f), ey = std::max(bb[4] - bb[1], 1e-30f),
               ez = std::max(bb[5] - bb[2], 1e-30f);
-  hipLaunchKernelGGL(k_hilbert_q, dim3(div_up(nq, 256)), dim3(256), 0, st, Q, nq, bb[0], bb[1], bb[2], 1024.0f / ex,
-                     1024.0f / ey, 1024.0f / ez, keys, vals);
-  check_launch("k_hilbert_q");
+  const HilbertKey key{Q, bb[0], bb[1], bb[2], 1024.0f / ex, 1024.0f / ey, 1024.0f / ez};
+  const int64_t nt = radix_tiles(nq);
+  hipLaunchKernelGGL(k_rs_keys<HilbertKey>, dim3((unsigned)nt), dim3(RS_KEY_THREADS), 0, st, key, nq, keys, vals,
+                     radix_counts_u32(tmp, nq), nt);
+  check_launch("k_rs_keys");
 }
 
 // ---------------------------------------------------------------------------
@@ -1655,9 +1659,9 @@ void soup_query_device_ws(const gwn_soup* s, const float* Q, int64_t nq, float a
   {
     const size_t tmpb = radix_sort_temp_bytes(nq, false);
     void* tmp = take(tmpb);
-    hilbert_keys(Q, nq, s->bbox, keys, perm, st);
+    hilbert_keys(Q, nq, s->bbox, keys, perm, tmp, st);
     ProfileScope prof("radix_sort", st, prof_on);
-    radix_sort_u32(keys, perm, nq, 30, tmp, tmpb, st);
+    radix_sort_counted_u32(keys, perm, nq, 30, tmp, tmpb, st);
   }
   uint32_t* amb = (uint32_t*)take(4 * (size_t)nq);
   uint32_t* ambn = (uint32_t*)take(4);

@@ -71,3 +71,29 @@ def test_radix_sort_u64(n, bits):
         keys |= np.uint64(1) << np.uint64(63)
         keys[::3] &= ~(np.uint64(1) << np.uint64(63))
     _check(keys if bits == 64 else keys & np.uint64((1 << bits) - 1), bits)
+
+
+@pytest.mark.parametrize("n", [1, 2, 255, 2047, 2048, 2049, 4097, 100_003])
+def test_counted_sort_orders_queries_by_their_keys(n):
+    # hilbert_keys counts each tile's first digits as it writes the keys; the
+    # sort then starts from those counts and from the keys' positions
+    from hip_mem import DeviceArray
+    L = nat.lib()
+    keys_of = getattr(L, "_ZN3gwn12hilbert_keysEPKflS1_PjS2_PvP12ihipStream_t")
+    keys_of.argtypes, keys_of.restype = [C.c_void_p, C.c_int64] + [C.c_void_p] * 5, None
+    sort = getattr(L, "_ZN3gwn22radix_sort_counted_u32EPjS0_liPvmP12ihipStream_t")
+    sort.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_int, C.c_void_p, C.c_size_t, C.c_void_p]
+    sort.restype = None
+    tb = _fns()[0](n, False)
+    rng = np.random.default_rng(n)
+    Q = rng.uniform(-1.2, 1.2, (n, 3)).astype(np.float32)  # some outside the box, clamped to it
+    box = (C.c_float * 6)(-1, -1, -1, 1, 1, 1)
+    dq = DeviceArray.from_numpy(Q)
+    dk, dv = DeviceArray.from_numpy(np.zeros(n, np.uint32)), DeviceArray.from_numpy(np.full(n, 7, np.uint32))
+    tmp = DeviceArray((tb,), np.uint8)
+    keys_of(dq.data_ptr, n, C.addressof(box), dk.data_ptr, dv.data_ptr, tmp.data_ptr, None)
+    keys = dk.numpy()
+    assert keys.max() < 2**30 and (n < 1000 or np.unique(keys).size > n // 2)
+    sort(dk.data_ptr, dv.data_ptr, n, 30, tmp.data_ptr, tb, None)
+    order = np.argsort(keys, kind="stable").astype(np.uint32)
+    assert np.array_equal(dv.numpy(), order) and np.array_equal(dk.numpy(), keys[order])
