@@ -46,10 +46,18 @@ __device__ __attribute__((noinline)) double vos_atan2(const double* t, double px
 // Sum of vos_atan2 over triangles.  The determinant is the same, term for term
 // (a query in a triangle's plane gets the same zero, or the same sign); the
 // lengths come from the refined reciprocal square root and the rest uses
-// multiply-adds.  Where the angle hangs on the last bits (the query on an edge
-// or at a corner), and for a term the product does not take, vos_atan2 gives
-// it.  About 100 FP64 operations a triangle against 210 with a square root per
-// length and an atan2: 100,000 queries on 20,480 triangles 10.8 -> 6.4 ms.
+// multiply-adds.  About 100 FP64 operations a triangle against 210 with a
+// square root per length and an atan2: 100,000 queries on 20,480 triangles
+// 10.8 -> 6.4 ms.
+// An angle whose vector (den, det) is short against the lengths' product lll
+// (the query near an edge of the triangle) turns by the roundings of den, some
+// units of 1.1e-16 lll, over that vector's length.  Below kVosShort lll, and
+// for a term the product does not take, vos_atan2 gives it, so the two forms
+// differ by less than 1e-13 in any term.  On hierarchies of 5,000 to 89,400
+// faces one term in 8,000 takes vos_atan2 and the sums differ by 9e-16
+// (2-norm) and 3.5e-14 (largest, in root mean squares); at 1e-3 by 5e-15 and
+// 3.4e-13 with one term in 100,000, at 1e-9 by 5.5e-14 and 3.8e-12.
+constexpr double kVosShort = 1e-2;
 struct VosSum {
   AngleSum<double> angles;
   double extra = 0.0;
@@ -68,7 +76,7 @@ struct VosSum {
     const double dab = fma(a2, b2, fma(a1, b1, a0 * b0));
     const double lll = la * lb * lc;
     const double den = fma(dab, lc, fma(dca, lb, fma(dbc, la, lll)));
-    if (!(fmax(fabs(det), fabs(den)) > 1e-9 * lll) || !angles.add(det, den)) extra += vos_atan2(t, px, py, pz);
+    if (!(fmax(fabs(det), fabs(den)) > kVosShort * lll) || !angles.add(det, den)) extra += vos_atan2(t, px, py, pz);
   }
   __device__ __forceinline__ double total() const { return extra + angles.total(); }
 };

@@ -196,6 +196,31 @@ def test_queries_on_vertices_edges_and_faces(nq):
     np.testing.assert_allclose(W2[:125], O.winding_number_2d(P, E, Q[:125, :2]), rtol=0, atol=1e-12)
 
 
+@pytest.mark.parametrize("tris,nq", [(5_000, 20_000), (32_000, 10_000), (89_000, 70_000)])
+def test_hierarchy_sums_are_those_of_its_terms(tris, nq):
+    """Some queries of any batch lie near an edge of a face or a cap, where the
+    angle turns by the roundings of its vector over that vector's length: the
+    product leaves those terms to the per-triangle form, and the sums equal the
+    oracle's hierarchy, term by term.  Bounds: a term in the product differs by
+    less than 1e-13 rad (1.6e-14 in w), and two such may meet in a query; the
+    2-norm is twice what the forms differ by on the host with the same lists,
+    9e-16.  With every term in the product they differ by 2.5e-15 to 5.5e-14
+    (2-norm) and 1.7e-13 to 4e-12 (largest, in root mean squares)."""
+    V, F = D.uv_sphere(tris, 0, 3)
+    rng = np.random.default_rng(tris)
+    V = V * (1.0 + rng.normal(0.0, 0.01, (V.shape[0], 1)))
+    Q = rng.uniform(-1.5, 1.5, (nq, 3))
+    O.libc_srand(tris)
+    tree = gwn.WindingNumberAABB(V, F)
+    O.libc_srand(tris)
+    Wo = O.WNTree(V, F).query(Q)
+    d = tree.winding_number(Q) - Wo
+    rms = np.sqrt(np.mean(Wo * Wo))
+    print(f"{F.shape[0]} faces: rel {np.linalg.norm(d) / np.linalg.norm(Wo):.2e} max {np.abs(d).max() / rms:.2e}")
+    assert np.linalg.norm(d) <= 2e-15 * np.linalg.norm(Wo)
+    assert np.abs(d).max() <= 1e-13 * rms
+
+
 @pytest.mark.parametrize("nq", [1, 63, 65, 4097, 65_535, 65_536])
 def test_hierarchy_lanes_and_order_by_batch_size(nq):
     """64 lanes a query in input order below 65,536 queries, 32 lanes and the
