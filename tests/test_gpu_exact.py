@@ -260,3 +260,35 @@ def test_fp64_soup_exact_terms_on_edges_and_faces(nq):
     bvh = gwn.FastWindingNumberBVH().build(V, F, 2)
     W = bvh.query(Qn, 1e3, gwn.PREC_FP64)
     np.testing.assert_allclose(W, np.tile(ref / (4 * np.pi), -(-nq // 125))[:nq], rtol=0, atol=1e-12)
+
+
+@pytest.mark.parametrize("nq", [2_000, 65_541])
+def test_fp64_soup_terms_near_edges(nq):
+    """The FP64 walk with every triangle exact (accuracy_scale 1e3), queries
+    1e-6 to 1e-3 from the edges of 1,280 triangles: a triangle's vector
+    (den, num) is as short there as the distance over the edge, and turns by its
+    roundings over that length.  Such terms are UTsignedSolidAngleTri's own
+    (6070-6110), so W equals their sum.  Bound: the other terms' vectors are
+    1e-2 or longer and round by a few 1.1e-16 (a few 1e-14 rad, a fourth of it
+    in w, for the two triangles at the edge), and 1,280 products of 1.1e-16."""
+    V, F = D.bumpy_sphere(3, 8, 12)
+    rng = np.random.default_rng(12)
+    T = V.astype(np.float32).astype(np.float64)[F]
+    f, s = rng.integers(0, F.shape[0], 2000), rng.random((2000, 1))
+    r = 10.0 ** rng.uniform(-6, -3, (2000, 1))
+    Q = ((1 - s) * T[f, 0] + s * T[f, 1] + r * rng.normal(size=(2000, 3))).astype(np.float32).astype(np.float64)
+    ref = np.empty(2000)
+    for i, q in enumerate(Q):
+        d = T - q
+        inv = 1.0 / np.sqrt(d[..., 0] * d[..., 0] + d[..., 1] * d[..., 1] + d[..., 2] * d[..., 2])
+        d = d * inv[..., None]
+        (a0, a1, a2), (b0, b1, b2), (c0, c1, c2) = (d[:, k].T for k in range(3))
+        u0, u1, u2, w0, w1, w2 = b0 - a0, b1 - a1, b2 - a2, c0 - a0, c1 - a1, c2 - a2
+        num = a0 * (u1 * w2 - u2 * w1) + a1 * (u2 * w0 - u0 * w2) + a2 * (u0 * w1 - u1 * w0)
+        den = (1.0 + (a0 * b0 + a1 * b1 + a2 * b2) + (a0 * c0 + a1 * c1 + a2 * c2) + (b0 * c0 + b1 * c1 + b2 * c2))
+        ref[i] = (2.0 * np.where(num != 0, np.arctan2(num, den), 0.0)).astype(np.longdouble).sum() / (4 * np.pi)
+    bvh = gwn.FastWindingNumberBVH().build(V, F, 2)
+    W = bvh.query(np.tile(Q, (-(-nq // 2000), 1))[:nq], 1e3, gwn.PREC_FP64)
+    err = np.abs(W - np.tile(ref, -(-nq // 2000))[:nq])
+    print(f"max |W - sum of terms| {err.max():.2e}")
+    assert err.max() <= 1e-13
