@@ -68,9 +68,10 @@ struct ExactQueue {
 // visit(i, k, link, t) evaluates record i for the query, adds its far field (if
 // any) to the lane's own sums and says what is to be done; it sets link (the
 // record's link word) and k (kids[i]) for kDescend and t (the triangle) for
-// kExact and kExactNear.  exact(t) and exact_near(t) add a
-// triangle to the calling lane's own sums; subtree(first, end) adds records
-// first .. end - 1, which a full ring has no room for.
+// kExact and kExactNear, and may set them where they are not read.  exact(t)
+// and exact_near(t) add a triangle to the calling lane's own sums;
+// subtree(first, end) adds records first .. end - 1, the children of a record
+// descended into that a full ring has no room for.
 template <int BATCH = 64, typename VisitFn, typename Exact, typename ExactNear, typename Subtree>
 __device__ __forceinline__ void frontier_walk(uint32_t* __restrict__ ring, uint32_t* __restrict__ q,
                                               uint32_t* __restrict__ qn, uint32_t lane,
@@ -108,7 +109,7 @@ __device__ __forceinline__ void frontier_walk(uint32_t* __restrict__ ring, uint3
       }
       const uint64_t in = __ballot(fits);
       tail += (uint32_t)__popcll(b0 & in) + 2u * (uint32_t)__popcll(b1 & in) + 4u * (uint32_t)__popcll(b2 & in);
-      if (!fits) subtree(k.x, link);
+      if (down && !fits) subtree(k.x, link);  // (fits is false for later lanes that do not descend, too)
     }
     far.push(what == Visit::kExact, t);
     near.push(what == Visit::kExactNear, t);

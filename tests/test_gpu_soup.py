@@ -150,6 +150,52 @@ def test_frontier_walk_at_its_edges(ntri, nq):
             assert np.array_equal(W[:1], bvh.query(Q[:1], beta, prec))
 
 
+def _full_ring_with_far_lanes(nodes, boxdata, q, beta, ring=1024):
+    """Rounds of the one-wavefront walk of query q in which some lane's children
+    find no room in the ring while a later lane takes a far field (the walk of
+    ring_walk.h: 64 records a round, children pushed in lane order)."""
+    bd = boxdata.astype(np.float64)
+    q = np.asarray(q, np.float32).astype(np.float64)
+    kids = [[s for s in range(4) if nodes[n, s] != 0xFFFFFFFF] for n in range(nodes.shape[0])]
+    pend, rounds = [(0, s) for s in kids[0]], 0
+    while pend:
+        take, pend = pend[:64], pend[64:]
+        full = False
+        for n, s in take:
+            far = ((q - bd[n, [4 + s, 8 + s, 12 + s]]) ** 2).sum() > bd[n, s] * beta * beta
+            c = int(nodes[n, s])
+            if far:
+                if full:
+                    rounds += 1
+                    break
+            elif c & 0x80000000:
+                c &= 0x7FFFFFFF
+                full = full or len(pend) + len(kids[c]) > ring
+                if not full:
+                    pend += [(c, k) for k in kids[c]]
+    return rounds
+
+
+@pytest.mark.parametrize("beta", [8.0, 10.0, 20.0])
+@pytest.mark.parametrize("nq", [1, 2047, 2048])
+def test_frontier_walk_full_ring_among_far_lanes(nq, beta):
+    """Accuracy scales at which the frontier outgrows the ring while other lanes
+    of the round take far fields: only the lanes without room walk their
+    subtrees, so W is the wave-coherent walk's.  The records are fetched whole
+    below 2,048 queries and as needed from there; a batch of 2,047 gives what
+    2,048 give."""
+    V, F = D.bumpy_sphere(4, 16, 57)
+    rng = np.random.default_rng(58)
+    inside = V[rng.integers(0, V.shape[0], nq)] * rng.uniform(0.0, 0.6, (nq, 1))
+    Q = np.concatenate([inside, rng.uniform(-1.4, 1.4, (65_536 - nq, 3))])
+    bvh = gwn.FastWindingNumberBVH().build(V, F, 2)
+    assert _full_ring_with_far_lanes(bvh.nodes(), bvh.boxdata(), Q[0], beta) > 0
+    for prec, tol in ((gwn.PREC_FP32, 1e-5), (gwn.PREC_MIXED, 1e-5), (gwn.PREC_FP64, 1e-12)):
+        W = bvh.query(Q[:nq], beta, prec)
+        assert np.abs(W - bvh.query(Q, beta, prec)[:nq]).max() <= tol, prec
+        assert np.abs(W[:2047] - bvh.query(Q[:min(nq, 2047)], beta, prec)).max() <= tol, prec
+
+
 @pytest.mark.parametrize("order", [0, 1, 2])
 @pytest.mark.parametrize("nq", [300, 65_541])
 def test_far_fields_that_overflow_are_descended(order, nq):
