@@ -349,8 +349,11 @@ void antipodal_build(gwn_antipodal* a, const double* V, int64_t nv, const int32_
                 (a->x0[0] != 0.0 || a->x0[1] != 0.0 || a->x0[2] != 0.0),
             GWN_ERR_INVALID, "x0 must be a finite non-zero direction");
   GWN_CHECK(nv == 0 || V != nullptr, GWN_ERR_INVALID, "null vertices");
-  // the frame of the rays: w along x0, u and v any two axes across it
-  const double* x = a->x0;
+  // the frame of the rays: w along x0, u and v any two axes across it.  Any
+  // finite x0 is taken, so it is scaled by its largest component first: the
+  // squares of the components themselves may overflow or vanish.
+  const double most = std::max({std::fabs(a->x0[0]), std::fabs(a->x0[1]), std::fabs(a->x0[2])});
+  const double x[3] = {a->x0[0] / most, a->x0[1] / most, a->x0[2] / most};
   const double len = std::sqrt((x[0] * x[0] + x[1] * x[1]) + x[2] * x[2]);
   int k0 = 0;  // the axis least along x0
   for (int k = 1; k < 3; ++k)

@@ -123,3 +123,17 @@ def test_turned_boxes_and_both_walks(x0, shift, scale):
         k = keep[(keep >= part.start) & (keep < part.stop)]
         assert np.array_equal(s.winding_number(Qs[part])[k - part.start], W[k])
     assert W[50_000] == 0.0
+
+
+@pytest.mark.parametrize("x0", [[1e200, 1e200, 1e200], [-2e180, 1e200, 3e170], [1e-200, 2e-200, 0], [3e-170, -1e-180, 1e-200]])
+def test_directions_of_any_length(x0):
+    """Any finite non-zero direction is taken, also one whose squared length is
+    beyond FP64 at either end: a closed mesh's counts are its winding numbers
+    (one wavefront a ray, and 64 rays a wavefront)."""
+    V, F = D.bumpy_sphere(3, 8, 77)
+    Q = np.random.default_rng(78).uniform(-1.4, 1.4, (66_000, 3))
+    exact = np.round(gwn.winding_number_bruteforce(V, F, Q))
+    s = gwn.WindingNumberAntipodalScene(V, F, np.asarray(x0, float))
+    assert np.array_equal(s.info()["x0"], np.asarray(x0, float))
+    for n in (1000, 66_000):
+        assert np.array_equal(s.winding_number(Q[:n]), exact[:n])
