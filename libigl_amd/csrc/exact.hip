@@ -283,31 +283,34 @@ void exact_device(const double* V, int64_t nv, const int32_t* F, int64_t nf, con
 
 
 // ---------------------------------------------------------------------------
-// The reference's hierarchy (wntree.cpp), G lanes per query (queries in
+// The reference's hierarchy (wntree.cpp), one wavefront per query (queries in
 // Hilbert order when perm is given).  The lanes walk the query's pre-order
 // records together: inside an internal node's closed box they step to the
 // first child; otherwise they sum the node's triangle list (inside a leaf: its
 // faces; outside the box: its cap, or its faces when the cap is not smaller)
 // and jump past the subtree.  They share each list, lane l taking its
-// triangles l, l+G, ...; each lane sums its angles as one product, and the
+// triangles l, l+64, ...; each lane sums its angles as one product, and the
 // lanes' FP64 totals are added in a fixed order.  The reference adds a node's
-// children's sums; the orders agree to rounding.  A query's result depends on
-// the query and G only.
-// 20,480 triangles, 100,000 queries: 0.45 ms a call with an atan2 per triangle
-// and 64 lanes a query, 0.28 ms.
-template <int G>
+// children's sums; the orders agree to rounding.  A query's result does not
+// depend on the batch it is in, which is why batches of every size take 64
+// lanes a query: 32 lanes leave fewer of them idle at the lists' ends, but add
+// the terms in another order (20,480 triangles, 64 / 32 lanes: 36 / 50 us for
+// 1,000 queries, 313 / 298 us for 100,000, 2.26 / 1.82 ms for 1M; 32 lanes of
+// two sums each, which do add in this order, 36 / 327 us and 2.05 ms).
+// 20,480 triangles, 100,000 queries: 0.45 ms a call with an atan2 per triangle,
+// 0.31 ms.
 __global__ __launch_bounds__(256) void k_wn_tree_lanes(const WNRecord* __restrict__ rec, uint32_t nrec,
                                                         const double* __restrict__ tri,
                                                         const double* __restrict__ O,
                                                         const uint32_t* __restrict__ perm, int64_t no,
                                                         double* __restrict__ W) {
-  const uint32_t lane = threadIdx.x % G;
-  const int64_t w = ((int64_t)xcd_block() * 256 + threadIdx.x) / G;
+  const uint32_t lane = threadIdx.x & 63;
+  const int64_t w = (int64_t)xcd_block() * 4 + (threadIdx.x >> 6);
   if (w >= no) return;
   const int64_t q = perm ? (int64_t)perm[w] : w;
   const double px = O[3 * q], py = O[3 * q + 1], pz = O[3 * q + 2];
   VosSum sum;
-  uint32_t i = 0, at = 0, end = 0;  // the next record; the rest of the list being summed (the same on the G lanes)
+  uint32_t i = 0, at = 0, end = 0;  // the next record; the rest of the list being summed (the same on all lanes)
   for (;;) {
     while (at >= end && i < nrec) {  // to the next record with triangles for this query
       const WNRecord& r = rec[i];
@@ -323,10 +326,9 @@ __global__ __launch_bounds__(256) void k_wn_tree_lanes(const WNRecord* __restric
     }
     if (at >= end) break;
     if (lane < end - at) sum.add(tri + 9 * (size_t)(at + lane), px, py, pz);
-    at += G;
+    at += 64;
   }
-  double v = sum.total();
-  for (int off = G / 2; off >= 1; off >>= 1) v = __dadd_rn(v, __shfl_xor(v, off, 64));
+  const double v = wave_sum(sum.total());
   if (lane == 0) W[q] = v / (2.0 * EX_PI);
 }
 
@@ -344,13 +346,6 @@ void wntree_upload(const WNTreeHost& T, DevBuf<uint8_t>& rec, DevBuf<double>& tr
     GWN_HIP(hipMemcpyAsync(tri.p, T.tri.data(), sizeof(double) * T.tri.size(), hipMemcpyHostToDevice, st));
   GWN_HIP(hipStreamSynchronize(st));
 }
-
-// Batches below this take 64 lanes a query, larger ones 32.  Half the lanes
-// leave fewer of them idle at the ends of the lists, but a query then takes
-// twice as long: 20,480 triangles, 64 / 32 lanes: 35 / 50 us for 1,000
-// queries, 106 / 120 us for 10,000, 297 / 281 us for 100,000, 2.13 / 1.72 ms
-// for 1M.
-constexpr int64_t kWideLanesBelow = 65536;
 
 // O no x 3 and W no, device pointers; bbox: the root's box (query order)
 void wntree_query_device(const uint8_t* rec, int64_t nrec, const double* tri, const float* bbox, const double* O,
@@ -381,12 +376,7 @@ void wntree_query_device(const uint8_t* rec, int64_t nrec, const double* tri, co
   }
   ProfileScope prof("exact_tree", st);
   const WNRecord* r = reinterpret_cast<const WNRecord*>(rec);
-  if (no < kWideLanesBelow)
-    hipLaunchKernelGGL(k_wn_tree_lanes<64>, dim3(div_up(no, 4)), dim3(256), 0, st, r, (uint32_t)nrec, tri, O, perm, no,
-                       W);
-  else
-    hipLaunchKernelGGL(k_wn_tree_lanes<32>, dim3(div_up(no, 8)), dim3(256), 0, st, r, (uint32_t)nrec, tri, O, perm, no,
-                       W);
+  hipLaunchKernelGGL(k_wn_tree_lanes, dim3(div_up(no, 4)), dim3(256), 0, st, r, (uint32_t)nrec, tri, O, perm, no, W);
   check_launch("k_wn_tree_lanes");
 }
 

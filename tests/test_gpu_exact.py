@@ -46,19 +46,20 @@ def test_exact_hierarchy_matches_oracle_tree():
 
 
 def test_exact_hierarchy_result_independent_of_batch():
-    """One wavefront per query: batches of 4,096+ queries take them in
+    """One wavefront per query: batches of 65,536+ queries take them in
     Hilbert order, smaller ones in input order, and a query's lanes add the
     same terms in the same order either way, so its result does not depend on
     the batch it is in: bit for bit."""
     V, F, Q = D.exact_workload()
     rng = np.random.default_rng(7)
-    Q = np.concatenate([Q[:12000], D.near_surface_queries(V, F, 4000, 1e-4, rng), V[:50]])
+    Q = np.concatenate([Q[:66000], D.near_surface_queries(V, F, 4000, 1e-4, rng), V[:50]])
     tree = gwn.WindingNumberAABB(V, F)
-    W = tree.winding_number(Q)  # 16,050 queries, sorted
+    W = tree.winding_number(Q)  # 70,050 queries, sorted
     Wl = np.concatenate([tree.winding_number(Q[k:k + 4000]) for k in range(0, Q.shape[0], 4000)])
-    assert Q.shape[0] % 4000 != 0 and Q[16000:].shape[0] < 4096
+    assert Q.shape[0] > 65_536 and Q.shape[0] % 4000 != 0
     assert np.array_equal(W, Wl)
     assert np.array_equal(tree.winding_number(Q[::-1][:3000]), W[::-1][:3000])
+    assert np.array_equal(tree.winding_number(Q[:65_536]), W[:65_536])
 
 
 def test_exact_hierarchy_1310720_tris_vs_brute_force():
@@ -223,10 +224,9 @@ def test_hierarchy_sums_are_those_of_its_terms(tris, nq):
 
 @pytest.mark.parametrize("nq", [1, 63, 65, 4097, 65_535, 65_536])
 def test_hierarchy_lanes_and_order_by_batch_size(nq):
-    """64 lanes a query in input order below 65,536 queries, 32 lanes and the
-    Hilbert order from there: both sum the reference's lists (leaves of up to
-    100 faces, caps of any length), which agree with the sum over every face
-    to rounding."""
+    """Input order below 65,536 queries and the Hilbert order from there, 64
+    lanes a query: the reference's lists (leaves of up to 100 faces, caps of any
+    length) agree with the sum over every face to rounding."""
     V, F = D.noisy_sphere(4, 0.01, 5)
     Q = np.random.default_rng(nq).uniform(-1.3, 1.3, (nq, 3))
     W = gwn.WindingNumberAABB(V, F).winding_number(Q)
