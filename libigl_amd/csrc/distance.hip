@@ -30,11 +30,15 @@ inline uint32_t closest_budget(int64_t nslots) {
 }
 // Batches below this take one wavefront per point: a wavefront of 64 points
 // walks the union of their boxes one record at a time, up to its budget, and
-// few of them do not fill the GPU meanwhile.  Per point / by 64, whole signed
-// distance calls: 1,000 points on 5,000 triangles 43 / 735 us, 10,000 on
-// 100,000 0.34 / 1.58 ms, 100,000 on 20,480 0.92 / 1.34 ms, 325,392 on 1,063
-// 1.41 / 0.59 ms, 1M on 81,920 10.2 / 4.1 ms.
-constexpr int64_t kRingPointsBelow = 131072;
+// few of them do not fill the GPU meanwhile.  The smaller the mesh, the shorter
+// that union and the sooner the sort pays: whole signed distance calls with
+// the two took as long at 27,000 points on 20 triangles, 36,000 on 80, 58,000
+// on 320, 64,000 on 500, 75,000 on 700, 93,000 on 1,000 and some 150,000 on
+// 2,500 and more.  Per point / by 64: 48,000 points on 20 triangles 183 / 124
+// us, 65,000 on 320 353 / 328, 100,000 on 1,000 628 / 580, 65,000 on 1,000
+// 399 / 545, 100,000 on 20,480 0.93 / 1.36 ms, 131,071 on 81,920 1.88 / 2.19,
+// 262,144 on 81,920 3.32 / 2.41.
+inline int64_t ring_points_below(int64_t nf) { return std::min<int64_t>(131072, 28000 + 64 * nf); }
 constexpr int kStarts = 16;  // greedy descents of k_closest_ring below the root's
 
 __device__ __forceinline__ double dot3(const double* a, const double* b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
@@ -669,11 +673,12 @@ void signed_distance_device(gwn_soup* s, const double* P, int64_t np, int sign_t
   uint32_t* ndeferred = ws.take_n<uint32_t>(1);
   Centre centre{s->centre[0], s->centre[1], s->centre[2], 0.0f};
   for (int k = 0; k < 3; ++k) centre.reach += std::max(s->bbox[3 + k] - s->centre[k], s->centre[k] - s->bbox[k]);
-  if (sign_type == GWN_SIGN_FAST_WINDING_NUMBER || np >= kRingPointsBelow) {
+  const bool ring = np < ring_points_below(s->nf);
+  if (sign_type == GWN_SIGN_FAST_WINDING_NUMBER || !ring) {
     hipLaunchKernelGGL(k_narrow3, dim3(div_up(3 * np, 256)), dim3(256), 0, st, P, np, Pf);
     check_launch("k_narrow3");
   }
-  if (np < kRingPointsBelow) {
+  if (ring) {
     ProfileScope prof("closest_point", st);
     hipLaunchKernelGGL(k_closest_ring, dim3(div_up(np, 4)), dim3(256), 0, st, s->dbox.p, s->planes.p, s->kids.p,
                        (uint32_t)s->nslots, s->V64.p, s->F.p, centre, P, (const uint32_t*)nullptr,

@@ -145,7 +145,7 @@ def test_closest_point_deep_interior_queries():
     rng = np.random.default_rng(17)
     d = rng.normal(size=(3000, 3))
     inner = d / np.linalg.norm(d, axis=1)[:, None] * rng.uniform(0, 0.3, (3000, 1))
-    near = D.near_surface_queries(V, F, 60000, 1e-3, rng)
+    near = D.near_surface_queries(V, F, 130_000, 1e-3, rng)  # (small batches take the second walk for every point)
     P = np.concatenate([inner, near[:30000], [[np.nan, 0.0, 0.0]], near[30000:]])
     bvh = gwn.FastWindingNumberBVH().build(V, F, 2)
     for sign in (gwn.SIGN_UNSIGNED, gwn.SIGN_FAST_WINDING_NUMBER):
@@ -171,6 +171,28 @@ def test_signed_distance_large_batch():
     S1, I1, C1 = bvh.signed_distance(Q[12345:12346], gwn.SIGN_FAST_WINDING_NUMBER)
     assert I1[0] == I[12345] and np.array_equal(C1[0], C[12345])
     assert abs(S1[0] - S[12345]) <= 2e-5 * np.linalg.norm(C1[0] - Q[12345])
+
+
+@pytest.mark.parametrize("tris,line", [(20, 29_280), (320, 48_480), (1280, 109_920)])
+def test_closest_point_walks_on_small_meshes(tris, line):
+    """The line between the walks lies at 28,000 points and 64 more a triangle
+    (131,072 at most): the same answers bit for bit on either side of it, ties
+    between faces and points that are not finite included."""
+    V, F = D.icosphere({20: 0, 320: 2, 1280: 3}[tris])
+    assert line == 28_000 + 64 * F.shape[0]
+    rng = np.random.default_rng(tris)
+    P = np.concatenate([V, V[F].mean(1), 0.5 * (V[F[:, 0]] + V[F[:, 1]]), np.zeros((1, 3)),
+                        [[np.nan, 0, 0], [0, np.inf, 0], [1e30, 0, 0]]])
+    P = np.concatenate([P, rng.uniform(-1.5, 1.5, (line - P.shape[0], 3))])
+    bvh = gwn.FastWindingNumberBVH().build(V, F, 2)
+    by64 = bvh.signed_distance(P, gwn.SIGN_PSEUDONORMAL)
+    each = bvh.signed_distance(P[:-1], gwn.SIGN_PSEUDONORMAL)
+    for a, b in zip(each, by64):
+        assert np.array_equal(a, b[:-1], equal_nan=True)
+    sub = np.arange(0, line, 31)
+    So, Io, Co = O.signed_distance(V, F, P[sub], gwn.SIGN_UNSIGNED)
+    ok = np.isfinite(So)
+    np.testing.assert_allclose(np.abs(by64[0][sub][ok]), So[ok], rtol=1e-12, atol=1e-12)
 
 
 @pytest.mark.parametrize("shift", [0.0, 1e4])
