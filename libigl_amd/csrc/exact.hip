@@ -14,6 +14,8 @@
 // per query; the reference takes an atan2 per triangle and divides each.
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 #include "device_math.h"
 #include "gwn_internal.h"
 #include "ring_walk.h"
@@ -357,11 +359,13 @@ void wntree_query_device(const uint8_t* rec, int64_t nrec, const double* tri, co
   }
   uint32_t* perm = nullptr;
   // small batches walk in input order; larger ones along the Hilbert curve
-  // (neighbouring wavefronts then read the same records and triangles).  On
-  // 20,480 triangles the sort cost more than it saved up to 60,000 queries (209
-  // against 160 us) and as much at 100,000 (281 us); on 100,000 triangles it
-  // saved 65 us of 457 at 100,000 queries.
-  const bool sorted = no >= 65536;
+  // (neighbouring wavefronts then read the same records and triangles), the
+  // sooner the larger the tree.  Sorted / not: 200,000 queries on 20,480
+  // triangles (511 records) 534 / 513 us, 500,000 1.19 / 1.25 ms; 100,000 on
+  // 100,000 triangles (2,047) 411 / 398 us, 150,000 568 / 575; 70,000 on
+  // 327,680 (8,191) 485 / 507; 20,000 on 1.31M (32,767) 379 / 364, 40,000
+  // 580 / 624.  The two meet where queries x sqrt(records) is 5 to 7 million.
+  const bool sorted = (double)no * std::sqrt((double)nrec) >= 6e6;
   const size_t tb = sorted ? radix_sort_temp_bytes(no, false) : 0;
   Scratch ws(sorted ? scratch_bytes({12 * (size_t)no, 4 * (size_t)no, 4 * (size_t)no, tb}) : 1, st);
   if (sorted) {

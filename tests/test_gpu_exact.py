@@ -46,20 +46,22 @@ def test_exact_hierarchy_matches_oracle_tree():
 
 
 def test_exact_hierarchy_result_independent_of_batch():
-    """One wavefront per query: batches of 65,536+ queries take them in
-    Hilbert order, smaller ones in input order, and a query's lanes add the
-    same terms in the same order either way, so its result does not depend on
-    the batch it is in: bit for bit."""
+    """One wavefront per query: large batches (from 6e6 over the root of the
+    number of records on, here about 265,000) take them in Hilbert order, smaller
+    ones in input order, and a query's lanes add the same terms in the same order
+    either way, so its result does not depend on the batch it is in: bit for bit."""
     V, F, Q = D.exact_workload()
     rng = np.random.default_rng(7)
-    Q = np.concatenate([Q[:66000], D.near_surface_queries(V, F, 4000, 1e-4, rng), V[:50]])
     tree = gwn.WindingNumberAABB(V, F)
-    W = tree.winding_number(Q)  # 70,050 queries, sorted
-    Wl = np.concatenate([tree.winding_number(Q[k:k + 4000]) for k in range(0, Q.shape[0], 4000)])
-    assert Q.shape[0] > 65_536 and Q.shape[0] % 4000 != 0
+    n = int(np.ceil(6e6 / np.sqrt(tree.nodes().shape[0])))
+    Q = np.concatenate([Q, D.near_surface_queries(V, F, 4000, 1e-4, rng), V[:50]])
+    Q = np.concatenate([Q, rng.uniform(-1.5, 1.5, (n - Q.shape[0], 3))])
+    W = tree.winding_number(Q)  # sorted
+    Wl = np.concatenate([tree.winding_number(Q[k:k + 40_000]) for k in range(0, Q.shape[0], 40_000)])
     assert np.array_equal(W, Wl)
     assert np.array_equal(tree.winding_number(Q[::-1][:3000]), W[::-1][:3000])
-    assert np.array_equal(tree.winding_number(Q[:65_536]), W[:65_536])
+    assert np.array_equal(tree.winding_number(Q[:-1]), W[:-1])
+    assert np.array_equal(tree.winding_number(Q[99_000:105_000]), W[99_000:105_000])
 
 
 def test_exact_hierarchy_1310720_tris_vs_brute_force():
@@ -222,10 +224,10 @@ def test_hierarchy_sums_are_those_of_its_terms(tris, nq):
     assert np.abs(d).max() <= 1e-13 * rms
 
 
-@pytest.mark.parametrize("nq", [1, 63, 65, 4097, 65_535, 65_536])
+@pytest.mark.parametrize("nq", [1, 63, 65, 4097, 65_535, 65_536, 540_001])
 def test_hierarchy_lanes_and_order_by_batch_size(nq):
-    """Input order below 65,536 queries and the Hilbert order from there, 64
-    lanes a query: the reference's lists (leaves of up to 100 faces, caps of any
+    """Input order, and the Hilbert order from 532,414 queries on (a tree of 127
+    records), 64 lanes a query: the reference's lists (leaves of up to 100 faces, caps of any
     length) agree with the sum over every face to rounding."""
     V, F = D.noisy_sphere(4, 0.01, 5)
     Q = np.random.default_rng(nq).uniform(-1.3, 1.3, (nq, 3))
