@@ -119,8 +119,9 @@ __device__ __forceinline__ void pack_far_field(const double* b, const double* q,
   r[19] = (T)g[9];           // f.w  xyz
 }
 
-// 1/sqrt(x) to FP64 rounding: the hardware estimate (about 2^-26 relative) and
-// one third-order step
+// 1/sqrt(x) to FP64 rounding: with the hardware estimate r (about 2^-26
+// relative) and e = 1 - x r^2 it is r (1 - e)^(-1/2), the binomial series of
+// which is taken to e^2: 1 + e/2 + 3 e^2/8
 __device__ __forceinline__ double rsqrt64(double x) {
   const double r = __builtin_amdgcn_rsq(x);
   const double e = fma(-(x * r), r, 1.0);
@@ -140,12 +141,14 @@ struct AngleSum {
   int32_t turns = 0;
 
   // Adds atan2(y, x) (y, x not NaN, not both zero, their product with the
-  // unit-sized sum neither overflowing nor vanishing) and returns true;
-  // otherwise leaves the sum as it is and returns false.
+  // unit-sized sum not overflowing, and far enough above the denormals that
+  // its parts round as the sum does) and returns true; otherwise leaves the
+  // sum as it is and returns false.
   __device__ __forceinline__ bool add(T y, T x) {
+    constexpr T least = sizeof(T) == 4 ? T(1e-30) : T(1e-290);  // smallest normal / epsilon: 1.0e-31, 1.0e-292
     const T r = fma(-im, y, re * x), i = fma(re, y, im * x);
     const T s = fmax(fabs(r), fabs(i));
-    if (!(s > T(0) && s < T(INFINITY))) return false;
+    if (!(s > least && s < T(INFINITY))) return false;
     // both arguments on one side of the real axis and the product on the
     // other: the sum of the two left [-pi, pi]
     const int32_t a = sign_word(im), b = sign_word(y), c = sign_word(i);

@@ -294,3 +294,21 @@ def test_fp64_soup_terms_near_edges(nq):
     err = np.abs(W - np.tile(ref, -(-nq // 2000))[:nq])
     print(f"max |W - sum of terms| {err.max():.2e}")
     assert err.max() <= 1e-13
+
+
+@pytest.mark.parametrize("power", [-525, -300, 300])
+@pytest.mark.parametrize("nq", [300, 20_000])
+def test_exact_2d_at_any_scale(power, nq):
+    """A curve and its queries scaled by a power of two have the same angles, also
+    where the products of two lengths are denormal (2^-525: 1e-316): the angle
+    product takes no vector that the denormals have rounded."""
+    n = 1500
+    t = np.linspace(0, 2 * np.pi, n, endpoint=False)
+    r = 1 + 0.3 * np.sin(7 * t)
+    V = np.stack([r * np.cos(t), r * np.sin(t)], 1)
+    E = np.stack([np.arange(n), (np.arange(n) + 1) % n], 1).astype(np.int32)
+    Q = np.random.default_rng(9).uniform(-1.6, 1.6, (nq, 2))
+    Wo = O.winding_number_2d(V, E, Q)
+    err = np.abs(gwn.winding_number(np.ldexp(V, power), E, np.ldexp(Q, power)) - Wo).max()
+    print(f"2^{power}: max |dW| {err:.2e}")
+    assert err < 1e-12
