@@ -237,3 +237,22 @@ def test_closest_point_on_slivers_and_points():
     S, I, C = gwn.signed_distance(P, V, F, gwn.SIGN_UNSIGNED)
     So, Io, Co = O.signed_distance(V, F, P, gwn.SIGN_UNSIGNED)
     np.testing.assert_allclose(S, So, rtol=1e-9, atol=1e-12)
+
+
+@pytest.mark.parametrize("power", [-70, -74, -77, 40])
+@pytest.mark.parametrize("n", [3000, 131_072])
+def test_closest_point_at_any_scale(power, n):
+    """A mesh scaled by a power of two has the scaled closest points, bit for
+    bit, also where the FP32 tests' squared distances are denormal (2^-70 and
+    below: 1e-43): they reject nothing that FP64 would take."""
+    V, F = D.bumpy_sphere(3, 8, 41)
+    V = V.astype(np.float32).astype(np.float64)
+    rng = np.random.default_rng(41)
+    P = np.concatenate([D.near_surface_queries(V, F, n // 2, 1e-2, rng), rng.uniform(-1.3, 1.3, (n - n // 2, 3))])
+    S, I, C = gwn.FastWindingNumberBVH().build(V, F, 2).signed_distance(P, gwn.SIGN_UNSIGNED)
+    scaled = gwn.FastWindingNumberBVH().build(np.ldexp(V, power), F, 2)
+    # (the lower bound on distances, DBL_MIN by default, is far below both)
+    Ss, Is, Cs = scaled.signed_distance(np.ldexp(P, power), gwn.SIGN_UNSIGNED)
+    assert np.array_equal(np.ldexp(Ss, -power), S)
+    same = Is == I  # faces that share the closest edge or vertex may differ with the tree
+    assert same.mean() > 0.5 and np.abs(np.ldexp(Cs, -power) - C).max() <= 1e-12
