@@ -512,11 +512,9 @@ struct SolidAngleSum {
       const T k0 = fma(u1, w2, -(u2 * w1)), k1 = fma(u2, w0, -(u0 * w2)), k2 = fma(u0, w1, -(u1 * w0));
       num = fma(a2, k2, fma(a1, k1, a0 * k0));
     } else {
-      // rounded product by product, as tri_solid_angle: where products cancel
-      // (a query in the triangle's plane) the numerator is zero
       num = a0 * (u1 * w2 - u2 * w1) + a1 * (u2 * w0 - u0 * w2) + a2 * (u0 * w1 - u1 * w0);
     }
-    if (num == T(0)) return;
+    if (sizeof(T) == 4 && num == T(0)) return;
     const T ab = fma(a2, b2, fma(a1, b1, a0 * b0));
     const T ac = fma(a2, c2, fma(a1, c1, a0 * c0));
     const T bc = fma(b2, c2, fma(b1, c1, b0 * c0));
@@ -526,8 +524,11 @@ struct SolidAngleSum {
     // tri_solid_angle's.  Sums over the triangles near 6,000 queries, half of
     // them 1e-6 from the surface, differ from that form's by 4.6e-16 (rms) and
     // 4e-15 (at most); with a line at 1e-9 by 6.7e-15 and 4.6e-13, and lay
-    // further from the true sums.  One term in 20,000 there is so short.
-    const bool fine = sizeof(T) == 4 || fmax(fabs(num), fabs(den)) > T(1e-2);
+    // further from the true sums.  One term in 20,000 there is so short.  The
+    // same for a query (nearly) in the triangle's plane and inside it, where
+    // whether num is zero, and its sign, hang on the last bits, and with them
+    // a whole turn of the angle.
+    const bool fine = sizeof(T) == 4 || (fmax(fabs(num), fabs(den)) > T(1e-2) && fabs(num) >= T(-1e-9) * den);
     if (!fine || !half.add(num, den))
       extra += tri_solid_angle<T>(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], qx, qy, qz);
   }

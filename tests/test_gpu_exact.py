@@ -265,35 +265,45 @@ def test_fp64_soup_exact_terms_on_edges_and_faces(nq):
 
 
 @pytest.mark.parametrize("nq", [2_000, 65_541])
-def test_fp64_soup_terms_near_edges(nq):
+@pytest.mark.parametrize("where", ["near edges", "on the surface"])
+def test_fp64_soup_terms_at_the_surface(where, nq):
     """The FP64 walk with every triangle exact (accuracy_scale 1e3), queries
-    1e-6 to 1e-3 from the edges of 1,280 triangles: a triangle's vector
-    (den, num) is as short there as the distance over the edge, and turns by its
-    roundings over that length.  Such terms are UTsignedSolidAngleTri's own
-    (6070-6110), so W equals their sum.  Bound: the other terms' vectors are
-    1e-2 or longer and round by a few 1.1e-16 (a few 1e-14 rad, a fourth of it
-    in w, for the two triangles at the edge), and 1,280 products of 1.1e-16."""
+    1e-6 to 1e-3 from the edges of 1,280 triangles, or at their corners, the
+    middles of their edges and their centroids: a triangle's vector (den, num)
+    may be short there and turns by its roundings over its length, and in a
+    triangle's plane the sign of num decides a half turn.  Such terms are
+    UTsignedSolidAngleTri's own (6070-6110), so W equals their sum.  Bound: the
+    other terms' vectors are 1e-2 or longer and round by a few 1.1e-16 (a few
+    1e-14 rad, a fourth of it in w, for the two triangles at the edge), and
+    1,280 products of 1.1e-16.  The mixed form takes these terms in FP64 too and
+    the others in FP32."""
     V, F = D.bumpy_sphere(3, 8, 12)
     rng = np.random.default_rng(12)
     T = V.astype(np.float32).astype(np.float64)[F]
     f, s = rng.integers(0, F.shape[0], 2000), rng.random((2000, 1))
-    r = 10.0 ** rng.uniform(-6, -3, (2000, 1))
-    Q = ((1 - s) * T[f, 0] + s * T[f, 1] + r * rng.normal(size=(2000, 3))).astype(np.float32).astype(np.float64)
+    if where == "near edges":
+        r = 10.0 ** rng.uniform(-6, -3, (2000, 1))
+        Q = (1 - s) * T[f, 0] + s * T[f, 1] + r * rng.normal(size=(2000, 3))
+    else:
+        Q = np.concatenate([T[f[:200], 0], 0.5 * (T[f[200:1200], 0] + T[f[200:1200], 1]), T[f[1200:]].mean(1)])
+    Q = Q.astype(np.float32).astype(np.float64)
     ref = np.empty(2000)
     for i, q in enumerate(Q):
         d = T - q
-        inv = 1.0 / np.sqrt(d[..., 0] * d[..., 0] + d[..., 1] * d[..., 1] + d[..., 2] * d[..., 2])
-        d = d * inv[..., None]
+        l = np.sqrt(d[..., 0] * d[..., 0] + d[..., 1] * d[..., 1] + d[..., 2] * d[..., 2])
+        d = d * (1.0 / np.where(l == 0, 1.0, l))[..., None]
         (a0, a1, a2), (b0, b1, b2), (c0, c1, c2) = (d[:, k].T for k in range(3))
         u0, u1, u2, w0, w1, w2 = b0 - a0, b1 - a1, b2 - a2, c0 - a0, c1 - a1, c2 - a2
         num = a0 * (u1 * w2 - u2 * w1) + a1 * (u2 * w0 - u0 * w2) + a2 * (u0 * w1 - u1 * w0)
         den = (1.0 + (a0 * b0 + a1 * b1 + a2 * b2) + (a0 * c0 + a1 * c1 + a2 * c2) + (b0 * c0 + b1 * c1 + b2 * c2))
-        ref[i] = (2.0 * np.where(num != 0, np.arctan2(num, den), 0.0)).astype(np.longdouble).sum() / (4 * np.pi)
+        t = np.where((num != 0) & (l != 0).all(1), 2.0 * np.arctan2(num, den), 0.0)
+        ref[i] = t.astype(np.longdouble).sum() / (4 * np.pi)
     bvh = gwn.FastWindingNumberBVH().build(V, F, 2)
-    W = bvh.query(np.tile(Q, (-(-nq // 2000), 1))[:nq], 1e3, gwn.PREC_FP64)
-    err = np.abs(W - np.tile(ref, -(-nq // 2000))[:nq])
-    print(f"max |W - sum of terms| {err.max():.2e}")
-    assert err.max() <= 1e-13
+    for prec, tol in ((gwn.PREC_FP64, 1e-13), (gwn.PREC_MIXED, 1e-5)):
+        W = bvh.query(np.tile(Q, (-(-nq // 2000), 1))[:nq], 1e3, prec)
+        err = np.abs(W - np.tile(ref, -(-nq // 2000))[:nq])
+        print(f"{where}: max |W - sum of terms| {err.max():.2e}")
+        assert err.max() <= tol
 
 
 @pytest.mark.parametrize("power", [-525, -300, 300])
