@@ -1280,9 +1280,9 @@ void cloud_build_device(gwn_cloud* c, hipStream_t st, bool moments) {
     GWN_HIP(hipMemcpyAsync(made.p, &one, 4, hipMemcpyHostToDevice, st));
     for (size_t d = 0; d < nlev; ++d) {
       const uint32_t b = lvl_off[d], e = lvl_off[d + 1];
-      hipLaunchKernelGGL(k_oct_level, dim3(div_up(8 * (int64_t)(e - b), OCT_THREADS)), dim3(OCT_THREADS), 0, st, all.p + b, made.p + d, e - b,
-                         HS, LS, lcp.p, oscan.p, c->CH.p, c->CN.p, c->Wd.p, c->cstart.p, c->ccount.p, all.p + e,
-                         made.p + d + 1, S - e, ncells, made.p + nlev + 1);
+      hipLaunchKernelGGL(k_oct_level, dim3(div_up(8 * (int64_t)(e - b), OCT_THREADS)), dim3(OCT_THREADS), 0, st,
+                         all.p + b, made.p + d, e - b, HS, LS, lcp.p, oscan.p, c->CH.p, c->CN.p, c->Wd.p, c->cstart.p,
+                         c->ccount.p, all.p + e, made.p + d + 1, S - e, ncells, made.p + nlev + 1);
     }
     check_launch("k_oct_level");
     std::vector<uint32_t> hm(nlev + 2);

@@ -177,7 +177,7 @@ __device__ __attribute__((noinline)) double signed_angle_2d(const double* e, dou
 // the product takes the unscaled cross and dot products.  A query (nearly) on
 // an edge, where the sign of the half turn hangs on the last bits, and a term
 // the product does not take are left to signed_angle_2d.  20,000 queries on
-// 26,214 edges, host arrays: 7.7 -> 0.9 ms.
+// 26,214 edges, host arrays: 3.9 -> 0.72 ms.
 struct Edge2dSum {
   AngleSum<double> angles;
   double extra = 0.0;
@@ -297,10 +297,10 @@ void exact_device(const double* V, int64_t nv, const int32_t* F, int64_t nf, con
 // depend on the batch it is in, which is why batches of every size take 64
 // lanes a query: 32 lanes leave fewer of them idle at the lists' ends, but add
 // the terms in another order (20,480 triangles, 64 / 32 lanes: 36 / 50 us for
-// 1,000 queries, 313 / 298 us for 100,000, 2.26 / 1.82 ms for 1M; 32 lanes of
-// two sums each, which do add in this order, 36 / 327 us and 2.05 ms).
+// 1,000 queries, 313 / 298 us for 100,000 in Hilbert order, 2.26 / 1.82 ms for
+// 1M; 32 lanes of two sums each, which do add in this order, 327 us and 2.05 ms).
 // 20,480 triangles, 100,000 queries: 0.45 ms a call with an atan2 per triangle,
-// 0.31 ms.
+// now 0.27 ms, in input order.
 __global__ __launch_bounds__(256) void k_wn_tree_lanes(const WNRecord* __restrict__ rec, uint32_t nrec,
                                                         const double* __restrict__ tri,
                                                         const double* __restrict__ O,

@@ -264,7 +264,8 @@ size_t radix_sort_temp_bytes(int64_t n, bool key64) {
 // the keys come from k_rs_keys, their first counts are made and the values
 // are to be the keys' positions.
 template <typename K>
-static const uint32_t* radix_sort(bool in_place, bool counted, K* keys, uint32_t* vals, int64_t n, int bits, void* tmp, size_t tmp_bytes, hipStream_t st) {
+static const uint32_t* radix_sort(bool in_place, bool counted, K* keys, uint32_t* vals, int64_t n, int bits, void* tmp,
+                                  size_t tmp_bytes, hipStream_t st) {
   if (n <= 1) return vals;
   GWN_CHECK(tmp_bytes >= radix_sort_temp_bytes(n, sizeof(K) == 8), GWN_ERR_INVALID, "radix sort temp too small");
   GWN_CHECK(n < ((int64_t)1 << 32), GWN_ERR_INVALID, "radix sort: more than 2^32 - 1 keys");
@@ -290,9 +291,8 @@ static const uint32_t* radix_sort(bool in_place, bool counted, K* keys, uint32_t
     }
     hipLaunchKernelGGL(k_rs_digit_scan, dim3(256), dim3(256), 0, st, counts, nt, totals);
     check_launch("k_rs_digit_scan");
-    hipLaunchKernelGGL(k_rs_scatter<K>, dim3((unsigned)nt), dim3(RS_THREADS), 0, st, ka,
-                       first ? nullptr : va, kb, vb, n, shift, counts,
-                       totals, nt);
+    hipLaunchKernelGGL(k_rs_scatter<K>, dim3((unsigned)nt), dim3(RS_THREADS), 0, st, ka, first ? nullptr : va, kb, vb,
+                       n, shift, counts, totals, nt);
     check_launch("k_rs_scatter");
     std::swap(ka, kb);
     std::swap(va, vb);

@@ -549,8 +549,8 @@ struct SolidAngleSum {
 // lane that takes a far field moves it past the subtree.)  The wave steps to
 // i+1 when some lane needs it (a near child, or an item) and otherwise to
 // link(i): every lane that is not taking part needs a record at or beyond
-// link(i), because the subtrees of the rope are nested intervals.  So each lane visits exactly the records
-// of its own walk, in the same order, and sums the same terms in the same
+// link(i), because the subtrees of the rope are nested intervals.  So each lane
+// visits exactly the records of its own walk, in the same order, and sums the same terms in the same
 // order as an independent per-lane walk; but every record (and triangle) a
 // wave reads is the same for all its lanes, so it is fetched once per wave
 // through the scalar cache instead of 64 times through the vector memory path.
@@ -560,7 +560,8 @@ __device__ __forceinline__ uint32_t wave_uniform(uint32_t v) { return __builtin_
 // (|q - P| < sqrt(maxP2) + near_d, P the slot's centre and maxP2 its squared
 // radius) has its solid angle computed in FP64 (UTsignedSolidAngleTri,
 // 6070-6110, in double) and summed in an FP64 accumulator of its own; the far
-// field and every other exact term go to the FP32 running sum.
+// field and every other exact term go to the FP32 sums.  The square root is the
+// hardware's, within an ulp: where the line lies is a choice, not a bound.
 __device__ __forceinline__ bool near_triangle(float maxp2, float l2, float near_d) {
   const float rr = __builtin_amdgcn_sqrtf(maxp2) + near_d;
   return l2 < rr * rr;
@@ -1366,7 +1367,6 @@ size_t soup_query_work_bytes(int64_t nq) {
   auto up = [&](size_t b) { return (b + a - 1) / a * a; };
   return up(4 * (size_t)nq) * 2 + up(radix_sort_temp_bytes(nq, false)) + up(4 * (size_t)nq) + up(4);
 }
-// Workspace of an unsorted (per-lane) call: the ambiguous list and count only.
 
 // 30-bit Morton keys of the queries over a box (queries outside are clamped
 // to it), and the identity permutation to be sorted along with them
